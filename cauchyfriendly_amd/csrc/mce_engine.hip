@@ -675,15 +675,8 @@ struct Engine {
     // reduction
     DBuf<uint64_t> fkeys, fskeys;
     DBuf<uint32_t> fidx, fsidx;
-    DBuf<double> fvals;
-    DBuf<int> ecnt, eoff, edges, indeg, inoff, cursor, cursor2, round_slots, Fc;
-    DBuf<uint8_t> st0, st1, isroot;
-    DBuf<uint32_t> memkey, memval, smkey, smval, roots, jiota;
-    DBuf<int> memcnt, memoff, inedges, dboff, gbase_dev, wlo;
-    DBuf<int64_t> wcnt, woff;
-    DBuf<double> fgb, fgp, fgA;
-    DBuf<uint8_t> pflag;
-    DBuf<uint32_t> bkey, bskey;
+    DBuf<int> rootpos, memrank, big_comp, Fc, dboff, gbase_dev;
+    DBuf<int64_t> gval, groff;
     std::vector<int> h_boff;
     // groups (all buckets of an update)
     DBuf<int> grp_root, grp_moff, grp_mcnt, grp_m, mem_slots, b2n, surv, gxor, sort_list, spos, sflag;
@@ -937,16 +930,6 @@ struct Engine {
             sk = dk;
             sv = dv;
         }
-    }
-    // out <- in[i] where flags[i] != 0, in order; the count into *count.
-    void select_flagged(const uint32_t* in_, const uint8_t* flags, uint32_t* out_, int* count, int n) {
-        if (n <= kSmallScan) {
-            MCE_RUN(k_small_select, dim3(1), dim3(kSmallScanThreads), 0, st, in_, flags, out_, count, n);
-            return;
-        }
-        cub("select", [=](void* t, size_t& bytes, hipStream_t s) {
-            return hipcub::DeviceSelect::Flagged(t, bytes, in_, flags, out_, count, n, s);
-        });
     }
     // *out <- max of n ints.
     void reduce_max(const int* in_, int* out_, int n) {
@@ -1577,10 +1560,10 @@ struct Engine {
         bt_base.reserve(np);
         btcap.reserve(np);
         TermPool IN = in.view();
-        // counters: [5] root count, [8] enumeration guard, [16] parents to enumerate, [17] MU
-        // errors, [18] groups to sort, [19] rare-path flags; the shape histograms of the gather
-        // (hist) and of the compaction (hist_mx, with the largest g-table after it): all
-        // cleared here, once per update
+        // counters: [8] enumeration guard, [16] parents to enumerate, [17] MU errors, [18] groups
+        // to sort, [19] rare-path flags, [24] a NaN in p, [25] large reduction components; the
+        // shape histograms of the gather (hist) and of the compaction (hist_mx, with the
+        // largest g-table after it): all cleared here, once per update
         fill_multi({{counters.ptr, 32 * sizeof(int), 0},
                     {slot_base.ptr, sizeof(int), 0},
                     {hist.ptr, (sr + 1) * sizeof(int), 0},
@@ -2089,139 +2072,42 @@ struct Engine {
         const int N = off[sr];
         gbase_of.assign(sr + 1, 0);
         if (N == 0) co_return 0;
-        const int a0 = g_search_order[0];
-        if (a0 < 0 || a0 >= d)
-            throw std::runtime_error("term-reduction search ordering names axis " + std::to_string(a0) + " of a " +
-                                     std::to_string(d) + "-state estimator");
         h_boff = off;
         dboff.reserve(sr + 1);
         upload(dboff.ptr, h_boff.data(), (sr + 1) * sizeof(int));
         const int* boff = dboff.ptr;
+        bool chunked = false;
+        for (int m = 0; m < sr; m++) chunked |= off[m + 1] - off[m] > kFtrChunkTerms;
+        const int waves = ceil_div(N, kCompOwn);
         fkeys.reserve(N);
         fskeys.reserve(N);
         fidx.reserve(N);
         fsidx.reserve(N);
-        bkey.reserve(N);
-        bskey.reserve(N);
-        fvals.reserve(N);
-        ecnt.reserve(N);
-        eoff.reserve(N);
-        const dim3 g1(ceil_div(N, 256)), b1(256);
-        // value order on the first search axis, then (stable) bucket order
-        MCE_RUN(k_ftr_keys, g1, b1, 0, st, OUT, perm.ptr, N, d, a0, fkeys.ptr, fidx.ptr);
-        sort_pairs(fkeys.ptr, fskeys.ptr, fidx.ptr, fsidx.ptr, N, 0, 64);
-        MCE_RUN(k_ftr_bkeys, g1, b1, 0, st, N, boff, sr, fsidx.ptr, bkey.ptr);
-        int bbits = 1;
-        while ((1 << bbits) < sr) bbits++;
-        sort_pairs(bkey.ptr, bskey.ptr, fsidx.ptr, fidx.ptr, N, 0, bbits);
-        const uint32_t* sidx = fidx.ptr;
-        MCE_RUN(k_ftr_vals, g1, b1, 0, st, OUT, perm.ptr, N, d, a0, sidx, fvals.ptr);
-        // candidate windows on the first search axis; the predicate runs one thread per
-        // (term, window slot) pair unless the pairs would not fit, then one per term
-        wlo.reserve(N);
-        wcnt.reserve(N);
-        woff.reserve(N);
-        MCE_RUN(k_ftr_win, g1, b1, 0, st, N, boff, sr, fvals.ptr, wlo.ptr, wcnt.ptr, ecnt.ptr);
-        const int64_t npairs = co_await scan_excl_total(wcnt.ptr, woff.ptr, N);
-        const bool by_pairs = npairs < ((int64_t)1 << 31);
-        if (by_pairs && npairs > 0) {
-            fgb.reserve((size_t)N * d);
-            fgp.reserve((size_t)N * MM);
-            fgA.reserve((size_t)N * MM);
-            pflag.reserve((size_t)npairs);
-            MCE_DISPATCH_D(d, MCE_RUN(k_ftr_gather<DD>, g1, b1, 0, st, OUT, perm.ptr, N, boff, sr, sidx,
-                                                 fgb.ptr, fgp.ptr, fgA.ptr));
-            MCE_DISPATCH_D(d, MCE_RUN(k_ftr_pairs<DD>, dim3(ceil_div(npairs, 256)), b1, 0, st, npairs, N,
-                                                 boff, sr, dconst.ptr, woff.ptr, wlo.ptr, sidx, MM, fgb.ptr, fgp.ptr,
-                                                 fgA.ptr, pflag.ptr, ecnt.ptr, eoff.ptr, cursor.ptr, edges.ptr, 0));
-        } else if (!by_pairs) {
-            MCE_DISPATCH_D(d, MCE_RUN(k_ftr_edges<DD>, g1, b1, 0, st, OUT, perm.ptr, N, boff, sr,
-                                                 dconst.ptr, fvals.ptr, sidx, ecnt.ptr, eoff.ptr, edges.ptr, 0));
-        }
-        HIPCHK(hipGetLastError());
-        const int E = (int)(co_await scan_excl_total(ecnt.ptr, eoff.ptr, N));
-        Fc.reserve((size_t)8 * N);
-        MCE_RUN(k_ftr_finit, g1, b1, 0, st, Fc.ptr, N, boff, sr);
-        if (E > 0) {
-            edges.reserve(E);
-            inedges.reserve(E);
-            cursor.reserve(N);
-            cursor2.reserve(N);
-            indeg.reserve(N);
-            inoff.reserve(N);
-            st0.reserve(N);
-            st1.reserve(N);
-            round_slots.reserve(kRoundSlots);
-            // every buffer the edge passes and the rounds start from, in one launch
-            fill_multi({{cursor.ptr, N * sizeof(int), 0},
-                        {cursor2.ptr, N * sizeof(int), 0},
-                        {indeg.ptr, N * sizeof(int), 0},
-                        {st0.ptr, (size_t)N, kUnknown},
-                        {round_slots.ptr, kRoundSlots * sizeof(int), 0}});
-            if (by_pairs) {
-                MCE_DISPATCH_D(d, MCE_RUN(k_ftr_pairs<DD>, dim3(ceil_div(npairs, 256)), b1, 0, st, npairs,
-                                                     N, boff, sr, dconst.ptr, woff.ptr, wlo.ptr, sidx, MM, fgb.ptr,
-                                                     fgp.ptr, fgA.ptr, pflag.ptr, ecnt.ptr, eoff.ptr, cursor.ptr,
-                                                     edges.ptr, 1));
-            } else {
-                MCE_DISPATCH_D(d, MCE_RUN(k_ftr_edges<DD>, g1, b1, 0, st, OUT, perm.ptr, N, boff, sr,
-                                                     dconst.ptr, fvals.ptr, sidx, ecnt.ptr, eoff.ptr, edges.ptr, 1));
-            }
-            MCE_RUN(k_ftr_inedges, g1, b1, 0, st, N, boff, sr, eoff.ptr, ecnt.ptr, edges.ptr, indeg.ptr,
-                               (const int*)nullptr, (int*)nullptr, (int*)nullptr, 0);
-            scan_i32_excl(indeg.ptr, inoff.ptr, N);
-            MCE_RUN(k_ftr_inedges, g1, b1, 0, st, N, boff, sr, eoff.ptr, ecnt.ptr, edges.ptr, indeg.ptr,
-                               inoff.ptr, cursor2.ptr, inedges.ptr, 1);
-            uint8_t* sa = st0.ptr;
-            uint8_t* sb = st1.ptr;
-            // Rounds are idempotent once every term is resolved, so several run between
-            // reads of the unresolved count (taken from the last round of a batch).
-            int batch = 2, round = 0;
-            for (int done = 0; done <= N + 1;) {
-                for (int r = 0; r < batch; r++, round++) {
-                    MCE_RUN(k_ftr_round, g1, b1, 0, st, N, inoff.ptr, indeg.ptr, inedges.ptr, sa, sb,
-                                       round_slots.ptr, round);
-                    std::swap(sa, sb);
-                }
-                done += batch;
-                if ((co_await rd1(round_slots.ptr + (round - 1) % kRoundSlots)) == 0) break;
-                batch = std::min(batch * 2, 16);
-            }
-            MCE_RUN(k_ftr_claim, g1, b1, 0, st, N, boff, sr, eoff.ptr, ecnt.ptr, edges.ptr, sa, Fc.ptr);
-            if (N > 10000) {
-                for (int lvl = 0; lvl < 3; lvl++)
-                    MCE_RUN(k_ftr_merge, dim3(ceil_div(N, 256), 8 >> (lvl + 1)), b1, 0, st, N, boff, sr,
-                                       Fc.ptr, lvl);
-            }
-            HIPCHK(hipGetLastError());
-        }
-        // reduction groups
-        isroot.reserve(N);
-        memkey.reserve(N);
-        memval.reserve(N);
-        smkey.reserve(N);
-        smval.reserve(N);
-        roots.reserve(N);
-        jiota.reserve(N);
-        memcnt.reserve(N + 1);
-        memoff.reserve(N + 1);
-        MCE_RUN(k_ftr_rootflags, g1, b1, 0, st, N, boff, sr, Fc.ptr, isroot.ptr, memkey.ptr, memval.ptr);
-        MCE_RUN(k_iota, g1, b1, 0, st, jiota.ptr, N);
-        select_flagged(jiota.ptr, isroot.ptr, roots.ptr, counters.ptr + 5, N);
-        int kbits = 1;
-        while (((int64_t)1 << kbits) <= N) kbits++;
-        sort_pairs(memkey.ptr, smkey.ptr, memval.ptr, smval.ptr, N, 0, kbits);
+        rootpos.reserve(N);
+        memrank.reserve(N);
+        gval.reserve(N);
+        groff.reserve(N);
         gbase_dev.reserve(sr + 1);
-        const int* d_nroots = counters.ptr + 5;
-        MCE_RUN(k_ftr_gbase, dim3(1), dim3(64), 0, st, d_nroots, roots.ptr, boff, sr, gbase_dev.ptr);
-        fill_multi({{memcnt.ptr, (N + 1) * sizeof(int), 0}});
-        MCE_RUN(k_ftr_memcount, g1, b1, 0, st, N, d_nroots, smkey.ptr, memcnt.ptr);
-        MCE_RUN(k_ftr_memslots, g1, b1, 0, st, N, d_nroots, smval.ptr, perm.ptr, mem_slots.ptr);
-        scan_i32_excl(memcnt.ptr, memoff.ptr, N);
-        MCE_RUN(k_ftr_groups, g1, b1, 0, st, d_nroots, roots.ptr, perm.ptr, boff, sr, memcnt.ptr,
-                           memoff.ptr, grp_root.ptr, grp_moff.ptr, grp_mcnt.ptr, grp_m.ptr);
+        big_comp.reserve(waves);  // at most one per wavefront
+        Fc.reserve((size_t)(chunked ? kFtrChunks : 1) * N);
+        const dim3 g1(ceil_div(std::max(N, sr + 1), 256)), b1(256);
+        int* nbig = counters.ptr + kCtrBigComp;
+        MCE_DISPATCH_D(d, MCE_RUN(k_ftr_keys<DD>, g1, b1, 0, st, OUT, perm.ptr, N, boff, sr, dconst.ptr,
+                                  counters.ptr + kCtrNanP, fkeys.ptr, fidx.ptr));
+        sort_pairs(fkeys.ptr, fskeys.ptr, fidx.ptr, fsidx.ptr, N, 0, kFtrKeyBits);
+        MCE_DISPATCH_D(d, MCE_RUN(k_ftr_comp<DD>, dim3(ceil_div(waves, 4)), b1, 0, st, OUT, perm.ptr, N, boff,
+                                  dconst.ptr, fskeys.ptr, fsidx.ptr, rootpos.ptr, memrank.ptr, gval.ptr, nbig,
+                                  big_comp.ptr));
+        // a workgroup takes 8 listed components at a time, and at most one is listed per wavefront
+        const int bigb = std::max(1, std::min(1024, waves / 16));
+        MCE_DISPATCH_D(d, MCE_RUN(k_ftr_comp_big<DD>, dim3(bigb), dim3(kCompThreads), 0, st, OUT, perm.ptr, N,
+                                  boff, dconst.ptr, fskeys.ptr, fsidx.ptr, rootpos.ptr, memrank.ptr, gval.ptr, nbig,
+                                  big_comp.ptr, Fc.ptr));
+        scan_i64_excl(gval.ptr, groff.ptr, N);
+        MCE_RUN(k_ftr_emit, g1, b1, 0, st, N, boff, sr, perm.ptr, gval.ptr, groff.ptr, rootpos.ptr, memrank.ptr,
+                grp_root.ptr, grp_moff.ptr, grp_mcnt.ptr, grp_m.ptr, mem_slots.ptr, gbase_dev.ptr);
         HIPCHK(hipGetLastError());
-        // group offsets per shape; the last one is the root count
+        // group offsets per shape; the last one is the group count
         co_await rd(gbase_dev.ptr, gbase_of.data(), sr + 1);
         co_return gbase_of[sr];
     }

@@ -7,7 +7,7 @@
 //   k_mu               measurement update, one thread per output slot (parent x child)
 //   k_mom_terms/sum    fz / mean / covariance summands, then in-order sums per
 //                      reference thread (second stream, overlapped with reduction)
-//   k_ftr_*            fast term reduction of all shape buckets in single launches
+//   k_ftr_*            fast term reduction of all shape buckets: keys, components, groups
 //   k_group_btab       B-table of each reduction group's root, one wavefront per group
 //   k_group_eval       g-tables of each group: root, replacement chain, member sums
 //   k_group_sort       key order for groups whose root was replaced
@@ -30,6 +30,10 @@ constexpr uint32_t kGatherKeyNone = 0x3ffu;
 constexpr int kGatherKeyBits = 10;
 // Default: groups with more members than this add them with one wavefront per member.
 constexpr int kBigGroupMembers = 16;
+// Slots of an engine's device counters that more than one kernel knows.
+constexpr int kCtrMuErr = 17;     // measurement-update error bits
+constexpr int kCtrNanP = 24;      // set when a child's p holds a NaN
+constexpr int kCtrBigComp = 25;   // reduction components beyond one wavefront
 
 enum BtabMode : uint8_t { kModeNone = 0, kModeCopy = 1, kModeIdent = 2, kModeTrivial = 3, kModeEmpty = 4, kModeEnum = 5 };
 
@@ -253,6 +257,31 @@ __device__ __forceinline__ T wave_incl_scan(T x) {
         if (lane >= o) x += y;
     }
     return x;
+}
+
+// Largest input of the one-workgroup scans, and their threads.
+constexpr int kSmallScan = 65536;
+constexpr int kSmallScanThreads = 1024;
+
+// Exclusive prefix of each thread's `v` over a block of kSmallScanThreads threads, and the
+// block total: wavefront scans, then one wavefront scans the wavefront totals (two
+// barriers).  Every thread of the block must call it.
+template <class T>
+__device__ __forceinline__ T block_excl_scan(T v, T* total) {
+    constexpr int kWaves = kSmallScanThreads / kWave;
+    __shared__ T wsum[kWaves];
+    const int lane = (int)(threadIdx.x & (kWave - 1)), w = (int)(threadIdx.x / kWave);
+    const T x = wave_incl_scan(v);
+    if (lane == kWave - 1) wsum[w] = x;
+    __syncthreads();
+    if (w == 0) {
+        T y = lane < kWaves ? wsum[lane] : (T)0;
+        y = wave_incl_scan(y);
+        if (lane < kWaves) wsum[lane] = y;
+    }
+    __syncthreads();
+    *total = wsum[kWaves - 1];
+    return (w > 0 ? wsum[w - 1] : (T)0) + x - v;
 }
 
 // Exclusive prefix of each thread's v over a block of whole wavefronts (at most 4) and the
@@ -943,6 +972,9 @@ __device__ __forceinline__ void k_mu(MG<1024, 1> mg, TermPool IN, int np, const 
             mnew = dev_mu_coalign<D>(oA, op, oq, cm, cs, &hf, m, err);
             if (mnew < m) fl |= kHasCmap;
         }
+        bool nan_p = false;
+        for (int r = 0; r < mnew; r++) nan_p |= op[r] != op[r];
+        if (nan_p) atomicOr(err + (kCtrNanP - kCtrMuErr), 1);
     }
     OUT.hflag[s] = hf;
     OUT.flags[s] = fl;
@@ -1077,6 +1109,7 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
     for (int kk = 0; kk < D; kk++) ty[kk] = 0.0;
     double ygi = 0.0;
     uint32_t neg = 0, hf = 0;
+    bool nan_p = false;
     double x0[KM];
 #pragma unroll
     for (int r = 0; r < KM; r++) {
@@ -1101,6 +1134,7 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
                 for (int kk = 0; kk < D; kk++) n1 += fabs(row[kk]);
                 oq[r] = pr;
                 pr *= n1;
+                nan_p |= pr != pr;
 #pragma unroll
                 for (int kk = 0; kk < D; kk++) row[kk] /= n1;
                 x0[r] = fabs(row[0]);
@@ -1181,6 +1215,7 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
             }
         }
     }
+    if (nan_p) atomicOr(err + (kCtrNanP - kCtrMuErr), 1);
     OUT.hflag[s] = hf;
     OUT.flags[s] = fl;
     OUT.m[s] = mnew;
@@ -1425,288 +1460,7 @@ __device__ __forceinline__ void k_iota(MG<1024, 1> mg, uint32_t* __restrict__ v,
     if (i < n) v[i] = (uint32_t)i;
 }
 
-// ------------------------------------------------------------------ fast term reduction
-// All shape buckets are reduced together.  Global position p in [0, N) indexes the
-// gathered order (bucket m occupies [boff[m], boff[m+1]), slot perm[p]); reduction
-// decisions use bucket-local indices, as the reference reduces each bucket on its own
-// (fast_term_reduction_and_create_gtables, cauchy_estimator.hpp:1001-1137).
-__device__ inline int bucket_of(const int* __restrict__ boff, int nb, int p) {
-    int lo = 0, hi = nb - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (boff[mid] <= p) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
-// Chunk of local index l in a bucket of n terms: buckets above 10000 terms are reduced
-// in 8 chunks of n/8 (the last takes the rest), term_reduction.hpp:651-681.
-__device__ inline int ftr_chunk_of(int l, int n) {
-    if (n <= 10000) return 0;
-    const int c = l / (n / 8);
-    return c > 7 ? 7 : c;
-}
-
-__device__ __forceinline__ void k_ftr_keys(MG<1024, 1> mg, const TermPool OUT, const uint32_t* __restrict__ perm, int n, int d, int axis,
-                           uint64_t* __restrict__ keys, uint32_t* __restrict__ idx) {
-    const int p = mg.bx * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    keys[p] = f64_radix_key(OUT.b[(int64_t)perm[p] * d + axis]);
-    idx[p] = (uint32_t)p;
-}
-
-__device__ __forceinline__ void k_ftr_vals(MG<1024, 1> mg, const TermPool OUT, const uint32_t* __restrict__ perm, int n, int d, int axis,
-                           const uint32_t* __restrict__ sidx, double* __restrict__ vals) {
-    const int r = mg.bx * blockDim.x + threadIdx.x;
-    if (r >= n) return;
-    vals[r] = OUT.b[(int64_t)perm[sidx[r]] * d + axis];
-}
-
-// Bucket of each position of the value-sorted order (second, stable sort key).
-__device__ __forceinline__ void k_ftr_bkeys(MG<1024, 1> mg, int n, const int* __restrict__ boff, int nb, const uint32_t* __restrict__ sidx,
-                            uint32_t* __restrict__ bkey) {
-    const int r = mg.bx * blockDim.x + threadIdx.x;
-    if (r >= n) return;
-    bkey[r] = (uint32_t)bucket_of(boff, nb, (int)sidx[r]);
-}
-
-// Candidate pairs (i, j > i) of the greedy reduction, term_reduction.hpp:159-276:
-// b_j inside (b_i - ep, b_i + ep] on every axis (the window ftr_binary_search
-// selects, term_reduction.hpp:89-157, which must hold two points), then the p check
-// and the element-wise check over the first m flattened entries of A.  One thread
-// per sorted position; the window is found by scanning the sorted neighbours.
-// pass 0 counts, pass 1 writes the out-edges (global positions) of term i.
-template <int D>
-__device__ __forceinline__ void k_ftr_edges(MG<1024, 1> mg, const TermPool OUT, const uint32_t* __restrict__ perm, int n,
-                            const int* __restrict__ boff, int nb, const StepConst* __restrict__ sc,
-                            const double* __restrict__ vals, const uint32_t* __restrict__ sidx,
-                            int* __restrict__ cnt, const int* __restrict__ eoff, int* __restrict__ edges, int pass) {
-    const int sp = mg.bx * blockDim.x + threadIdx.x;
-    if (sp >= n) return;
-    const double ep = kReductionEps;
-    const int bk = bucket_of(boff, nb, sp);
-    const int beg = boff[bk], end = boff[bk + 1];
-    const int m = bk;  // bucket index is the shape
-    const int MM = OUT.MM;
-    const int ig = (int)sidx[sp];
-    const int il = ig - beg;
-    const int64_t si = perm[ig];
-    const double* bi = OUT.b + si * D;
-    const double* pi = OUT.p + si * MM;
-    const double* Ai = OUT.A + si * MM * D;
-    const double v = vals[sp];
-    const double lo = v - ep, hi = v + ep;
-    // r0 = first sorted position in the bucket with value > lo; r1 = first with value > hi
-    int r0 = sp;
-    if (vals[r0] > lo) {
-        while (r0 > beg && vals[r0 - 1] > lo) r0--;
-    } else {
-        while (r0 < end && vals[r0] <= lo) r0++;
-    }
-    int r1 = sp;
-    if (vals[r1] <= hi) {
-        while (r1 < end && vals[r1] <= hi) r1++;
-    } else {
-        while (r1 > beg && vals[r1 - 1] > hi) r1--;
-    }
-    int c = 0;
-    int w = pass ? eoff[ig] : 0;
-    if (r1 - r0 >= 2) {
-        for (int r = r0; r < r1; r++) {
-            const int jg = (int)sidx[r];
-            if (jg - beg <= il) continue;
-            const int64_t sj = perm[jg];
-            const double* bj = OUT.b + sj * D;
-            bool ok = true;
-            for (int a = 1; a < D && ok; a++) {
-                const int ax = sc->order[a];
-                const double l2 = bi[ax] - ep, h2 = bi[ax] + ep;
-                const double x = bj[ax];
-                if (!(x > l2 && x <= h2)) ok = false;
-            }
-            if (!ok) continue;
-            const double* pj = OUT.p + sj * MM;
-            for (int k = 0; k < m; k++)
-                if (fabs(pj[k] - pi[k]) > ep) {
-                    ok = false;
-                    break;
-                }
-            if (!ok) continue;
-            const double* Aj = OUT.A + sj * MM * D;
-            for (int k = 0; k < m; k++) {
-                const double x = Ai[k], y = Aj[k];
-                if (!((fabs(x - y) < ep) || (fabs(x + y) < ep))) {
-                    ok = false;
-                    break;
-                }
-            }
-            if (!ok) continue;
-            if (pass) edges[w++] = jg;
-            c++;
-        }
-    }
-    if (!pass) cnt[ig] = c;
-}
-
-// Pair-parallel candidate search.  k_ftr_gather copies what the predicate reads
-// into the value-sorted order: b (d), p (first m) and the first m entries of the
-// flattened A, row stride MM.
-template <int D>
-__device__ __forceinline__ void k_ftr_gather(MG<1024, 1> mg, const TermPool OUT, const uint32_t* __restrict__ perm, int n,
-                             const int* __restrict__ boff, int nb, const uint32_t* __restrict__ sidx,
-                             double* __restrict__ gb, double* __restrict__ gp, double* __restrict__ gA) {
-    const int r = mg.bx * blockDim.x + threadIdx.x;
-    if (r >= n) return;
-    const int m = bucket_of(boff, nb, r);
-    const int MM = OUT.MM;
-    const int64_t s = perm[sidx[r]];
-#pragma unroll
-    for (int a = 0; a < D; a++) gb[(int64_t)r * D + a] = OUT.b[s * D + a];
-    for (int q = 0; q < m; q++) {
-        gp[(int64_t)r * MM + q] = OUT.p[s * MM + q];
-        gA[(int64_t)r * MM + q] = OUT.A[s * MM * D + q];
-    }
-}
-
-// Window of sorted position sp on the first search axis: positions r0 <= r < r1 of
-// its bucket with value in (v - ep, v + ep] (a window must hold two points,
-// ftr_binary_search, term_reduction.hpp:89-157).  wcnt = r1 - r0, or 0.
-// Also clears each position's edge count for the edge passes that follow.
-__device__ __forceinline__ void k_ftr_win(MG<1024, 1> mg, int n, const int* __restrict__ boff, int nb, const double* __restrict__ vals,
-                          int* __restrict__ wlo, int64_t* __restrict__ wcnt, int* __restrict__ ecnt) {
-    const int sp = mg.bx * blockDim.x + threadIdx.x;
-    if (sp >= n) return;
-    ecnt[sp] = 0;
-    const int bk = bucket_of(boff, nb, sp);
-    const int beg = boff[bk], end = boff[bk + 1];
-    const double v = vals[sp];
-    const double lo = v - kReductionEps, hi = v + kReductionEps;
-    int a = beg, b = end;  // first position with value > lo
-    while (a < b) {
-        const int mid = (a + b) >> 1;
-        if (vals[mid] > lo) b = mid;
-        else a = mid + 1;
-    }
-    const int r0 = a;
-    a = beg;
-    b = end;  // first position with value > hi
-    while (a < b) {
-        const int mid = (a + b) >> 1;
-        if (vals[mid] > hi) b = mid;
-        else a = mid + 1;
-    }
-    const int r1 = a;
-    wlo[sp] = r0;
-    wcnt[sp] = (r1 - r0 >= 2) ? (int64_t)(r1 - r0) : 0;
-}
-
-// One thread per (position, window slot) pair: the rest of the greedy predicate,
-// term_reduction.hpp:159-276 (j > i, every other axis inside (b_i - ep, b_i + ep],
-// |p_j - p_i| <= ep on the first m, and the element-wise check on the first m
-// entries of the flattened A).  pass 0 flags the pair and counts term i's out-edges;
-// pass 1 writes the flagged pairs into term i's list (edge order within a list does
-// not matter to the resolution that follows).
-template <int D>
-__device__ __forceinline__ void k_ftr_pairs(MG<1024, 1> mg, int64_t npairs, int n, const int* __restrict__ boff, int nb,
-                            const StepConst* __restrict__ sc, const int64_t* __restrict__ woff,
-                            const int* __restrict__ wlo, const uint32_t* __restrict__ sidx, int MM,
-                            const double* __restrict__ gb, const double* __restrict__ gp,
-                            const double* __restrict__ gA, uint8_t* __restrict__ flag, int* __restrict__ ecnt,
-                            const int* __restrict__ eoff, int* __restrict__ cursor, int* __restrict__ edges,
-                            int pass) {
-    const int64_t q = (int64_t)mg.bx * blockDim.x + threadIdx.x;
-    if (q >= npairs) return;
-    // owning position: largest sp with woff[sp] <= q
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (woff[mid] <= q) lo = mid;
-        else hi = mid - 1;
-    }
-    const int sp = lo;
-    const int r = wlo[sp] + (int)(q - woff[sp]);
-    const int ig = (int)sidx[sp];
-    const int jg = (int)sidx[r];
-    if (pass == 1) {
-        if (flag[q]) {
-            const int slot = atomicAdd(&cursor[ig], 1);
-            edges[eoff[ig] + slot] = jg;
-        }
-        return;
-    }
-    bool ok = jg > ig;
-    if (ok) {
-        const double ep = kReductionEps;
-        const double* bi = gb + (int64_t)sp * D;
-        const double* bj = gb + (int64_t)r * D;
-        for (int a = 1; a < D && ok; a++) {
-            const int ax = sc->order[a];
-            const double l2 = bi[ax] - ep, h2 = bi[ax] + ep;
-            const double x = bj[ax];
-            if (!(x > l2 && x <= h2)) ok = false;
-        }
-        const int m = bucket_of(boff, nb, sp);
-        const double* pi = gp + (int64_t)sp * MM;
-        const double* pj = gp + (int64_t)r * MM;
-        for (int kk = 0; kk < m && ok; kk++)
-            if (fabs(pj[kk] - pi[kk]) > ep) ok = false;
-        const double* Ai = gA + (int64_t)sp * MM;
-        const double* Aj = gA + (int64_t)r * MM;
-        for (int kk = 0; kk < m && ok; kk++) {
-            const double x = Ai[kk], y = Aj[kk];
-            if (!((fabs(x - y) < ep) || (fabs(x + y) < ep))) ok = false;
-        }
-    }
-    flag[q] = ok ? 1 : 0;
-    if (ok) atomicAdd(&ecnt[ig], 1);
-}
-
-// In-degree over edges whose ends share a chunk (pass 0), or the in-edge lists (pass 1).
-__device__ __forceinline__ void k_ftr_inedges(MG<1024, 1> mg, int n, const int* __restrict__ boff, int nb, const int* __restrict__ eoff,
-                              const int* __restrict__ ecnt, const int* __restrict__ edges, int* __restrict__ indeg,
-                              const int* __restrict__ inoff, int* __restrict__ cursor, int* __restrict__ inedges,
-                              int pass) {
-    const int ig = mg.bx * blockDim.x + threadIdx.x;
-    if (ig >= n) return;
-    const int bk = bucket_of(boff, nb, ig);
-    const int beg = boff[bk], nbk = boff[bk + 1] - beg;
-    const int ci = ftr_chunk_of(ig - beg, nbk);
-    // Edges in batches of kInBatch: a batch's loads, then its atomics, are all in flight
-    // before the first result is used.  The order of a term's in-edges is immaterial (the
-    // rounds only ask whether any of them is a root, or all are claimed).
-    constexpr int kInBatch = 4;
-    const int e0 = eoff[ig], e1 = e0 + ecnt[ig];
-    for (int e = e0; e < e1; e += kInBatch) {
-        int jg[kInBatch];
-#pragma unroll
-        for (int u = 0; u < kInBatch; u++) jg[u] = e + u < e1 ? edges[e + u] : -1;
-#pragma unroll
-        for (int u = 0; u < kInBatch; u++)
-            if (jg[u] >= 0 && ftr_chunk_of(jg[u] - beg, nbk) != ci) jg[u] = -1;
-        if (pass == 0) {
-#pragma unroll
-            for (int u = 0; u < kInBatch; u++)
-                if (jg[u] >= 0) atomicAdd(&indeg[jg[u]], 1);
-        } else {
-            int slot[kInBatch], base[kInBatch];
-#pragma unroll
-            for (int u = 0; u < kInBatch; u++)
-                if (jg[u] >= 0) {
-                    slot[u] = atomicAdd(&cursor[jg[u]], 1);
-                    base[u] = inoff[jg[u]];
-                }
-#pragma unroll
-            for (int u = 0; u < kInBatch; u++)
-                if (jg[u] >= 0) inedges[base[u] + slot[u]] = ig;
-        }
-    }
-}
-
-enum { kUnknown = 0, kRoot = 1, kClaimed = 2 };
-
-// One round of root resolution: a term is a root of its chunk's greedy pass when
-// no same-chunk root before it claims it.
+// ------------------------------------------------------------------ fills
 // Up to kFillRegions byte fills in one launch: region blockIdx.y gets `bytes` copies of
 // `val`, by 32-bit words where the pointer allows, then the tail bytes.
 constexpr int kFillRegions = 6;
@@ -1732,156 +1486,488 @@ __device__ __forceinline__ void k_fill_multi(MG<1024, 1> mg, FillArgs f) {
     for (int64_t i = 4 * words + t; i < nb; i += stride) p[i] = (uint8_t)v;
 }
 
-// Round r counts its unresolved terms in slots[r % kRoundSlots] and clears the next
-// round's slot (no other thread of round r touches it, and round r + 1 starts after round r
-// ends), so the rounds need no fill between them.
-constexpr int kRoundSlots = 64;
-__device__ __forceinline__ void k_ftr_round(MG<1024, 1> mg, int n, const int* __restrict__ inoff, const int* __restrict__ indeg,
-                            const int* __restrict__ inedges, const uint8_t* __restrict__ st_in,
-                            uint8_t* __restrict__ st_out, int* __restrict__ slots, int r) {
-    const int j = mg.bx * blockDim.x + threadIdx.x;
-    if (j == 0) slots[(r + 1) % kRoundSlots] = 0;
-    int* unresolved = slots + r % kRoundSlots;
-    if (j >= n) return;
-    uint8_t s = st_in[j];
-    if (s == kUnknown) {
-        // in-edges in batches of kRoundBatch: a batch's index loads, then its state loads,
-        // are all in flight before the first is tested; padding counts as claimed
-        constexpr int kRoundBatch = 4;
-        bool any_root = false, all_claimed = true;
-        const int e0 = inoff[j], e1 = e0 + indeg[j];
-        for (int e = e0; e < e1 && !any_root; e += kRoundBatch) {
-            int src[kRoundBatch];
+// ------------------------------------------------------------------ fast term reduction
+// All shape buckets are reduced together.  Global position p in [0, N) indexes the
+// gathered order (bucket m occupies [boff[m], boff[m+1]), slot perm[p]); reduction
+// decisions use bucket-local indices, as the reference reduces each bucket on its own
+// (fast_term_reduction_and_create_gtables, cauchy_estimator.hpp:1001-1137).
+//
+// The reference looks for the terms that term i claims among those near it on one axis.
+// Many terms share that coordinate (children of one parent, long windows of few states), and
+// the pairs of a shared coordinate grow with the square of their number.  Here the terms are
+// sorted by one number that every compared quantity enters instead (k_ftr_keys): two terms
+// that reduce differ by at most a known bound in it, so every reduction stays inside a run of
+// sorted neighbours that are no further apart than that bound, a component.  Components are
+// almost always the reduction groups themselves.  The greedy pass then runs inside each
+// component, with the reference's own comparisons on the terms' values (ftr_edge), so
+// what reduces with what is unchanged: the sort only decides which pairs are compared.
+//   k_ftr_keys      sort key of each term
+//   k_ftr_comp      components of up to one wavefront: greedy pass, chunk merge, member ranks
+//   k_ftr_comp_big  the others, one workgroup each
+//   k_ftr_emit      reduction groups and member lists, after a scan over the roots
+// 718k terms of a 2-state, 20-hyperplane window: the pair search, its edge lists and the
+// resolution rounds took 78 ms per window (3.3 ms per pair pass, 1.2 ms per edge pass).
+__device__ inline int bucket_of(const int* __restrict__ boff, int nb, int p) {
+    int lo = 0, hi = nb - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (boff[mid] <= p) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+// Chunk of local index l in a bucket of n terms: buckets above 10000 terms are reduced
+// in 8 chunks of n/8 (the last takes the rest), term_reduction.hpp:651-681.
+constexpr int kFtrChunkTerms = 10000;
+constexpr int kFtrChunks = 8;
+__device__ inline int ftr_chunk_of(int l, int n) {
+    if (n <= kFtrChunkTerms) return 0;
+    const int c = l / (n / kFtrChunks);
+    return c > kFtrChunks - 1 ? kFtrChunks - 1 : c;
+}
+
+// Sort key: shape, then s = sum_k w_k f(x_k) over the d coordinates of b, the m scales p and
+// the first m entries of A in magnitude, in units of 2^-26.  f(x) = x / (1 + |x|) never moves
+// two numbers further apart than they were and w_k <= 1, so terms that reduce, each of whose
+// compared quantities differ by at most kReductionEps, differ by at most (d + 2m) 1e-8 in s.
+// |s| < 70 keeps the key in kFtrKeyBits bits.  The w_k are spread over [0.5, 1) so that terms
+// that only exchange values get different keys.
+constexpr int kFtrValueBits = 34;
+constexpr int kFtrKeyBits = kFtrValueBits + 5;
+// A NaN in p compares as equal to anything (ftr_edge), which no finite key can express: when
+// the measurement update saw one, p is left out of every key.
+template <int D>
+__device__ __forceinline__ void k_ftr_keys(MG<256, 1> mg, const TermPool OUT, const uint32_t* __restrict__ perm, int n,
+                                           const int* __restrict__ boff, int nb, const StepConst* __restrict__ sc,
+                                           const int* __restrict__ nan_p, uint64_t* __restrict__ keys,
+                                           uint32_t* __restrict__ idx) {
+    const int p = mg.bx * blockDim.x + threadIdx.x;
+    if (p >= n) return;
+    const int m = bucket_of(boff, nb, p);
+    const int64_t s = perm[p];
+    const double* b = OUT.b + s * D;
+    const double* pp = OUT.p + s * OUT.MM;
+    const double* A = OUT.A + s * OUT.MM * D;
+    auto weight = [](int k) {
+        const double t = (k + 1) * 0.6180339887498949;
+        return 0.5 + 0.5 * (t - floor(t));
+    };
+    auto squash = [](double x) {  // f(|x|); a NaN counts as infinite
+        const double u = fmin(fabs(x), 1e300);
+        return u / (1.0 + u);
+    };
+    double v = 128.0;
 #pragma unroll
-            for (int u = 0; u < kRoundBatch; u++) src[u] = e + u < e1 ? inedges[e + u] : -1;
-            uint8_t si[kRoundBatch];
+    for (int a = 0; a < D; a++) {
+        const double x = b[sc->order[a]];
+        v += weight(a) * copysign(squash(x), x);
+    }
+    const bool with_p = *nan_p == 0;
+    for (int k = 0; k < m; k++) {
+        if (with_p) v += weight(D + 2 * k) * copysign(squash(pp[k]), pp[k]);
+        v += weight(D + 2 * k + 1) * squash(A[k]);
+    }
+    keys[p] = ((uint64_t)m << kFtrValueBits) | (uint64_t)(v * (double)(1 << 26));
+    idx[p] = (uint32_t)p;
+}
+
+// Whether sorted neighbours belong to one component: same shape, and keys no further apart
+// than (d + 2m) 1e-8 in units of 2^-26, rounded up (two keys are floors of their values).
+template <int D>
+__device__ __forceinline__ bool ftr_linked(uint64_t prev, uint64_t cur) {
+    const int m = (int)(cur >> kFtrValueBits);
+    return (int)(prev >> kFtrValueBits) == m && cur - prev <= (uint64_t)((int)(0.672 * (D + 2 * m)) + 3);
+}
+
+// Whether term si (earlier) claims term sj (later) of shape m, term_reduction.hpp:89-276:
+// b_j inside (b_i - ep, b_i + ep] on every axis, |p_j - p_i| <= ep on the first m, and the
+// element-wise check over the first m flattened entries of A.
+template <int D>
+__device__ inline bool ftr_edge(const TermPool& O, int64_t si, int64_t sj, int m, const StepConst* __restrict__ sc,
+                                const uint32_t* __restrict__ perm, int beg, int end) {
+    const double ep = kReductionEps;
+    const double* bi = O.b + si * D;
+    const double* bj = O.b + sj * D;
+    bool ok = true;
 #pragma unroll
-            for (int u = 0; u < kRoundBatch; u++) si[u] = src[u] >= 0 ? st_in[src[u]] : (uint8_t)kClaimed;
+    for (int a = 0; a < D; a++) {
+        const int ax = sc->order[a];
+        const double v = bi[ax], x = bj[ax];
+        ok &= x > v - ep && x <= v + ep;
+    }
+    if (!ok) return false;
+    const double* pi = O.p + si * O.MM;
+    const double* pj = O.p + sj * O.MM;
+    const double* Ai = O.A + si * O.MM * D;
+    const double* Aj = O.A + sj * O.MM * D;
+    for (int k = 0; k < m; k++) {
+        const double x = Ai[k], y = Aj[k];
+        ok &= !(fabs(pj[k] - pi[k]) > ep) && (fabs(x - y) < ep || fabs(x + y) < ep);
+    }
+    if (!ok) return false;
+    // The window on the first axis must hold two points.  It holds i and j, unless b_i - ep
+    // rounds to b_i (magnitudes above 2^27), where i itself is outside its window.
+    const int a0 = sc->order[0];
+    const double v = bi[a0], lo = v - ep, hi = v + ep;
+    if (!(v > lo)) {
+        int c = 0;
+        for (int p = beg; p < end && c < 2; p++) {
+            const double x = O.b[(int64_t)perm[p] * D + a0];
+            c += x > lo && x <= hi;
+        }
+        return c >= 2;
+    }
+    return true;
+}
+
+// Components that begin in the first kCompOwn of 64 sorted positions are reduced by the
+// wavefront that looks at these 64, a lane per term; the next wavefront begins kCompOwn
+// positions on.  A component that does not end inside the 64 goes to big_list (at most one
+// per wavefront).  No list of all components is made or counted.
+//
+// Greedy pass: the least unclaimed term of a component is a root and claims every later
+// unclaimed term that ftr_edge accepts.  In a bucket above kFtrChunkTerms terms each chunk c
+// has its own pass (roots of chunk c claim terms of chunks >= c), and the eight results are
+// merged pairwise, term_reduction.hpp:592-649: F_c[j] is the root claiming j, else j, every
+// value of F_c is a fixed point of it, so a merge level is data parallel.  Roots, members and
+// merges never leave a component.
+constexpr int kCompOwn = 48;
+// Reduces the components that begin in the first `own` of the 64 sorted positions from `base`
+// (< n).  Returns the position of the one that does not end inside the 64, or -1.
+template <int D>
+__device__ __forceinline__ int ftr_comp_wave(const TermPool& OUT, const uint32_t* __restrict__ perm, int n,
+                                             const int* __restrict__ boff, const StepConst* __restrict__ sc,
+                                             const uint64_t* __restrict__ skeys, const uint32_t* __restrict__ sidx,
+                                             int* __restrict__ rootpos, int* __restrict__ rank,
+                                             int64_t* __restrict__ gval, int base, int own_starts) {
+    const int lane = wave_lane();
+    const int r = base + lane;
+    const bool in = r < n;
+    const uint64_t q = in ? skeys[r] : 0;
+    const bool start = !(in && r > 0 && ftr_linked<D>(skeys[r - 1], q));  // past the end: a start
+    const uint64_t starts = __ballot(start);
+    const uint64_t upto = starts & (~0ull >> (kWave - 1 - lane));
+    const int sb = upto ? kWave - 1 - __clzll((long long)upto) : -1;
+    const uint64_t after = lane == kWave - 1 ? 0ull : starts >> (lane + 1);
+    const int se = after ? lane + __ffsll((unsigned long long)after) : kWave;
+    const bool ends = base + kWave >= n || !ftr_linked<D>(skeys[base + kWave - 1], skeys[base + kWave]);
+    const bool own = in && sb >= 0 && sb < own_starts;
+    const bool mine = own && (se < kWave || ends);
+    const uint64_t open_start = __ballot(own && !mine && lane == sb);
+    const int size = mine ? se - sb : 1;
+    const uint64_t seg = mine ? ((se == kWave ? ~0ull : (1ull << se) - 1ull) & ~((1ull << sb) - 1ull)) : 0ull;
+    const int p = mine ? (int)sidx[r] : INT_MAX;
+    const int m = (int)(q >> kFtrValueBits);
+    const int beg = mine ? boff[m] : 0, end = mine ? boff[m + 1] : 0;
+    const int slot = mine ? (int)perm[p] : 0;
+    const int last = mine ? se - 1 : lane;
+    // one greedy pass over every component of the wavefront: `cand` may become roots, `open`
+    // may be claimed; returns the lane of each lane's root (its own if unclaimed)
+    auto greedy = [&](bool cand, bool open) {
+        int f = lane;
+        for (;;) {
+            int v = cand ? p : INT_MAX;
 #pragma unroll
-            for (int u = 0; u < kRoundBatch; u++) {
-                any_root |= si[u] == kRoot;
-                all_claimed &= si[u] == kClaimed;
+            for (int o = 1; o < kWave; o <<= 1) {
+                const int y = __shfl_up(v, o, kWave);
+                if (lane - o >= sb) v = min(v, y);
+            }
+            const int mn = __shfl(v, last, kWave);
+            const uint64_t roots = __ballot(cand && p == mn);
+            if (!roots) return f;
+            const uint64_t mr = roots & seg;
+            const int rl = mr ? __ffsll((unsigned long long)mr) - 1 : lane;
+            const int rs = __shfl(slot, rl, kWave);
+            if (mr) {
+                if (rl == lane) {
+                    cand = open = false;
+                } else if (open && p > mn && ftr_edge<D>(OUT, rs, slot, m, sc, perm, beg, end)) {
+                    f = rl;
+                    cand = open = false;
+                }
             }
         }
-        s = any_root ? kClaimed : (all_claimed ? kRoot : kUnknown);
-        if (s == kUnknown) atomicAdd(unresolved, 1);
-    }
-    st_out[j] = s;
-}
-
-// Flag arrays F_c (c < 8) over global positions, holding bucket-local indices:
-// F_c[j] = smallest chunk-c root claiming j, else j itself.  Buckets reduced in one
-// chunk use F_0 only.
-__device__ __forceinline__ void k_ftr_finit(MG<1024, 1> mg, int* __restrict__ F, int n, const int* __restrict__ boff, int nb) {
-    const int p = mg.bx * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    const int bk = bucket_of(boff, nb, p);
-    const int l = p - boff[bk];
-    const int nc = (boff[bk + 1] - boff[bk] > 10000) ? 8 : 1;
-    for (int c = 0; c < nc; c++) F[(int64_t)c * n + p] = l;
-}
-
-__device__ __forceinline__ void k_ftr_claim(MG<1024, 1> mg, int n, const int* __restrict__ boff, int nb, const int* __restrict__ eoff,
-                            const int* __restrict__ ecnt, const int* __restrict__ edges,
-                            const uint8_t* __restrict__ st, int* __restrict__ F) {
-    const int ig = mg.bx * blockDim.x + threadIdx.x;
-    if (ig >= n || st[ig] != kRoot) return;
-    const int bk = bucket_of(boff, nb, ig);
-    const int beg = boff[bk], nbk = boff[bk + 1] - beg;
-    const int il = ig - beg;
-    int* Fc = F + (int64_t)ftr_chunk_of(il, nbk) * n;
-    // edges in batches of four: the batch's loads are in flight together, then its minima
-    const int e0 = eoff[ig], e1 = e0 + ecnt[ig];
-    for (int e = e0; e < e1; e += 4) {
-        int jg[4];
+    };
+    const int nbk = end - beg;
+    const bool multi = mine && size > 1;
+    int f0;
+    if (!__any(multi && nbk > kFtrChunkTerms)) {
+        f0 = greedy(multi, multi);
+    } else {
+        const int c0 = multi ? ftr_chunk_of(p - beg, nbk) : -1;
+        int F[kFtrChunks];
 #pragma unroll
-        for (int u = 0; u < 4; u++) jg[u] = e + u < e1 ? edges[e + u] : -1;
+        for (int c = 0; c < kFtrChunks; c++) F[c] = __any(c0 == c) ? greedy(c0 == c, c0 >= c) : lane;
 #pragma unroll
-        for (int u = 0; u < 4; u++)
-            if (jg[u] >= 0) atomicMin(&Fc[jg[u]], il);
+        for (int lvl = 0; lvl < 3; lvl++)
+#pragma unroll
+            for (int k = 0; k < (kFtrChunks >> (lvl + 1)); k++) {
+                const int rt = k << (lvl + 1), cm = rt + (1 << lvl);
+                const int f2 = F[cm];
+                const int x = __shfl(F[rt], f2, kWave);
+                if (nbk > kFtrChunkTerms && p - beg >= cm * (nbk / kFtrChunks) && f2 != lane && F[rt] == lane)
+                    F[rt] = x == f2 ? f2 : x;
+            }
+        f0 = F[0];
+    }
+    // members of each root, and each member's rank among them
+    int cnt = 0, less = 0;
+    for (int k = 1; __any(k < size); k++) {
+        int pl = lane + k;
+        if (pl >= se) pl -= size;
+        pl = k < size ? pl : lane;
+        const int pf = __shfl(f0, pl, kWave), pp = __shfl(p, pl, kWave);
+        if (k < size) {
+            cnt += pf == lane;
+            less += pf == f0 && pl != f0 && pp < p;
+        }
+    }
+    const int rp = __shfl(p, f0, kWave);
+    if (mine) {
+        rootpos[p] = rp;
+        rank[p] = less;
+        gval[p] = ((int64_t)(f0 == lane) << 32) | (uint32_t)cnt;
+    }
+    return open_start ? base + __ffsll((unsigned long long)open_start) - 1 : -1;
+}
+
+template <int D>
+__device__ __forceinline__ void k_ftr_comp(MG<256, 1> mg, const TermPool OUT, const uint32_t* __restrict__ perm, int n,
+                                           const int* __restrict__ boff, const StepConst* __restrict__ sc,
+                                           const uint64_t* __restrict__ skeys, const uint32_t* __restrict__ sidx,
+                                           int* __restrict__ rootpos, int* __restrict__ rank,
+                                           int64_t* __restrict__ gval, int* __restrict__ big_count,
+                                           int* __restrict__ big_list) {
+    const int base = (mg.bx * (blockDim.x / kWave) + threadIdx.x / kWave) * kCompOwn;
+    if (base >= n) return;
+    const int open = ftr_comp_wave<D>(OUT, perm, n, boff, sc, skeys, sidx, rootpos, rank, gval, base, kCompOwn);
+    if (open >= 0 && wave_lane() == 0) big_list[atomicAdd(big_count, 1)] = open;
+}
+
+// The component that begins at sorted position r0 and ends before r1, of any size, by T
+// threads: one wavefront, or (T > 64) a workgroup with T / 64 words of LDS in wred and wsum.
+// F: the flag arrays, indexed by sorted position.
+template <int D, int T>
+__device__ __forceinline__ void ftr_comp_many(const TermPool& OUT, const uint32_t* __restrict__ perm, int n,
+                                              const int* __restrict__ boff, const StepConst* __restrict__ sc,
+                                              const uint64_t* __restrict__ skeys, const uint32_t* __restrict__ sidx,
+                                              int* __restrict__ rootpos, int* __restrict__ rank,
+                                              int64_t* __restrict__ gval, int* __restrict__ F, int r0, int r1,
+                                              unsigned long long* wred, int* wsum) {
+    const int lane = wave_lane(), t = T == kWave ? lane : (int)threadIdx.x, w = t / kWave;
+    auto sync = [&]() {
+        if constexpr (T == kWave) {
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            __syncthreads();
+        }
+    };
+    // the minimum over all threads; what they wrote to F before is visible afterwards
+    auto least = [&](unsigned long long v) {
+        for (int o = kWave / 2; o > 0; o >>= 1) v = min(v, (unsigned long long)__shfl_xor(v, o, kWave));
+        sync();
+        if constexpr (T > kWave) {
+            if (lane == 0) wred[w] = v;
+            __syncthreads();
+            for (int k = 0; k < T / kWave; k++) v = min(v, wred[k]);
+        }
+        return v;
+    };
+    // set flags before this thread's, and of all threads
+    auto count = [&](bool flag, int* total) {
+        const uint64_t b = __ballot(flag);
+        int x = __popcll(b & ((1ull << lane) - 1ull)), all = __popcll(b);
+        if constexpr (T > kWave) {
+            __syncthreads();
+            if (lane == 0) wsum[w] = all;
+            __syncthreads();
+            all = 0;
+            for (int k = 0; k < T / kWave; k++) {
+                x += k < w ? wsum[k] : 0;
+                all += wsum[k];
+            }
+        }
+        *total = all;
+        return x;
+    };
+    const int m = (int)(skeys[r0] >> kFtrValueBits);
+    const int beg = boff[m], end = boff[m + 1], nbk = end - beg;
+    const int nc = nbk > kFtrChunkTerms ? kFtrChunks : 1;
+    for (int c = 0; c < nc; c++)
+        for (int r = r0 + t; r < r1; r += T) F[(int64_t)c * n + r] = r;
+    for (int c = 0; c < nc; c++) {
+        int* Fc = F + (int64_t)c * n;
+        for (int last = -1;;) {
+            unsigned long long v = ~0ull;
+            for (int r = r0 + t; r < r1; r += T) {
+                const int p = (int)sidx[r];
+                if (p > last && Fc[r] == r && ftr_chunk_of(p - beg, nbk) == c)
+                    v = min(v, ((unsigned long long)p << 32) | (unsigned)r);
+            }
+            v = least(v);
+            if (v == ~0ull) break;
+            const int rr = (int)(v & 0xffffffffu);
+            last = (int)(v >> 32);
+            const int64_t rs = perm[last];
+            for (int r = r0 + t; r < r1; r += T) {
+                const int p = (int)sidx[r];
+                if (p > last && Fc[r] == r && ftr_edge<D>(OUT, rs, perm[p], m, sc, perm, beg, end)) Fc[r] = rr;
+            }
+        }
+    }
+    for (int lvl = 0; nc > 1 && lvl < 3; lvl++) {
+        sync();
+        for (int k = 0; k < (kFtrChunks >> (lvl + 1)); k++) {
+            const int rt = k << (lvl + 1), cm = rt + (1 << lvl);
+            int* F1 = F + (int64_t)rt * n;
+            const int* F2 = F + (int64_t)cm * n;
+            for (int r = r0 + t; r < r1; r += T) {
+                if ((int)sidx[r] - beg < cm * (nbk / kFtrChunks)) continue;
+                const int f2 = F2[r];
+                if (f2 != r && F1[r] == r) F1[r] = F1[f2] == f2 ? f2 : F1[f2];
+            }
+        }
+    }
+    sync();
+    // members of each root and their ranks.  In term order (equal keys: the sort is stable):
+    // one prefix count per root, unless roots are many; else every pair of terms is compared.
+    const bool in_order = skeys[r0] == skeys[r1 - 1];
+    const int most = (r1 - r0) / kWave;
+    bool done = false;
+    for (int last = -1, k = 0; in_order && k <= most; k++) {
+        unsigned long long v = ~0ull;
+        for (int r = r0 + t; r < r1; r += T)
+            if (F[r] == r && r > last) {
+                v = (unsigned long long)r;
+                break;
+            }
+        v = least(v);
+        done = v == ~0ull;
+        if (done) break;
+        last = (int)v;
+        int before = 0;
+        for (int b = r0; b < r1; b += T) {
+            const int r = b + t;
+            const bool mem = r < r1 && r != last && F[r] == last;
+            int tot;
+            const int x = count(mem, &tot);
+            if (mem) {
+                const int p = (int)sidx[r];
+                rootpos[p] = (int)sidx[last];
+                rank[p] = before + x;
+                gval[p] = 0;
+            }
+            before += tot;
+        }
+        if (t == 0) {
+            const int p = (int)sidx[last];
+            rootpos[p] = p;
+            rank[p] = 0;
+            gval[p] = ((int64_t)1 << 32) | (uint32_t)before;
+        }
+    }
+    if (done) return;
+    for (int b = r0 + w * kWave; b < r1; b += T) {
+        const int r = b + lane;
+        const int f0 = r < r1 ? F[r] : -1, p = r < r1 ? (int)sidx[r] : 0;
+        int cnt = 0, less = 0;
+        for (int q0 = r0; q0 < r1; q0 += kWave) {
+            const int nq = min(kWave, r1 - q0);
+            const int fq = lane < nq ? F[q0 + lane] : -1, pq = lane < nq ? (int)sidx[q0 + lane] : 0;
+            for (int k = 0; k < nq; k++) {
+                const int fk = __shfl(fq, k, kWave), pk = __shfl(pq, k, kWave);
+                const int q = q0 + k;
+                cnt += fk == r && q != r;
+                less += fk == f0 && q != f0 && pk < p;
+            }
+        }
+        if (r < r1) {
+            rootpos[p] = (int)sidx[f0];
+            rank[p] = less;
+            gval[p] = ((int64_t)(f0 == r) << 32) | (uint32_t)cnt;
+        }
     }
 }
 
-// One level of the flag-array merge tree of every 8-chunk bucket,
-// term_reduction.hpp:592-649.  Every value of a flag array is a fixed point of it,
-// so a level is data parallel.
-__device__ __forceinline__ void k_ftr_merge(MG<1024, 1> mg, int n, const int* __restrict__ boff, int nb, int* __restrict__ F, int level) {
-    const int p = mg.bx * blockDim.x + threadIdx.x;
-    const int k = mg.by;
-    if (p >= n) return;
-    const int bk = bucket_of(boff, nb, p);
-    const int beg = boff[bk], nbk = boff[bk + 1] - beg;
-    if (nbk <= 10000) return;
-    const int pairs = 8 >> (level + 1);
-    if (k >= pairs) return;
-    const int rt = k * (1 << (level + 1));
-    const int cm = rt + (1 << level);
-    const int l = p - beg;
-    if (l < cm * (nbk / 8)) return;
-    int* F1 = F + (int64_t)rt * n + beg;
-    const int* F2 = F + (int64_t)cm * n + beg;
-    const int f2 = F2[l];
-    if (f2 != -1 && f2 != l && F1[l] == l) F1[l] = (F1[f2] == f2) ? f2 : F1[f2];
-}
-
-// Root flags; members are keyed by their root's global position, roots by n.
-__device__ __forceinline__ void k_ftr_rootflags(MG<1024, 1> mg, int n, const int* __restrict__ boff, int nb, const int* __restrict__ F,
-                                uint8_t* __restrict__ isroot, uint32_t* __restrict__ memkey,
-                                uint32_t* __restrict__ memval) {
-    const int p = mg.bx * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    const int beg = boff[bucket_of(boff, nb, p)];
-    const int f = F[p];
-    const bool r = (f == p - beg);
-    isroot[p] = r;
-    memkey[p] = r ? (uint32_t)n : (uint32_t)(beg + f);
-    memval[p] = (uint32_t)p;
-}
-
-// The root count is read on the device (grids are sized by the term count n).
-__device__ __forceinline__ void k_ftr_memcount(MG<1024, 1> mg, int n, const int* __restrict__ nroots, const uint32_t* __restrict__ skey,
-                               int* __restrict__ cnt) {
-    const int k = mg.bx * blockDim.x + threadIdx.x;
-    if (k >= n - *nroots) return;
-    atomicAdd(&cnt[skey[k]], 1);
-}
-
-__device__ __forceinline__ void k_ftr_memslots(MG<1024, 1> mg, int n, const int* __restrict__ nroots, const uint32_t* __restrict__ sval,
-                               const uint32_t* __restrict__ perm, int* __restrict__ mem_slots) {
-    const int k = mg.bx * blockDim.x + threadIdx.x;
-    if (k >= n - *nroots) return;
-    mem_slots[k] = (int)perm[sval[k]];
-}
-
-// First reduction group of every bucket: gbase[m] = number of roots before boff[m].
-__device__ __forceinline__ void k_ftr_gbase(MG<1024, 1> mg, const int* __restrict__ d_nroots, const uint32_t* __restrict__ roots,
-                            const int* __restrict__ boff, int nb, int* __restrict__ gbase) {
-    const int m = threadIdx.x;
-    if (m > nb) return;
-    const int nroots = *d_nroots;
-    const uint32_t x = (uint32_t)boff[m];
-    int lo = 0, hi = nroots;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (roots[mid] < x) lo = mid + 1;
-        else hi = mid;
+// The listed components.  Most only straddled the end of their wavefront's positions: a
+// wavefront takes each and reduces it as above from its own first position.  Up to
+// kCompWave terms it goes through them 64 at a time; a workgroup takes what is larger.
+// Long windows of few states have components of thousands of terms that all reduce into one
+// (16269 in a 10-step window of 2 states).  The F arrays (8 of n ints when a bucket is reduced
+// in chunks, else one) belong to these components alone.
+constexpr int kCompWave = 1024;
+constexpr int kCompThreads = 512;
+template <int D>
+__device__ __forceinline__ void k_ftr_comp_big(MG<kCompThreads, 1> mg, const TermPool OUT,
+                                               const uint32_t* __restrict__ perm, int n, const int* __restrict__ boff,
+                                               const StepConst* __restrict__ sc, const uint64_t* __restrict__ skeys,
+                                               const uint32_t* __restrict__ sidx, int* __restrict__ rootpos,
+                                               int* __restrict__ rank, int64_t* __restrict__ gval,
+                                               const int* __restrict__ big_count, const int* __restrict__ big_list,
+                                               int* __restrict__ F) {
+    constexpr int kWaves = kCompThreads / kWave;
+    __shared__ unsigned long long wred[kWaves];
+    __shared__ int wsum[kWaves];
+    __shared__ int2 large[kWaves];
+    const int lane = wave_lane(), w = threadIdx.x / kWave;
+    const int count = *big_count;
+    for (int e0 = mg.bx * kWaves; e0 < count; e0 += mg.gx * kWaves) {
+        int r0 = -1, r1 = -1;
+        if (e0 + w < count)
+            r0 = ftr_comp_wave<D>(OUT, perm, n, boff, sc, skeys, sidx, rootpos, rank, gval, big_list[e0 + w], 1);
+        if (r0 >= 0) {
+            for (int b = r0 + 1; r1 < 0; b += kWave) {  // ends: positions past n stop it
+                const int r = b + lane;
+                const uint64_t stop = __ballot(r >= n || !ftr_linked<D>(skeys[r - 1], skeys[r]));
+                if (stop) r1 = min(n, b + __ffsll((unsigned long long)stop) - 1);
+            }
+            if (r1 - r0 <= kCompWave) {
+                ftr_comp_many<D, kWave>(OUT, perm, n, boff, sc, skeys, sidx, rootpos, rank, gval, F, r0, r1, nullptr,
+                                        nullptr);
+                r0 = -1;
+            }
+        }
+        __syncthreads();  // the previous round's list has been read
+        if (lane == 0) large[w] = make_int2(r0, r1);
+        __syncthreads();
+        for (int e = 0; e < kWaves; e++)
+            if (large[e].x >= 0)
+                ftr_comp_many<D, kCompThreads>(OUT, perm, n, boff, sc, skeys, sidx, rootpos, rank, gval, F, large[e].x,
+                                               large[e].y, wred, wsum);
     }
-    gbase[m] = lo;
 }
 
-// Reduction groups in the reference's order: buckets ascending, roots ascending.
-__device__ __forceinline__ void k_ftr_groups(MG<1024, 1> mg, const int* __restrict__ nroots, const uint32_t* __restrict__ roots,
-                             const uint32_t* __restrict__ perm, const int* __restrict__ boff, int nb,
-                             const int* __restrict__ memcnt, const int* __restrict__ memoff,
-                             int* __restrict__ grp_root, int* __restrict__ grp_moff, int* __restrict__ grp_mcnt,
-                             int* __restrict__ grp_m) {
-    const int g = mg.bx * blockDim.x + threadIdx.x;
-    if (g >= *nroots) return;
-    const uint32_t r = roots[g];
-    grp_root[g] = (int)perm[r];
-    grp_moff[g] = memoff[r];
-    grp_mcnt[g] = memcnt[r];
-    grp_m[g] = bucket_of(boff, nb, (int)r);
+// Reduction groups in the reference's order: buckets ascending, roots ascending, members
+// ascending per root.  goff is the exclusive scan of gval: groups before position p in its
+// upper half, members before it in its lower.  gbase[m]: first group of shape m; gbase[nb]:
+// their number.
+__device__ __forceinline__ void k_ftr_emit(MG<256, 1> mg, int n, const int* __restrict__ boff, int nb,
+                                           const uint32_t* __restrict__ perm, const int64_t* __restrict__ gval,
+                                           const int64_t* __restrict__ goff, const int* __restrict__ rootpos,
+                                           const int* __restrict__ rank, int* __restrict__ grp_root,
+                                           int* __restrict__ grp_moff, int* __restrict__ grp_mcnt,
+                                           int* __restrict__ grp_m, int* __restrict__ mem_slots,
+                                           int* __restrict__ gbase) {
+    const int p = mg.bx * blockDim.x + threadIdx.x;
+    if (p <= nb) {
+        const int f = boff[p];
+        gbase[p] = (int)((f < n ? goff[f] : goff[n - 1] + gval[n - 1]) >> 32);
+    }
+    if (p >= n) return;
+    const int64_t v = gval[p];
+    const int slot = (int)perm[p];
+    if (v >> 32) {
+        const int64_t o = goff[p];
+        const int g = (int)(o >> 32);
+        grp_root[g] = slot;
+        grp_moff[g] = (int)(uint32_t)o;
+        grp_mcnt[g] = (int)(uint32_t)v;
+        grp_m[g] = bucket_of(boff, nb, p);
+    } else {
+        mem_slots[(int)(uint32_t)goff[rootpos[p]] + rank[p]] = slot;
+    }
 }
 
 // ------------------------------------------------------------------ group B-tables
@@ -2760,42 +2846,18 @@ __device__ __forceinline__ void k_scan_total_mapped(MG<1024, 1> mg, const A* __r
     if (host_out) *(volatile int64_t*)host_out = v;
 }
 
-// Scan of up to kSmallScan items by one workgroup: the small arrays of small estimators,
-// where a library scan costs more launches than work.  Each thread sums a contiguous run, a
-// block scan of the run sums gives each run's offset, and the run is written out.  With
-// `wide`, the input is also stored widened; with `out_total` / `host_total`, the sum of all
-// items goes to a device scalar and a device-mapped host slot.  Integer sums, so the result
-// is the same as any other summation order's.
-constexpr int kSmallScan = 65536;
-constexpr int kSmallScanThreads = 1024;
-
-// Exclusive prefix of each thread's `v` over a block of kSmallScanThreads threads, and the
-// block total: wavefront scans, then one wavefront scans the wavefront totals (two
-// barriers).  Every thread of the block must call it.
-template <class T>
-__device__ __forceinline__ T block_excl_scan(T v, T* total) {
-    constexpr int kWaves = kSmallScanThreads / kWave;
-    __shared__ T wsum[kWaves];
-    const int lane = (int)(threadIdx.x & (kWave - 1)), w = (int)(threadIdx.x / kWave);
-    const T x = wave_incl_scan(v);
-    if (lane == kWave - 1) wsum[w] = x;
-    __syncthreads();
-    if (w == 0) {
-        T y = lane < kWaves ? wsum[lane] : (T)0;
-        y = wave_incl_scan(y);
-        if (lane < kWaves) wsum[lane] = y;
-    }
-    __syncthreads();
-    *total = wsum[kWaves - 1];
-    return (w > 0 ? wsum[w - 1] : (T)0) + x - v;
-}
-
 // Items per thread of one tile of the small scan.  Above one tile, tiles of
 // kSmallScanThreads x kScanItems items are loaded coalesced (consecutive threads,
 // consecutive items) into LDS, each thread scans its kScanItems consecutive items there,
 // and the results go back out coalesced.
 constexpr int kScanItems = 4;
 
+// Scan of up to kSmallScan items by one workgroup: the small arrays of small estimators,
+// where a library scan costs more launches than work.  Each thread sums a contiguous run, a
+// block scan of the run sums gives each run's offset, and the run is written out.  With
+// `wide`, the input is also stored widened; with `out_total` / `host_total`, the sum of all
+// items goes to a device scalar and a device-mapped host slot.  Integer sums, so the result
+// is the same as any other summation order's.
 template <class In, class Out, bool Inclusive>
 __device__ __forceinline__ void k_small_scan(MG<kSmallScanThreads, 1> mg, const In* __restrict__ in,
                                              Out* __restrict__ out, int n, Out* __restrict__ wide,
@@ -3709,24 +3771,6 @@ __device__ __forceinline__ void k_small_sort(MG<kSmallSortThreads, 1> mg, const 
             vout[i] = v[j];
         }
     }
-}
-
-// Stable compaction of in[i] where flags[i] != 0 for up to kSmallScan items in one
-// workgroup, with the selected count in *count (a device select's result).
-__device__ __forceinline__ void k_small_select(MG<kSmallScanThreads, 1> mg, const uint32_t* __restrict__ in,
-                                               const uint8_t* __restrict__ flags, uint32_t* __restrict__ out,
-                                               int* __restrict__ count, int n) {
-    (void)mg;
-    const int t = threadIdx.x;
-    const int per = (n + kSmallScanThreads - 1) / kSmallScanThreads;
-    const int b = min(n, t * per), e = min(n, b + per);
-    int c = 0;
-    for (int i = b; i < e; i++) c += flags[i] != 0;
-    int tot;
-    int w = block_excl_scan(c, &tot);
-    for (int i = b; i < e; i++)
-        if (flags[i]) out[w++] = in[i];
-    if (t == kSmallScanThreads - 1) count[0] = tot;
 }
 
 // Largest of n ints in one workgroup (INT_MIN when n = 0, as a device max
