@@ -2141,9 +2141,9 @@ struct Engine {
     DBuf<uint8_t> rs_keep;
     DBuf<int> rs_idx, rs_cnt;
     DBuf<int> c2_mc, c2_err;
-    DBuf<double> c2_b2, c2_sn, c2_cs, c2_g1r, c2_g2r, c2_px, c2_py;
-    DBuf<cplx> c2_g;
-    DBuf<Cell2D> c2_fc;
+    DBuf<double> c2_b2, c2_px, c2_py;
+    DBuf<Wall2D> c2_wall;
+    DBuf<Cell2D> c2_cell;
 
     // Extended-mode finish of a measurement update (cauchy_estimator.hpp:1358-1394): the
     // terms' b-vectors move by -Re(mean) (skipped on a window's last update), the mean
@@ -2249,7 +2249,7 @@ int Engine::cpdf_1d_into(int marg, double lo, double hi, double res, double* xs_
         if (npts > 1) {
             MCE_LAUNCH(k_cpdf1d_grid, dim3(ceil_div(npts - 1, kCpdfPoints), nchunks), dim3(kCpdfPoints), 0, s, cache,
                        Nt, xs_dev + 1, npts - 1, part);
-            MCE_LAUNCH(k_cpdf1d_finish, dim3(ceil_div(npts - 1, 256)), dim3(256), 0, s, part, nchunks, npts - 1, norm,
+            MCE_LAUNCH(k_cpdf1d_finish, dim3(ceil_div(npts - 1, kFinishPoints)), dim3(kFinishPoints * kFinishSlices), 0, s, part, nchunks, npts - 1, norm,
                        ys_dev + 1);
         }
         MCE_LAUNCH(k_cpdf1d_first, dim3(1), dim3(64), 0, s, dsum, norm, ys_dev, 0);
@@ -2289,7 +2289,7 @@ int Engine::cpdf_1d(int marg, double lo, double hi, double res, std::vector<doub
         if (npts > 1) {
             MCE_LAUNCH(k_cpdf1d_grid, dim3(ceil_div(npts - 1, kCpdfPoints), nchunks), dim3(kCpdfPoints), 0, st,
                                cpdf_cache.ptr, Nt, cpdf_x.ptr + 1, npts - 1, cpdf_part.ptr);
-            MCE_LAUNCH(k_cpdf1d_finish, dim3(ceil_div(npts - 1, 256)), dim3(256), 0, st, cpdf_part.ptr,
+            MCE_LAUNCH(k_cpdf1d_finish, dim3(ceil_div(npts - 1, kFinishPoints)), dim3(kFinishPoints * kFinishSlices), 0, st, cpdf_part.ptr,
                                nchunks, npts - 1, norm, cpdf_y.ptr + 1);
             HIPCHK(hipGetLastError());
             HIPCHK(hipMemcpyAsync(ys.data() + 1, cpdf_y.ptr + 1, (npts - 1) * sizeof(double), hipMemcpyDeviceToHost,
@@ -2312,6 +2312,28 @@ void Engine::draw_bar_nu() {
     if (!bar_nu.empty()) return;
     bar_nu.resize(d);
     for (int i = 0; i < d; i++) bar_nu[i] = 2 * (((double)rand() + 1.0) / ((double)RAND_MAX + 2.0));
+}
+
+// How a 2D grid's work is split: points per lane and terms per workgroup.  Two points per
+// lane halve the wall reads per point once there are points for it; chunks shrink from
+// kCpdfChunk terms until about 2048 workgroups share the grid (8 per CU), so that a small
+// estimator's density is not one workgroup's serial walk over its terms.
+struct Grid2DShape {
+    int points, terms, chunks;
+    Grid2DShape(int n, int npts) : points(npts >= 2048 ? 2 : 1), terms(kCpdfChunk) {
+        const int64_t cols = ceil_div(npts, kGridLanes * points);
+        while (terms > 64 && cols * ceil_div(n, terms) < 2048) terms /= 2;
+        chunks = ceil_div(n, terms);
+    }
+};
+
+static void launch_grid_2d(hipStream_t st, const Cpdf2D& C, int n, const Grid2DShape& g, const int* idx,
+                           const double* px, const double* py, int npts, double* part, int* err) {
+    const dim3 grid(ceil_div(npts, kGridLanes * g.points), g.chunks), block(kGridLanes * kGridWaves);
+    if (g.points == 2)
+        MCE_LAUNCH((k_cpdf2d_grid<2>), grid, block, 0, st, C, n, g.terms, idx, px, py, npts, part, err);
+    else
+        MCE_LAUNCH((k_cpdf2d_grid<1>), grid, block, 0, st, C, n, g.terms, idx, px, py, npts, part, err);
 }
 
 int Engine::cpdf_2d(int i1, int i2, double lox, double hix, double resx, double loy, double hiy, double resy,
@@ -2344,16 +2366,13 @@ int Engine::cpdf_2d(int i1, int i2, double lox, double hix, double resx, double 
     const double R = kInvTwoPi;
     if (Nt > 0) {
         GraveyardScope gs(&graveyard);
-        const int nchunks = ceil_div(Nt, kCpdfChunk);
+        const Grid2DShape shape(Nt, std::max(npts - 1, 1));
+        const int nchunks = shape.chunks;
         const size_t cells = (size_t)Nt * MM;
         c2_mc.reserve(Nt);
         c2_b2.reserve(2 * (size_t)Nt);
-        c2_sn.reserve(cells + Nt);
-        c2_cs.reserve(cells + Nt);
-        c2_g1r.reserve(cells);
-        c2_g2r.reserve(cells);
-        c2_g.reserve(cells);
-        c2_fc.reserve(cells);
+        c2_wall.reserve(cells + Nt);
+        c2_cell.reserve(cells);
         c2_err.reserve(1);
         c2_px.reserve(npts);
         c2_py.reserve(npts);
@@ -2368,12 +2387,8 @@ int Engine::cpdf_2d(int i1, int i2, double lox, double hix, double resx, double 
         C.MM = MM;
         C.mc = c2_mc.ptr;
         C.b2 = c2_b2.ptr;
-        C.sn = c2_sn.ptr;
-        C.cs = c2_cs.ptr;
-        C.g1r = c2_g1r.ptr;
-        C.g2r = c2_g2r.ptr;
-        C.gc = c2_g.ptr;
-        C.fc = c2_fc.ptr;
+        C.wall = c2_wall.ptr;
+        C.cell = c2_cell.ptr;
         VecArg bn;
         for (int i = 0; i < d; i++) bn.v[i] = bar_nu[i];
         TermPool IN = in.view();
@@ -2382,10 +2397,8 @@ int Engine::cpdf_2d(int i1, int i2, double lox, double hix, double resx, double 
                                              cpdf_direct.ptr, c2_err.ptr));
         MCE_LAUNCH(k_sum_fixed, dim3(1), dim3(1024), 0, st, cpdf_direct.ptr, Nt, cpdf_sum.ptr);
         if (npts > 1) {
-            MCE_LAUNCH(k_cpdf2d_grid, dim3(ceil_div(npts - 1, kCpdfPoints), nchunks), dim3(kCpdfPoints), 0, st,
-                               C, Nt, (const int*)nullptr, c2_px.ptr + 1, c2_py.ptr + 1, npts - 1, cpdf_part.ptr,
-                               c2_err.ptr);
-            MCE_LAUNCH(k_cpdf1d_finish, dim3(ceil_div(npts - 1, 256)), dim3(256), 0, st, cpdf_part.ptr,
+            launch_grid_2d(st, C, Nt, shape, nullptr, c2_px.ptr + 1, c2_py.ptr + 1, npts - 1, cpdf_part.ptr, c2_err.ptr);
+            MCE_LAUNCH(k_cpdf1d_finish, dim3(ceil_div(npts - 1, kFinishPoints)), dim3(kFinishPoints * kFinishSlices), 0, st, cpdf_part.ptr,
                                nchunks, npts - 1, 1.0, cpdf_y.ptr + 1);
             HIPCHK(hipGetLastError());
             HIPCHK(hipMemcpyAsync(zs.data() + 1, cpdf_y.ptr + 1, (npts - 1) * sizeof(double), hipMemcpyDeviceToHost,
@@ -2445,7 +2458,7 @@ static int64_t rsys_2d(Engine& P, Engine& S, const double* Trel, double eps, dou
     const int64_t npairs = (int64_t)np * ns;
     const int CM = P.MM + S.MM;
     if (CM > kMaxM) throw std::runtime_error("the relative arrangement would exceed 31 hyperplanes");
-    const double bytes = (double)npairs * (CM * 72.0 + 8.0 * (CM + 1) * 2 + 14 * 8 + 32);
+    const double bytes = (double)npairs * (CM * 32.0 + 48.0 * (CM + 1) + 14 * 8 + 32);
     if (bytes > 64.0 * (1ull << 30))
         throw std::runtime_error("the relative system's pairs need more than 64 GiB; use estimators with fewer terms");
     GraveyardScope gs(&P.graveyard);
@@ -2453,12 +2466,8 @@ static int64_t rsys_2d(Engine& P, Engine& S, const double* Trel, double eps, dou
     HIPCHK(hipStreamSynchronize(S.st));
     P.c2_mc.reserve(npairs);
     P.c2_b2.reserve(2 * npairs);
-    P.c2_sn.reserve(npairs * (CM + 1));
-    P.c2_cs.reserve(npairs * (CM + 1));
-    P.c2_g1r.reserve(npairs * CM);
-    P.c2_g2r.reserve(npairs * CM);
-    P.c2_g.reserve(npairs * CM);
-    P.c2_fc.reserve(npairs * CM);
+    P.c2_wall.reserve(npairs * (CM + 1));
+    P.c2_cell.reserve(npairs * CM);
     P.rs_mom.reserve(npairs * 14);
     P.rs_keep.reserve(npairs);
     P.rs_idx.reserve(npairs);
@@ -2470,12 +2479,8 @@ static int64_t rsys_2d(Engine& P, Engine& S, const double* Trel, double eps, dou
     C.MM = CM;
     C.mc = P.c2_mc.ptr;
     C.b2 = P.c2_b2.ptr;
-    C.sn = P.c2_sn.ptr;
-    C.cs = P.c2_cs.ptr;
-    C.g1r = P.c2_g1r.ptr;
-    C.g2r = P.c2_g2r.ptr;
-    C.gc = P.c2_g.ptr;
-    C.fc = P.c2_fc.ptr;
+    C.wall = P.c2_wall.ptr;
+    C.cell = P.c2_cell.ptr;
     TermPool PI = P.in.view(), SI = S.in.view();
     if (npairs > 0) {
         const unsigned blocks = (unsigned)((npairs + 127) / 128);
@@ -2547,7 +2552,8 @@ static int64_t rsys_2d(Engine& P, Engine& S, const double* Trel, double eps, dou
             py[i * ny + j] = ys[j];
         }
     if (nkeep > 0) {
-        const int nchunks = ceil_div(nkeep, kCpdfChunk);
+        const Grid2DShape shape(nkeep, npts);
+        const int nchunks = shape.chunks;
         P.c2_px.reserve(npts);
         P.c2_py.reserve(npts);
         P.cpdf_part.reserve((size_t)nchunks * npts);
@@ -2555,9 +2561,8 @@ static int64_t rsys_2d(Engine& P, Engine& S, const double* Trel, double eps, dou
         HIPCHK(hipMemcpyAsync(P.c2_px.ptr, px.data(), npts * sizeof(double), hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(P.c2_py.ptr, py.data(), npts * sizeof(double), hipMemcpyHostToDevice, st));
         HIPCHK(hipMemsetAsync(P.c2_err.ptr, 0, sizeof(int), st));
-        MCE_LAUNCH(k_cpdf2d_grid, dim3(ceil_div(npts, kCpdfPoints), nchunks), dim3(kCpdfPoints), 0, st, C,
-                           nkeep, P.rs_idx.ptr, P.c2_px.ptr, P.c2_py.ptr, npts, P.cpdf_part.ptr, P.c2_err.ptr);
-        MCE_LAUNCH(k_cpdf1d_finish, dim3(ceil_div(npts, 256)), dim3(256), 0, st, P.cpdf_part.ptr, nchunks, npts,
+        launch_grid_2d(st, C, nkeep, shape, P.rs_idx.ptr, P.c2_px.ptr, P.c2_py.ptr, npts, P.cpdf_part.ptr, P.c2_err.ptr);
+        MCE_LAUNCH(k_cpdf1d_finish, dim3(ceil_div(npts, kFinishPoints)), dim3(kFinishPoints * kFinishSlices), 0, st, P.cpdf_part.ptr, nchunks, npts,
                            1.0, P.cpdf_y.ptr);
         HIPCHK(hipGetLastError());
         int singular = 0;

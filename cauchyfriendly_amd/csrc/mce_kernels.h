@@ -3056,7 +3056,15 @@ __global__ void k_sum_fixed(const double* __restrict__ v, int n, double* __restr
     __shared__ double sh[1024];
     const int t = threadIdx.x;
     double s = 0.0;
-    for (int i = t; i < n; i += blockDim.x) s += v[i];
+    int i = t;
+    for (; i + 15 * (int)blockDim.x < n; i += 16 * blockDim.x) {  // sixteen loads in flight
+        double x[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) x[u] = v[i + u * blockDim.x];
+#pragma unroll
+        for (int u = 0; u < 16; u++) s += x[u];
+    }
+    for (; i < n; i += blockDim.x) s += v[i];
     sh[t] = s;
     __syncthreads();
     for (int h = blockDim.x / 2; h > 0; h >>= 1) {
@@ -3065,6 +3073,16 @@ __global__ void k_sum_fixed(const double* __restrict__ v, int n, double* __restr
     }
     if (t == 0) out[0] = sh[0];
 }
+
+// 1 / d to the last bit or two: the hardware's 2^-24 estimate x with error e = 1 - d x, then
+// x (1 + e + e^2), three fused operations where a division takes about ten.  Not finite where
+// d is zero, subnormal or not finite; the callers look for that in their sums.
+__device__ __forceinline__ double fast_rcp(double d) {
+    const double x = __builtin_amdgcn_rcp(d);
+    const double e = __builtin_fma(-d, x, 1.0);
+    return __builtin_fma(x, __builtin_fma(e, e, e), x);
+}
+__device__ __forceinline__ bool is_finite(double x) { return fabs(x) < __builtin_inf(); }
 
 constexpr int kCpdfChunk = 1024;   // terms staged in LDS per block
 constexpr int kCpdfPoints = 256;   // grid points per block (one per thread)
@@ -3084,35 +3102,69 @@ __global__ void __launch_bounds__(kCpdfPoints) k_cpdf1d_grid(const CpdfTerm1D* _
     if (k >= npts) return;
     const double x = xs[k];
     double acc = 0.0;
-    // terms in pairs, n0 / d0 + n1 / d1 = (n0 d1 + n1 d0) / (d0 d1): one division per two
-    // terms where d0 d1 (each d = w^2 + (x - s)^2 > 0) stays in range, two otherwise
-    int j = 0;
-    for (; j + 1 < nt; j += 2) {
-        const CpdfTerm1D c0 = sh[j], c1 = sh[j + 1];
-        const double x0 = x - c0.s, x1 = x - c1.s;
-        const double d0 = c0.w2 + x0 * x0, d1 = c1.w2 + x1 * x1;
-        const double n0 = c0.a * x + c0.bb, n1 = c1.a * x + c1.bb;
-        const double dd = d0 * d1;
-        if (dd > 1e-280 && dd < 1e280) acc += (n0 * d1 + n1 * d0) / dd;
-        else acc += n0 / d0 + n1 / d1;
-    }
-    if (j < nt) {
-        const CpdfTerm1D c = sh[j];
-        double xm = x - c.s;
-        xm *= xm;
-        acc += (c.a * x + c.bb) / (c.w2 + xm);
+    // Terms in pairs, n0 / d0 + n1 / d1 = (n0 d1 + n1 d0) / (d0 d1), each d = w^2 + (x - s)^2: one
+    // reciprocal per two terms.  Where d0 d1 leaves the range of a double the reciprocal is not
+    // a number, and the run of pairs is added again by divisions.
+    constexpr int kRun = 32;
+    for (int j0 = 0; j0 < nt; j0 += kRun) {
+        const int j1 = min(nt, j0 + kRun);
+        double run = 0.0;
+        int j = j0;
+        for (; j + 1 < j1; j += 2) {
+            const CpdfTerm1D c0 = sh[j], c1 = sh[j + 1];
+            const double x0 = x - c0.s, x1 = x - c1.s;
+            const double d0 = __builtin_fma(x0, x0, c0.w2), d1 = __builtin_fma(x1, x1, c1.w2);
+            const double n0 = __builtin_fma(c0.a, x, c0.bb), n1 = __builtin_fma(c1.a, x, c1.bb);
+            run = __builtin_fma(__builtin_fma(n0, d1, n1 * d0), fast_rcp(d0 * d1), run);
+        }
+        if (j < j1) {
+            const CpdfTerm1D c = sh[j];
+            const double xm = x - c.s;
+            run += (c.a * x + c.bb) / (c.w2 + xm * xm);
+        }
+        if (!is_finite(run)) {
+            run = 0.0;
+            for (j = j0; j < j1; j++) {
+                const CpdfTerm1D c = sh[j];
+                const double xm = x - c.s;
+                run += (c.a * x + c.bb) / (c.w2 + xm * xm);
+            }
+        }
+        acc += run;
     }
     part[(int64_t)chunk * npts + k] = acc;
 }
 
-// y_k = (sum over chunks of part) / norm, the chunks added in order.
-__global__ void k_cpdf1d_finish(const double* __restrict__ part, int nchunks, int npts, double norm,
-                                double* __restrict__ y) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= npts) return;
+// y_k = (sum over chunks of part) / norm.  Workgroup of kFinishPoints points x kFinishSlices
+// wavefronts; slice w adds chunks w, w + kFinishSlices, ... in order, then the slices are added
+// in order.  (One thread per point left a 21 x 21 grid's 441 points to two workgroups, which
+// took 606 us over 1600 chunks.)
+constexpr int kFinishPoints = 64;
+constexpr int kFinishSlices = 16;
+__global__ void __launch_bounds__(kFinishPoints* kFinishSlices) k_cpdf1d_finish(const double* __restrict__ part,
+                                                                                int nchunks, int npts, double norm,
+                                                                                double* __restrict__ y) {
+    __shared__ double sh[kFinishSlices][kFinishPoints];
+    const int lane = threadIdx.x % kFinishPoints, w = threadIdx.x / kFinishPoints;
+    const int k = blockIdx.x * kFinishPoints + lane;
     double s = 0.0;
-    for (int c = 0; c < nchunks; c++) s += part[(int64_t)c * npts + k];
-    y[k] = s / norm;
+    if (k < npts) {
+        int c = w;
+        for (; c + 7 * kFinishSlices < nchunks; c += 8 * kFinishSlices) {
+            double x[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) x[u] = part[(int64_t)(c + u * kFinishSlices) * npts + k];
+#pragma unroll
+            for (int u = 0; u < 8; u++) s += x[u];
+        }
+        for (; c < nchunks; c += kFinishSlices) s += part[(int64_t)c * npts + k];
+    }
+    sh[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && k < npts) {
+        for (int u = 1; u < kFinishSlices; u++) s += sh[u][lane];
+        y[k] = s / norm;
+    }
 }
 
 
@@ -3153,28 +3205,33 @@ __device__ __forceinline__ void k_sub_b(MG<1024, 1> mg, TermPool P, int n, VecAr
 // (marg2d_remove_zeros_and_coalign), the cell walls' angles sorted over a full turn,
 // and for each of the m' cells of a half turn its g numerator and the real parts of
 // gamma1, gamma2.  Arrays have a stride of MM cells per term (MM + 1 angles).
-// The point-independent parts of a cell's integral sin(t2 - t1) g / (D1 D2), with
-// Dk = gamma1 cos tk + gamma2 sin tk: Re D1, Re D2 and the numerator.  Only Im gamma1 and
-// Im gamma2 depend on the grid point.
+// A cell's integral is sin(t2 - t1) g / (D1 D2), Dk = gamma1 cos tk + gamma2 sin tk at its two
+// walls.  Re gamma changes from cell to cell by the rows whose sides change there, and those
+// vanish at the wall between: the two cells of a wall have the same D there.  So a wall holds
+// its direction and Re D, and with the cell after it the numerator; a grid point adds Im D =
+// (b1 - x) cos t + (b2 - y) sin t.
+struct Wall2D {
+    double c, s;      // cos, sin of the wall's angle
+    double r, r2;     // Re D and its square
+    double nre, nim;  // g sin(t2 - t1) of the cell that begins here
+};
+// What the reference's other form of the integral needs (gamma1 near zero), per cell.
 struct Cell2D {
-    double d1r, d2r, nre, nim;
+    double g1r, g2r;  // Re gamma
+    cplx g;           // g numerator
 };
 
 struct Cpdf2D {
     int MM;
-    int* mc;           // cells per term
-    double* b2;        // b of the two states
-    double* sn;        // sin of the wall angles
-    double* cs;        // cos of the wall angles
-    double* g1r;       // Re gamma1 per cell
-    double* g2r;       // Re gamma2 per cell
-    cplx* gc;          // g numerator per cell
-    Cell2D* fc;        // point-independent parts per cell
+    int* mc;       // cells per term
+    double* b2;    // b of the two states
+    Wall2D* wall;  // MM + 1 walls per term
+    Cell2D* cell;  // MM cells per term
 };
 
-__device__ inline Cell2D cell2d_parts(double s1, double c1, double s2, double c2, double g1re, double g2re, cplx g) {
-    const double sd = s2 * c1 - s1 * c2;
-    return Cell2D{g1re * c1 + g2re * s1, g1re * c2 + g2re * s2, g.re * sd, g.im * sd};
+__device__ inline Wall2D wall2d(double s1, double c1, double s2, double c2, double g1re, double g2re, cplx g) {
+    const double sd = s2 * c1 - s1 * c2, r = g1re * c1 + g2re * s1;
+    return Wall2D{c1, s1, r, r * r, g.re * sd, g.im * sd};
 }
 
 constexpr double kIntegralGammaEps = 1e-8;  // INTEGRAL_GAMMA_EPS, cauchy_constants.hpp:76
@@ -3338,17 +3395,15 @@ __global__ void k_cpdf2d_terms(TermPool P, int n, int i1, int i2, VecArg bar_nu,
         }
         const double s2 = sin(th[c + 1]), c2 = cos(th[c + 1]);
         total += cpdf2d_cell(s1, c1, s2, c2, g1re, g2re, g1im, g2im, g, check_g1, singular);
-        C.sn[co + i + c] = s1;
-        C.cs[co + i + c] = c1;
-        C.g1r[co + c] = g1re;
-        C.g2r[co + c] = g2re;
-        C.gc[co + c] = g;
-        C.fc[co + c] = cell2d_parts(s1, c1, s2, c2, g1re, g2re, g);
+        C.wall[co + i + c] = wall2d(s1, c1, s2, c2, g1re, g2re, g);
+        C.cell[co + c] = Cell2D{g1re, g2re, g};
         s1 = s2;
         c1 = c2;
+        if (c == u - 1) {
+            const double r = g1re * c2 + g2re * s2;
+            C.wall[co + i + u] = Wall2D{c2, s2, r, r * r, 0.0, 0.0};
+        }
     }
-    C.sn[co + i + u] = s1;
-    C.cs[co + i + u] = c1;
     C.mc[i] = u;
     C.b2[2 * i] = bx;
     C.b2[2 * i + 1] = by;
@@ -3356,50 +3411,129 @@ __global__ void k_cpdf2d_terms(TermPool P, int n, int i1, int i2, VecArg bar_nu,
     if (singular) atomicOr(err, 1);
 }
 
-// Partial sums over one chunk of terms for a block of grid points (the cached cell
+// Partial sums over one chunk of terms for kGridLanes * P grid points (the cached cell
 // integrals, marg2d_cached_eval_term_for_cpdf, cpdf_ndim.hpp:1654-1735).
 // `idx`, when given, lists the terms to add (the kept ones of a relative system).
-__global__ void __launch_bounds__(kCpdfPoints) k_cpdf2d_grid(Cpdf2D C, int n, const int* __restrict__ idx,
-                                                             const double* __restrict__ px,
-                                                             const double* __restrict__ py, int npts,
-                                                             double* __restrict__ part, int* __restrict__ err) {
+//
+// FP64 VALU bound.  A wavefront holds P points per lane and goes through a quarter of the
+// chunk's terms, whose walls it reads as scalars (every lane is at the same term).  The sum over a
+// term's cells is sum_c Re(n_c q_c q_c+1) with q = 1 / D, one q per wall instead of one quotient
+// per cell, and two walls share a reciprocal: about 16 operations a wall and point, where the
+// quotient per cell took about 35.  A sum that is not finite (some |D|^2 left the range of a
+// double) and a term with |b1 - x| < kIntegralGammaEps (the reference's other form) are
+// evaluated cell by cell.  101 x 101 points, 579k terms of 13 cells: 110.5 ms before.
+constexpr int kGridLanes = 64;
+constexpr int kGridWaves = 4;
+template <int P>
+__global__ void __launch_bounds__(kGridLanes* kGridWaves) k_cpdf2d_grid(Cpdf2D C, int n, int chunk_terms,
+                                                                        const int* __restrict__ idx,
+                                                                        const double* __restrict__ px,
+                                                                        const double* __restrict__ py, int npts,
+                                                                        double* __restrict__ part,
+                                                                        int* __restrict__ err) {
+    __shared__ double sh[kGridWaves][P][kGridLanes];
+    const int lane = threadIdx.x % kGridLanes;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kGridLanes));
     const int chunk = blockIdx.y;
-    const int t0 = chunk * kCpdfChunk;
-    const int t1 = min(n, t0 + kCpdfChunk);
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= npts) return;
-    const double x = px[k], y = py[k];
+    const int per = (chunk_terms + kGridWaves - 1) / kGridWaves;
+    const int t0 = min(n, chunk * chunk_terms + w * per);
+    const int t1 = min(min(n, (chunk + 1) * chunk_terms), t0 + per);
+    const int k0 = blockIdx.x * kGridLanes * P + lane;
     const int MM = C.MM;
-    double acc = 0.0;
+    double x[P], y[P], acc[P];
+#pragma unroll
+    for (int j = 0; j < P; j++) {
+        const int k = min(k0 + j * kGridLanes, npts - 1);
+        x[j] = px[k];
+        y[j] = py[k];
+        acc[j] = 0.0;
+    }
     bool singular = false;
     for (int tt = t0; tt < t1; tt++) {
-        const int t = idx ? idx[tt] : tt;
+        const int64_t t = idx ? idx[tt] : tt;
         const int u = C.mc[t];
-        const double g1im = C.b2[2 * t] - x, g2im = C.b2[2 * t + 1] - y;
-        const bool check_g1 = fabs(g1im) < kIntegralGammaEps;
-        const int64_t co = (int64_t)t * MM;
-        const double* sn = C.sn + co + t;
-        const double* cs = C.cs + co + t;
-        double term = 0.0;
-        for (int c = 0; c < u; c++) {
-            const double s1 = sn[c], c1 = cs[c], s2 = sn[c + 1], c2 = cs[c + 1];
-            if (check_g1 && fabs(C.g1r[co + c]) < kIntegralGammaEps) {
-                term += cpdf2d_cell(s1, c1, s2, c2, C.g1r[co + c], C.g2r[co + c], g1im, g2im, C.gc[co + c], true,
-                                    singular);
-                continue;
-            }
-            // Re(n / (D1 D2)) from the cell's point-independent parts: one real division where
-            // |D1 D2|^2 stays in range, the complex quotient otherwise
-            const Cell2D f = C.fc[co + c];
-            const double d1i = g1im * c1 + g2im * s1, d2i = g1im * c2 + g2im * s2;
-            const cplx den = cmake(f.d1r * f.d2r - d1i * d2i, f.d1r * d2i + d1i * f.d2r);
-            const double n2 = den.re * den.re + den.im * den.im;
-            if (n2 > 1e-280 && n2 < 1e280) term += (f.nre * den.re + f.nim * den.im) / n2;
-            else term += cdiv(cmake(f.nre, f.nim), den).re;
+        if (u <= 0) continue;
+        const Wall2D* __restrict__ W = C.wall + t * (MM + 1);
+        const double bx = C.b2[2 * t], by = C.b2[2 * t + 1];
+        double gx[P], gy[P], sum[P], qr[P], qi[P];
+        bool plain = true;
+#pragma unroll
+        for (int j = 0; j < P; j++) {
+            gx[j] = bx - x[j];
+            gy[j] = by - y[j];
+            plain &= !(fabs(gx[j]) < kIntegralGammaEps);
+            sum[j] = 0.0;
+            const double i0 = __builtin_fma(gx[j], W[0].c, gy[j] * W[0].s);
+            const double v = fast_rcp(__builtin_fma(i0, i0, W[0].r2));
+            qr[j] = W[0].r * v;
+            qi[j] = -(i0 * v);
         }
-        acc += term;
+        if (__all(plain)) {
+            int c = 0;
+            for (; c + 1 < u; c += 2) {
+                const Wall2D wa = W[c + 1], wb = W[c + 2];
+                const double n0r = W[c].nre, n0i = W[c].nim;
+#pragma unroll
+                for (int j = 0; j < P; j++) {
+                    const double ia = __builtin_fma(gx[j], wa.c, gy[j] * wa.s);
+                    const double ib = __builtin_fma(gx[j], wb.c, gy[j] * wb.s);
+                    const double da = __builtin_fma(ia, ia, wa.r2), db = __builtin_fma(ib, ib, wb.r2);
+                    const double v = fast_rcp(da * db);
+                    const double va = v * db, vb = v * da;
+                    const double ar = wa.r * va, ai = -(ia * va), br = wb.r * vb, bi = -(ib * vb);
+                    const double ur = __builtin_fma(n0r, qr[j], -(n0i * qi[j]));
+                    const double ui = __builtin_fma(n0r, qi[j], n0i * qr[j]);
+                    const double vr = __builtin_fma(wa.nre, br, -(wa.nim * bi));
+                    const double vi = __builtin_fma(wa.nre, bi, wa.nim * br);
+                    // Re((n0 q + na qb) qa): both cells share the wall between them
+                    const double er = ur + vr, ei = ui + vi;
+                    sum[j] = __builtin_fma(er, ar, __builtin_fma(-ei, ai, sum[j]));
+                    qr[j] = br;
+                    qi[j] = bi;
+                }
+            }
+            if (c < u) {
+                const Wall2D wa = W[c + 1];
+                const double n0r = W[c].nre, n0i = W[c].nim;
+#pragma unroll
+                for (int j = 0; j < P; j++) {
+                    const double ia = __builtin_fma(gx[j], wa.c, gy[j] * wa.s);
+                    const double v = fast_rcp(__builtin_fma(ia, ia, wa.r2));
+                    const double ar = wa.r * v, ai = -(ia * v);
+                    const double ur = __builtin_fma(n0r, qr[j], -(n0i * qi[j]));
+                    const double ui = __builtin_fma(n0r, qi[j], n0i * qr[j]);
+                    sum[j] = __builtin_fma(ur, ar, __builtin_fma(-ui, ai, sum[j]));
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < P; j++) plain &= is_finite(sum[j]);
+        }
+        if (!__all(plain)) {
+            const Cell2D* __restrict__ L = C.cell + t * MM;
+#pragma unroll 1
+            for (int j = 0; j < P; j++) {
+                double z = 0.0;
+                const bool check_g1 = fabs(gx[j]) < kIntegralGammaEps;
+                for (int c = 0; c < u; c++)
+                    z += cpdf2d_cell(W[c].s, W[c].c, W[c + 1].s, W[c + 1].c, L[c].g1r, L[c].g2r, gx[j], gy[j], L[c].g,
+                                     check_g1, singular);
+                sum[j] = z;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < P; j++) acc[j] += sum[j];
     }
-    part[(int64_t)chunk * npts + k] = acc;
+#pragma unroll
+    for (int j = 0; j < P; j++) sh[w][j][lane] = acc[j];
+    __syncthreads();
+    if (w == 0)
+#pragma unroll
+        for (int j = 0; j < P; j++) {
+            const int k = k0 + j * kGridLanes;
+            double z = sh[0][j][lane];
+            for (int v = 1; v < kGridWaves; v++) z += sh[v][j][lane];
+            if (k < npts) part[(int64_t)chunk * npts + k] = z;
+        }
     if (singular) atomicOr(err, 1);
 }
 
@@ -3671,22 +3805,18 @@ __global__ void k_rsys_pairs(TermPool P, int np, const uint32_t* __restrict__ pk
         const double s2 = sin(th[c + 1]), c2 = cos(th[c + 1]);
         s_hi = s2;
         c_hi = c2;
-        C.sn[co + q + c] = s1;
-        C.cs[co + q + c] = c1;
-        C.g1r[co + c] = g1re;
-        C.g2r[co + c] = g2re;
-        C.gc[co + c] = g;
-        C.fc[co + c] = cell2d_parts(s1, c1, s2, c2, g1re, g2re, g);
+        C.wall[co + q + c] = wall2d(s1, c1, s2, c2, g1re, g2re, g);
+        C.cell[co + c] = Cell2D{g1re, g2re, g};
+        if (c == u - 1) {
+            const double r = g1re * c2 + g2re * s2;
+            C.wall[co + q + u] = Wall2D{c2, s2, r, r * r, 0.0, 0.0};
+        }
         // the approximation's bound on the cell's contribution
         const double den1 = g1re * (g1re * c1 + g2re * s1);
         const double den2 = g1re * (g1re * c2 + g2re * s2);
         if (fabs(den1) < 1e-14 || fabs(den2) < 1e-14) keep_term = true;
         const double gr = hypot(g.re, g.im);
         total += fabs((gr * s2) / den2) + fabs((gr * s1) / den1);
-    }
-    if (u > 0) {  // th[u], the last cell's upper edge
-        C.sn[co + q + u] = s_hi;
-        C.cs[co + q + u] = c_hi;
     }
     C.mc[q] = u;
     C.b2[2 * q] = b2[0];
