@@ -662,7 +662,7 @@ struct Engine {
     std::vector<cplx> dfz_tan;   // d fz of the last update, per direction
     int gcur = 0;
     DBuf<uint32_t> barena, b2arena, tmpk;
-    DBuf<cplx> scratch, tmpv;
+    DBuf<cplx> tmpv;
     DBuf<StepConst> dconst;
     DBuf<double> dbpert, gy, mom_part, mom_out, mom_x;
     DBuf<uint8_t> dcombos;
@@ -707,7 +707,6 @@ struct Engine {
     DBuf<int> defer_k0, big_icnt, big_ioff, big_hcnt, big_hoff, hist_mx;
     DBuf<int64_t> big_ccnt, big_coff;
     DBuf<cplx> contrib;
-    DBuf<uint8_t> cneg;
     Profiler prof;
     Graveyard graveyard;
     static constexpr size_t kGraveyardBytes = size_t(4) << 30;  // released early beyond this
@@ -731,7 +730,7 @@ struct Engine {
         sr = maxhp + 1;
         MM = maxhp;
         if (maxhp > 31) throw std::runtime_error("largest hyperplane count exceeds 31");
-        if (maxhp > 20) throw std::runtime_error("largest hyperplane count above 20 is not supported by the LDS cell tables");
+        if (maxhp > kMaxShape) throw std::runtime_error("largest hyperplane count above 20 is not supported by the LDS cell tables");
         A0.assign(A0_, A0_ + d * d);
         p0.assign(p0_, p0_ + d);
         b0.assign(b0_, b0_ + d);
@@ -1353,14 +1352,14 @@ struct Engine {
     // for the update.
     void pick_lookup(int& mode, size_t& lds, int& wmax) const {
         wmax = (std::max(4, (((1 << (MM - 1)) + 31) >> 5)) + 3) & ~3;  // multiple of 4 words
-        const size_t rank_b = (size_t)wmax * 12;  // parent bitset, prefix counts, group bitset
+        const size_t rank_b = (size_t)wmax * 8;  // parent bitset, prefix counts
         const size_t vals_b = (size_t)std::max(max_gp_cells, 1) * sizeof(cplx);
         const size_t keys_b = (size_t)std::max(max_gp_cells, 1) * sizeof(uint32_t);
         const size_t budget = 48 * 1024;
         // the rank structure with values read from global memory is the default: the
         // parent values are L2-resident and the smaller LDS footprint keeps more wavefronts
         // resident than staging the values (measured on MI355X)
-        if (MM <= 24 && rank_b <= budget) {
+        if (MM <= kRankShape) {
             mode = kLookupRank;
             lds = rank_b;
         } else if (keys_b <= budget) {
@@ -1868,7 +1867,6 @@ struct Engine {
         const int nx = gcur ^ 1;
         gk[nx].reserve((size_t)cells_total + 1);
         gv[nx].reserve((size_t)cells_total + 1);
-        scratch.reserve((size_t)cells_total + 1);
         if (ntan) {
             // which members each group adds, written by k_group_eval / k_group_members
             mem_add.reserve(std::max(total, 1));
@@ -1895,13 +1893,13 @@ struct Engine {
             ge_mode = mode;
             ge_lds = lds;
             ge_wmax = wmax;
-            const int big_members = mode >= kLookupRank ? big_group_members : INT_MAX;
+            const int big_members = big_group_members;
             defer_k0.reserve(std::max(ng, 1));
 #define MCE_GEVAL(M_, K_)                                                                                        \
     do {                                                                                                          \
         MCE_RUN((k_group_eval<M_, K_>), dim3(ng), dim3(64), lds, st, OUT, ng, d, wmax, grp_root.ptr,    \
                            grp_moff.ptr, grp_mcnt.ptr, grp_m.ptr, mem_slots.ptr, b2arena.ptr, b2off.ptr,           \
-                           b2n.ptr, goff.ptr, gk[gcur].ptr, gv[gcur].ptr, gk[nx].ptr, gv[nx].ptr, scratch.ptr,     \
+                           b2n.ptr, goff.ptr, gk[gcur].ptr, gv[gcur].ptr, gk[nx].ptr, gv[nx].ptr,                  \
                            gscale, surv.ptr, gxor.ptr, sort_list.ptr, counters.ptr + 18, counters.ptr + 19,          \
                            big_members, defer_k0.ptr, ntan ? mem_add.ptr : nullptr, (const uint2*)rank_arena.ptr);  \
     } while (0)
@@ -1909,15 +1907,12 @@ struct Engine {
             if (mode == kLookupRankVals && MM <= 8) MCE_GEVAL(kLookupRankVals, 8);
             else if (mode == kLookupRankVals && MM <= 11) MCE_GEVAL(kLookupRankVals, 11);
             else if (mode == kLookupRankVals && MM <= 14) MCE_GEVAL(kLookupRankVals, 14);
-            else if (mode == kLookupRankVals && MM <= 16) MCE_GEVAL(kLookupRankVals, 16);
-            else if (mode == kLookupRankVals && MM <= 24) MCE_GEVAL(kLookupRankVals, 24);
-            else if (mode == kLookupRankVals) MCE_GEVAL(kLookupRankVals, 32);
+            else if (mode == kLookupRankVals) MCE_GEVAL(kLookupRankVals, kRankShape);
             else if (mode == kLookupRank && MM <= 8) MCE_GEVAL(kLookupRank, 8);
             else if (mode == kLookupRank && MM <= 14) MCE_GEVAL(kLookupRank, 14);
-            else if (mode == kLookupRank && MM <= 16) MCE_GEVAL(kLookupRank, 16);
-            else if (mode == kLookupRank) MCE_GEVAL(kLookupRank, 32);
-            else if (mode == kLookupSearchLds) MCE_GEVAL(kLookupSearchLds, 32);
-            else MCE_GEVAL(kLookupSearch, 32);
+            else if (mode == kLookupRank) MCE_GEVAL(kLookupRank, kRankShape);
+            else if (mode == kLookupSearchLds) MCE_GEVAL(kLookupSearchLds, kMaxShape);
+            else MCE_GEVAL(kLookupSearch, kMaxShape);
 #undef MCE_GEVAL
         }
         HIPCHK(hipGetLastError());
@@ -1927,7 +1922,7 @@ struct Engine {
             fill_multi({{bytes_acc.ptr, sizeof(unsigned long long), 0}});
             MCE_RUN(k_geval_bytes, dim3(ceil_div(ng, 256)), dim3(256), 0, st, ng, d, grp_m.ptr,
                                grp_mcnt.ptr, b2n.ptr, surv.ptr, defer_k0.ptr,
-                               ge_mode >= kLookupRank ? big_group_members : INT_MAX, bytes_acc.ptr);
+                               big_group_members, bytes_acc.ptr);
             const unsigned long long bytes = read1(bytes_acc.ptr);
             float t = 0;
             HIPCHK(hipEventElapsedTime(&t, prof.k0, prof.k1));
@@ -1950,8 +1945,8 @@ struct Engine {
         }
         if (bs && bs->geval_bytes)
             MCE_RUN(k_geval_bytes, dim3(ceil_div(ng, 256)), dim3(256), 0, st, ng, d, grp_m.ptr, grp_mcnt.ptr, b2n.ptr,
-                    surv.ptr, defer_k0.ptr, ge_mode >= kLookupRank ? big_group_members : INT_MAX, bs->geval_bytes);
-        if (ge_mode >= kLookupRank) co_await big_groups(ng, ge_mode, ge_lds, ge_wmax, gscale, nx);
+                    surv.ptr, defer_k0.ptr, big_group_members, bs->geval_bytes);
+        co_await big_groups(ng, ge_mode, ge_lds, ge_wmax, gscale, nx);
         if (prof.on && !bs) prof.alg_bytes += 24.0 * prof_device_sum(ng, grp_mcnt.ptr, b2n.ptr, surv.ptr);
         int nr_[2];
         co_await rd(counters.ptr + 18, nr_, 2);
@@ -2038,30 +2033,28 @@ struct Engine {
         const int nh = (int)tt[1];
         const int64_t nc = tt[2];
         contrib.reserve((size_t)std::max<int64_t>(nc, 1));
-        cneg.reserve(ni);
         TermPool OUT = out.view();
 #define MCE_GMEM(M_, K_)                                                                                         \
     do {                                                                                                          \
         MCE_RUN((k_group_members<M_, K_>), dim3(ni), dim3(64), lds, st, OUT, ng, d, wmax, big_ioff.ptr, \
                            ni, big_coff.ptr, grp_moff.ptr, grp_mcnt.ptr, grp_m.ptr, mem_slots.ptr, b2arena.ptr,    \
                            b2off.ptr, b2n.ptr, gk[gcur].ptr, gv[gcur].ptr, gscale, surv.ptr, gxor.ptr,             \
-                           defer_k0.ptr, contrib.ptr, cneg.ptr, counters.ptr + 19, ntan ? mem_add.ptr : nullptr,    \
+                           defer_k0.ptr, contrib.ptr, counters.ptr + 19, ntan ? mem_add.ptr : nullptr,    \
                            (const uint2*)rank_arena.ptr);                                                          \
     } while (0)
         if (mode == kLookupRankVals && MM <= 8) MCE_GMEM(kLookupRankVals, 8);
         else if (mode == kLookupRankVals && MM <= 11) MCE_GMEM(kLookupRankVals, 11);
         else if (mode == kLookupRankVals && MM <= 14) MCE_GMEM(kLookupRankVals, 14);
-        else if (mode == kLookupRankVals && MM <= 16) MCE_GMEM(kLookupRankVals, 16);
-        else if (mode == kLookupRankVals && MM <= 24) MCE_GMEM(kLookupRankVals, 24);
-        else if (mode == kLookupRankVals) MCE_GMEM(kLookupRankVals, 32);
+        else if (mode == kLookupRankVals) MCE_GMEM(kLookupRankVals, kRankShape);
         else if (mode == kLookupRank && MM <= 8) MCE_GMEM(kLookupRank, 8);
         else if (mode == kLookupRank && MM <= 14) MCE_GMEM(kLookupRank, 14);
-        else if (mode == kLookupRank && MM <= 16) MCE_GMEM(kLookupRank, 16);
-        else MCE_GMEM(kLookupRank, 32);
+        else if (mode == kLookupRank) MCE_GMEM(kLookupRank, kRankShape);
+        else if (mode == kLookupSearchLds) MCE_GMEM(kLookupSearchLds, kMaxShape);
+        else MCE_GMEM(kLookupSearch, kMaxShape);
 #undef MCE_GMEM
         HIPCHK(hipGetLastError());
-        MCE_RUN(k_group_sum, dim3(nh), dim3(64), 0, st, ng, big_hoff.ptr, nh, big_ioff.ptr, big_coff.ptr,
-                           grp_mcnt.ptr, b2n.ptr, goff.ptr, surv.ptr, defer_k0.ptr, contrib.ptr, cneg.ptr, gv[nx].ptr);
+        MCE_RUN(k_group_sum, dim3(nh), dim3(64), 0, st, ng, big_hoff.ptr, nh, big_coff.ptr, grp_mcnt.ptr, b2n.ptr,
+                goff.ptr, surv.ptr, defer_k0.ptr, contrib.ptr, gv[nx].ptr);
         HIPCHK(hipGetLastError());
     }
 

@@ -236,7 +236,12 @@ __device__ inline int wave_excl_scan(int v, int* total) {
     return x - v;
 }
 
-__device__ inline bool wave_all(bool pred) { return __all(pred); }
+// A value that every lane of the wavefront holds alike, in scalar registers.
+__device__ __forceinline__ int wave_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int64_t wave_uniform(int64_t v) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    return ((int64_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) | lo;
+}
 
 // Orders the LDS accesses of the lanes of one wavefront (for workgroups of one wavefront):
 // a wavefront's LDS operations complete in issue order, so only the compiler has to be
@@ -2099,6 +2104,12 @@ __device__ __forceinline__ void k_group_btab(MG<1024, 1> mg, const TermPool OUT,
 //                     prefix counts), values read from global memory
 //   kLookupRankVals   rank structure and an LDS copy of the parent values
 // Every mode finds the same entry; they differ only in where the index comes from.
+// Largest shape of an estimator, and the largest for which the rank structure is used.  A rank
+// structure has 2^(shape-1) bits and as many prefix words / 32; beyond kRankShape it would leave
+// few wavefronts their LDS for tables of some hundred keys, which a binary search of the staged
+// keys finds in 5 to 9 steps.
+constexpr int kMaxShape = 20;
+constexpr int kRankShape = 16;
 enum LookupMode { kLookupSearch = 0, kLookupSearchLds = 1, kLookupRank = 2, kLookupRankVals = 3 };
 
 // Per-term data of one g-table evaluation, staged once per evaluated term: its
@@ -2198,34 +2209,67 @@ __device__ inline cplx eval_cell(const EvalTerm& T, const double (&qr)[KM], cons
     return cscale(v, T.gscale);
 }
 
-__device__ inline double dev_psum2(const TermPool& T, int64_t s, int m) {
-    const double* p = T.p + s * T.MM;
+// (sum of p over the first m rows)^2 of term s, summed in row order.  A wavefront's lanes load
+// the rows at once; the sum then takes them from the lanes one by one.
+__device__ __forceinline__ double wave_psum2(const TermPool& T, int64_t s, int m) {
+    const int lane = wave_lane();
+    const double x = lane < m ? T.p[s * T.MM + lane] : 0.0;
+    const int lo = __double2loint(x), hi = __double2hiint(x);
     double ps = 0;
-    for (int k = 0; k < m; k++) ps += p[k];
+    for (int k = 0; k < m; k++)
+        ps += __hiloint2double(__builtin_amdgcn_readlane(hi, k), __builtin_amdgcn_readlane(lo, k));
     return ps * ps;
+}
+
+// orientation_mask of two terms' rows by a whole wavefront, lane k on row k.  `ai` holds
+// Ai[k d] on lane k (kept by the caller for its root, which meets every member of its group).
+__device__ __forceinline__ int wave_orientation(const double* Ai, double ai, const double* Aj, int m, int d) {
+    const int k = wave_lane();
+    const bool row = k < m;
+    const double aj = row ? Aj[k * d] : 1.0;
+    bool neg = row && ai * aj < 0;
+    if (__any(row && (fabs(ai) < kReductionEps || fabs(aj) < kReductionEps))) {
+        neg = false;
+        if (row) {
+            int e = k * d;
+            while (e < m * d && ((fabs(Ai[e]) < kReductionEps) || (fabs(Aj[e]) < kReductionEps))) e++;
+            neg = e < m * d && (Ai[e] * Aj[e]) < 0;
+        }
+    }
+    return (int)__ballot(neg);
+}
+
+// Whether any lane's value v (of the lanes in `on`) is large, ps |v| > kApproxEps.  |v| is at
+// least either part, so a part that is large by more than the rounding of hypot and of the
+// products decides it; only if no lane's is, the reference's test is taken.
+__device__ __forceinline__ bool wave_large(bool on, double ps, cplx v) {
+    constexpr double lim = kApproxEps * (1.0 + 1e-10);
+    const bool sure = on && v.re == v.re && v.im == v.im && (ps * fabs(v.re) > lim || ps * fabs(v.im) > lim);
+    if (__any(sure)) return true;
+    return __any(on && (ps * hypot(v.re, v.im)) > kApproxEps);
 }
 
 // Stages term s for evaluation (a workgroup of one wavefront, blockDim == 64).  `lds` is the
 // kernel's dynamic LDS: parent keys (kLookupSearchLds), or the rank structure of
-// `wmax` words of bits and `wmax` prefix counts, then `wmax` words of the group's
-// own key bitset (built by the kernel), then the parent values.
+// `wmax` words of bits and `wmax` prefix counts, then the parent values.
 template <int MODE, int KM>
 __device__ inline EvalTerm stage_term(const TermPool& O, int64_t s, int m, const uint32_t* gk_prev,
                                       const cplx* gv_prev, const uint2* rank, double gscale, uint32_t* lds, int wmax,
-                                      double (&qr)[KM], uint8_t* cm_s, int8_t* cs_s, int* rare) {
+                                      double (&qr)[KM], uint8_t* cm_s, int8_t* cs_s) {
     EvalTerm T;
-    const int64_t go = O.gp_off[s];
-    T.pn = O.gp_n[s];
+    // every lane loads the same record; its scalars go to scalar registers
+    const int64_t go = wave_uniform(O.gp_off[s]);
+    T.pn = wave_uniform(O.gp_n[s]);
     T.pvals = gv_prev + go;
     T.pkeys = gk_prev + go;
     T.rbits = nullptr;
     T.rpre = nullptr;
     T.m = m;
-    T.phc = O.phc[s];
-    T.z = O.z[s];
-    T.lhp = O.lhp[s];
-    T.hf = O.hflag[s];
-    const uint8_t fl = O.flags[s];
+    T.phc = wave_uniform(O.phc[s]);
+    T.z = wave_uniform(O.z[s]);
+    T.lhp = wave_uniform(O.lhp[s]);
+    T.hf = (uint32_t)wave_uniform((int)O.hflag[s]);
+    const int fl = wave_uniform((int)O.flags[s]);
     T.is_new = fl & kIsNew;
     T.has_cmap = fl & kHasCmap;
     T.c = O.c[s];
@@ -2243,7 +2287,7 @@ __device__ inline EvalTerm stage_term(const TermPool& O, int64_t s, int m, const
         const int W = (int)((T.klim + 31u) >> 5);
         uint32_t* bits = lds;
         uint32_t* pre = lds + wmax;
-        const uint2* R = rank + O.rk_off[s];
+        const uint2* R = rank + wave_uniform(O.rk_off[s]);
         for (int w = lane; w < W; w += kWave) {
             const uint2 v = R[w];
             bits[w] = v.x;
@@ -2252,7 +2296,7 @@ __device__ inline EvalTerm stage_term(const TermPool& O, int64_t s, int m, const
         T.rbits = bits;
         T.rpre = pre;
         if (MODE == kLookupRankVals) {
-            cplx* dst = reinterpret_cast<cplx*>(lds + 3 * wmax);
+            cplx* dst = reinterpret_cast<cplx*>(lds + 2 * wmax);
             const cplx* vs = gv_prev + go;
             for (int i = lane; i < T.pn; i += kWave) dst[i] = vs[i];
             if (T.pn == 0 && lane == 0) dst[0] = cmake(0, 0);
@@ -2263,8 +2307,7 @@ __device__ inline EvalTerm stage_term(const TermPool& O, int64_t s, int m, const
     T.fm = (m >= 32 ? 0xffffffffu : ((1u << m) - 1u)) & ~T.hf;
 #pragma unroll
     for (int kk = 0; kk < KM; kk++) qr[kk] = ((T.fm >> kk) & 1u) ? O.q[s * MM + kk] : -0.0;
-    const int pbc = O.pbc[s];
-    if (T.has_cmap && lane < pbc) {
+    if (T.has_cmap && lane < O.pbc[s]) {
         cm_s[lane] = O.cmap[s * MM + lane];
         cs_s[lane] = O.csmap[s * MM + lane];
     }
@@ -2329,12 +2372,60 @@ __device__ __forceinline__ void k_rank_build(MG<64, 1> mg, const TermPool P, int
     for (int w = lane; w < W; w += kWave) rank[off + w] = make_uint2(bits[w], pre[w]);
 }
 
+// One member of a reduction group, added into the group's root table (add_gtables,
+// flattening.hpp:259-315) in the root's orientation sig: root cell bi takes the member's value
+// at bi ^ sig, reversed and conjugated when that key is in the upper half; a key outside the
+// member's table adds nothing.  A negligible member (term approximation) adds nothing at all.
+// add(i, v) receives the values.  The approximation test looks at the member's own cells
+// B ^ own, which are the same keys wherever bi is in the lower half: the values it evaluates
+// are the ones that are added.  (A coaligned child's projected cells are not re-normalised,
+// cell_enumeration.hpp:206-371, so a key of B can have bit m-1 set.)  Returns whether the
+// member is negligible.
+template <int MODE, int KM, class Add>
+__device__ __forceinline__ bool eval_member(const EvalTerm& T, const double (&qr)[KM], const uint8_t* cm_s,
+                                            const int8_t* cs_s, const uint32_t* __restrict__ B, int n, int m,
+                                            uint32_t X, uint32_t sig, double ps, Add add) {
+    const int lane = wave_lane();
+    const uint32_t top = 1u << (m - 1), rev = (m >= 32) ? 0xffffffffu : ((1u << m) - 1u);
+    const uint32_t own = X ^ ((sig & top) ? (sig ^ rev) : sig);  // a cell of B is the member's key B ^ own
+    // the first 64 cells with a large one among them
+    int at = 0;
+    uint32_t b = 0;
+    cplx v = cmake(0, 0);
+    for (; at < n; at += kWave) {
+        const int i = at + lane;
+        b = B[min(i, n - 1)];
+        if (i < n) v = eval_cell<MODE, KM>(T, qr, cm_s, cs_s, b ^ own);
+        if (wave_large(i < n, ps, v)) break;
+    }
+    if (at >= n) return true;
+    for (int i0 = 0; i0 < n; i0 += kWave) {
+        const int i = i0 + lane;
+        const uint32_t bi = i0 == at ? b : B[min(i, n - 1)];
+        uint32_t x = bi ^ X ^ sig;
+        const bool cj = (x & top) != 0;
+        if (cj) x ^= rev;
+        bool on = i < n, known = i0 == at;
+        if (x != (bi ^ own)) {
+            on = on && bsearch_u32(B, x ^ own, n) >= 0;
+            known = false;
+        }
+        cplx c = v;
+        if (__any(on && !known) && on && !known) c = eval_cell<MODE, KM>(T, qr, cm_s, cs_s, x);
+        if (on) add(i, cj ? cconj(c) : c);
+    }
+    return false;
+}
+
 // Flattening of one reduction group, make_gtables (flattening.hpp:351-564):
 // the root's g-table; if the root is negligible (term approximation), the
 // members in order re-orient the group B-table until one is not (root
 // replacement); then every later non-negligible member's g-table is added into
 // the root's in member order (add_gtables, flattening.hpp:259-315).
-// One wavefront per group; lanes own cells.
+// One wavefront per group; lanes own cells.  What bounds it is the chain of loads that each
+// evaluated term waits for (its record, then its parent's rank structure, then the parent
+// values its cells look up), so a term's p, A and q are loaded by all lanes at once, and every
+// cell of a member is evaluated once.
 template <int MODE, int KM>
 __device__ __forceinline__ void k_group_eval(MG<64, 1> mg, const TermPool OUT, int ng, int d, int wmax,
                                                   const int* __restrict__ grp_root,
@@ -2344,7 +2435,7 @@ __device__ __forceinline__ void k_group_eval(MG<64, 1> mg, const TermPool OUT, i
                                                   const int* __restrict__ b2_n, const int64_t* __restrict__ g_off,
                                                   const uint32_t* __restrict__ gk_prev, const cplx* __restrict__ gv_prev,
                                                   uint32_t* __restrict__ gk_out, cplx* __restrict__ gv_out,
-                                                  cplx* __restrict__ scratch, double gscale, int* __restrict__ surv,
+                                                  double gscale, int* __restrict__ surv,
                                                   int* __restrict__ gxor, int* __restrict__ sort_list,
                                                   int* __restrict__ sort_count, int* __restrict__ rare,
                                                   int big_members, int* __restrict__ defer_k0,
@@ -2362,32 +2453,19 @@ __device__ __forceinline__ void k_group_eval(MG<64, 1> mg, const TermPool OUT, i
     const int n = b2_n[g];
     uint32_t* ok = gk_out + g_off[g];
     cplx* ov = gv_out + g_off[g];
-    cplx* sc = scratch + g_off[g];
     const int* mem = mem_slots + grp_moff[g];
     const int nmem = grp_mcnt[g];
     const uint32_t top = 1u << (m - 1);
     const uint32_t rev = (m >= 32) ? 0xffffffffu : ((1u << m) - 1u);
     int r = grp_root[g];
     uint32_t X = 0;
-    if constexpr (MODE >= kLookupRank) {
-        // bitset of the group's B-table keys below 2^(m-1), for add_gtables.  A coaligned
-        // child's projected cells are not re-normalised (cell_enumeration.hpp:206-371), so
-        // a key can have bit m-1 set; add_gtables only ever asks for keys below 2^(m-1)
-        // (flattening.hpp:297-312), so such a key is never found and is left out.
-        uint32_t* bset = lds_dyn + 2 * wmax;
-        const int WB = (int)((top + 31u) >> 5);
-        for (int w = lane; w < WB; w += kWave) bset[w] = 0;
-        wave_lds_sync();
-        for (int i = lane; i < n; i += kWave) {
-            const uint32_t key = B[i];
-            if (key < top) atomicOr(&bset[key >> 5], 1u << (key & 31));
-        }
-        // ordered before its reads by the LDS syncs of stage_term
-    }
-    {
-        EvalTerm T = stage_term<MODE, KM>(OUT, r, m, gk_prev, gv_prev, rank, gscale, lds_dyn, wmax, qr, cm_s, cs_s, rare);
-        const double ps = dev_psum2(OUT, r, m);
-        // negligible iff every cell is small; the test stops at the first large cell
+    // The root's cells are written as the group's table.  While a root is negligible (every cell
+    // is small; the test stops at the first large one), the next member re-orients the group and
+    // replaces it (replacement chain, flattening.hpp:412-489).
+    int k = 0;
+    for (;;) {
+        const EvalTerm T = stage_term<MODE, KM>(OUT, r, m, gk_prev, gv_prev, rank, gscale, lds_dyn, wmax, qr, cm_s, cs_s);
+        const double ps = wave_psum2(OUT, r, m);
         bool negl = true;
         uint32_t bnext = n > 0 ? B[min(lane, n - 1)] : 0u;  // cell key of the next pass, loaded a pass ahead
         for (int i0 = 0; i0 < n; i0 += kWave) {
@@ -2396,132 +2474,40 @@ __device__ __forceinline__ void k_group_eval(MG<64, 1> mg, const TermPool OUT, i
             bnext = B[min(i + kWave, n - 1)];
             cplx v = cmake(0, 0);
             if (i < n) {
-                v = eval_cell<MODE, KM>(T, qr, cm_s, cs_s, bcur);
+                v = eval_cell<MODE, KM>(T, qr, cm_s, cs_s, bcur ^ X);
                 ov[i] = v;
             }
-            if (negl) negl = wave_all(i >= n || !((ps * hypot(v.re, v.im)) > kApproxEps));
+            if (negl) negl = !wave_large(i < n, ps, v);
         }
-        int k = 0;
-        if (negl) {
-            // replacement chain (flattening.hpp:412-489)
-            int lfr = r;
-            r = -1;
-            while (k < nmem) {
-                const int sk = mem[k++];
-                if (!(OUT.flags[sk] & kIsNew) && lane == 0) atomicOr(rare, 1);
-                int sig = orientation_mask(OUT.A + (int64_t)lfr * MM * d, OUT.A + (int64_t)sk * MM * d, m, d);
-                if ((uint32_t)sig & top) sig ^= (int)rev;
-                X ^= (uint32_t)sig;
-                EvalTerm Tk = stage_term<MODE, KM>(OUT, sk, m, gk_prev, gv_prev, rank, gscale, lds_dyn, wmax, qr, cm_s, cs_s, rare);
-                const double psk = dev_psum2(OUT, sk, m);
-                bool sm = true;
-                uint32_t bnext = n > 0 ? B[min(lane, n - 1)] : 0u;
-                for (int i0 = 0; i0 < n; i0 += kWave) {
-                    const int i = i0 + lane;
-                    const uint32_t bcur = bnext;
-                    bnext = B[min(i + kWave, n - 1)];
-                    cplx v = cmake(0, 0);
-                    if (i < n) {
-                        v = eval_cell<MODE, KM>(Tk, qr, cm_s, cs_s, bcur ^ X);
-                        ov[i] = v;
-                    }
-                    if (sm) sm = wave_all(i >= n || !((psk * hypot(v.re, v.im)) > kApproxEps));
-                }
-                if (!sm) {
-                    r = sk;
-                    break;
-                }
-                lfr = sk;
-            }
-            if (r < 0) {
-                if (lane == 0) surv[g] = -1;
-                return;
-            }
+        if (!negl) break;
+        if (k >= nmem) {
+            if (lane == 0) surv[g] = -1;
+            return;
         }
-        // later members are added into the root's table; in a group with more than
-        // big_members members that is left to k_group_members / k_group_sum
-        const double* Ar = OUT.A + (int64_t)r * MM * d;
-        if (MODE >= kLookupRank && nmem > big_members) {
-            if (lane == 0) defer_k0[g] = k;
-            k = nmem;
-        }
-        for (; k < nmem; k++) {
-            const int sk = mem[k];
-            if (!(OUT.flags[sk] & kIsNew) && lane == 0) atomicOr(rare, 2);
-            const int sig = orientation_mask(Ar, OUT.A + (int64_t)sk * MM * d, m, d);
-            const uint32_t sh = ((uint32_t)sig & top) ? ((uint32_t)sig ^ rev) : (uint32_t)sig;
-            EvalTerm Tk = stage_term<MODE, KM>(OUT, sk, m, gk_prev, gv_prev, rank, gscale, lds_dyn, wmax, qr, cm_s, cs_s, rare);
-            const double psk = dev_psum2(OUT, sk, m);
-            if constexpr (MODE >= kLookupRank) {
-                // negligibility over the member's own cells B ^ X ^ sh, stopping at the
-                // first large cell
-                bool sm = true;
-                for (int i0 = 0; i0 < n && sm; i0 += kWave) {
-                    const int i = i0 + lane;
-                    cplx v = cmake(0, 0);
-                    if (i < n) v = eval_cell<MODE, KM>(Tk, qr, cm_s, cs_s, B[i] ^ X ^ sh);
-                    sm = wave_all(i >= n || !((psk * hypot(v.re, v.im)) > kApproxEps));
-                }
-                if (mem_add && lane == 0) mem_add[grp_moff[g] + k] = sm ? 0 : 1;
-                if (sm) continue;
-                // add_gtables: root cell bi takes the member's value at bi ^ sigma
-                // (reversed and conjugated when that key is in the lower half), which
-                // is evaluated directly; a key outside the member's table adds nothing
-                const uint32_t* bset = lds_dyn + 2 * wmax;
-                for (int i = lane; i < n; i += kWave) {
-                    const uint32_t bi = B[i] ^ X;
-                    uint32_t x = bi ^ (uint32_t)sig;
-                    bool cj = false;
-                    if (x & top) {
-                        cj = true;
-                        x ^= rev;
-                    }
-                    const uint32_t y = x ^ sh ^ X;  // the member's key x as a key of B
-                    if (!((bset[y >> 5] >> (y & 31)) & 1u)) continue;
-                    const cplx v = eval_cell<MODE, KM>(Tk, qr, cm_s, cs_s, x);
-                    const cplx cur = ov[i];
-                    ov[i] = cadd(cur, cj ? cconj(v) : v);
-                }
-            } else {
-                bool sm = true;
-                uint32_t bnext = n > 0 ? B[min(lane, n - 1)] : 0u;
-                for (int i0 = 0; i0 < n; i0 += kWave) {
-                    const int i = i0 + lane;
-                    const uint32_t bcur = bnext;
-                    bnext = B[min(i + kWave, n - 1)];
-                    cplx v = cmake(0, 0);
-                    if (i < n) {
-                        v = eval_cell<MODE, KM>(Tk, qr, cm_s, cs_s, bcur ^ X ^ sh);
-                        sc[i] = v;
-                    }
-                    if (sm) sm = wave_all(i >= n || !((psk * hypot(v.re, v.im)) > kApproxEps));
-                }
-                if (mem_add && lane == 0) mem_add[grp_moff[g] + k] = sm ? 0 : 1;
-                if (sm) continue;
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-                __syncthreads();
-                for (int i = lane; i < n; i += kWave) {
-                    const uint32_t bi = B[i] ^ X;
-                    uint32_t x = bi ^ (uint32_t)sig;
-                    bool cj = false;
-                    if (x & top) {
-                        cj = true;
-                        x ^= rev;
-                    }
-                    cplx v;
-                    if (x == (bi ^ sh)) {
-                        v = sc[i];
-                    } else {
-                        const int ii = bsearch_u32(B, x ^ sh ^ X, n);
-                        if (ii < 0) continue;
-                        v = sc[ii];
-                    }
-                    const cplx cur = ov[i];
-                    ov[i] = cadd(cur, cj ? cconj(v) : v);
-                }
-                __syncthreads();
-            }
-        }
+        const int sk = wave_uniform(mem[k++]);
+        if (!(OUT.flags[sk] & kIsNew) && lane == 0) atomicOr(rare, 1);
+        const double* Al = OUT.A + (int64_t)r * MM * d;
+        int sig = wave_orientation(Al, lane < m ? Al[lane * d] : 1.0, OUT.A + (int64_t)sk * MM * d, m, d);
+        if ((uint32_t)sig & top) sig ^= (int)rev;
+        X ^= (uint32_t)sig;
+        r = sk;
+    }
+    // later members are added into the root's table; in a group with more than
+    // big_members members that is left to k_group_members / k_group_sum
+    const double* Ar = OUT.A + (int64_t)r * MM * d;
+    const double ar = lane < m ? Ar[lane * d] : 1.0;
+    if (nmem > big_members) {
+        if (lane == 0) defer_k0[g] = k;
+        k = nmem;
+    }
+    for (; k < nmem; k++) {
+        const int sk = wave_uniform(mem[k]);
+        if (!(OUT.flags[sk] & kIsNew) && lane == 0) atomicOr(rare, 2);
+        const int sig = wave_orientation(Ar, ar, OUT.A + (int64_t)sk * MM * d, m, d);
+        const EvalTerm T = stage_term<MODE, KM>(OUT, sk, m, gk_prev, gv_prev, rank, gscale, lds_dyn, wmax, qr, cm_s, cs_s);
+        const bool negl = eval_member<MODE, KM>(T, qr, cm_s, cs_s, B, n, m, X, (uint32_t)sig, wave_psum2(OUT, sk, m),
+                                                [&](int i, cplx v) { ov[i] = cadd(ov[i], v); });
+        if (mem_add && lane == 0) mem_add[grp_moff[g] + k] = negl ? 0 : 1;
     }
     for (int i = lane; i < n; i += kWave) ok[i] = B[i] ^ X;
     if (lane == 0) {
@@ -2560,9 +2546,9 @@ __device__ inline int owner_of(const int* __restrict__ off, int n, int item) {
 
 // One wavefront per (large group, member k): the member's g-table contribution to
 // every cell of the group's root, in the root's orientation (add_gtables,
-// flattening.hpp:259-315), written to contrib[coff[g] + k * n + i].  A key outside
-// the member's table contributes (-0.0, -0.0), which leaves any sum unchanged; a
-// negligible member is flagged in cneg and contributes nothing.
+// flattening.hpp:259-315), written to contrib[coff[g] + k * n + i].  A cell that receives
+// nothing, and every cell of a negligible member, gets (-0.0, -0.0), which leaves any sum
+// unchanged.
 template <int MODE, int KM>
 __device__ __forceinline__ void k_group_members(MG<64, 1> mg, const TermPool OUT, int ng, int d, int wmax,
                                                      const int* __restrict__ ioff, int nitems,
@@ -2574,9 +2560,8 @@ __device__ __forceinline__ void k_group_members(MG<64, 1> mg, const TermPool OUT
                                                      const cplx* __restrict__ gv_prev, double gscale,
                                                      const int* __restrict__ surv, const int* __restrict__ gxor,
                                                      const int* __restrict__ defer_k0, cplx* __restrict__ contrib,
-                                                     uint8_t* __restrict__ cneg, int* __restrict__ rare,
+                                                     int* __restrict__ rare,
                                                      uint8_t* __restrict__ mem_add, const uint2* __restrict__ rank) {
-    static_assert(MODE >= kLookupRank, "parallel member sums use the rank lookup");
     extern __shared__ __align__(16) uint32_t lds_dyn[];
     double qr[KM];
     __shared__ uint8_t cm_s[kMaxM];
@@ -2592,62 +2577,27 @@ __device__ __forceinline__ void k_group_members(MG<64, 1> mg, const TermPool OUT
     const int MM = OUT.MM;
     const uint32_t* B = B2 + b2_off[g];
     const int n = b2_n[g];
-    const uint32_t X = (uint32_t)gxor[g];
-    const uint32_t top = 1u << (m - 1);
-    const uint32_t rev = (m >= 32) ? 0xffffffffu : ((1u << m) - 1u);
-    uint32_t* bset = lds_dyn + 2 * wmax;
-    {
-        const int WB = (int)((top + 31u) >> 5);
-        for (int w = lane; w < WB; w += kWave) bset[w] = 0;
-        __syncthreads();
-        for (int i = lane; i < n; i += kWave) {
-            const uint32_t key = B[i];
-            if (key < top) atomicOr(&bset[key >> 5], 1u << (key & 31));
-        }
-    }
     const int sk = mem_slots[grp_moff[g] + k];
     if (!(OUT.flags[sk] & kIsNew) && lane == 0) atomicOr(rare, 2);
-    const int sig = orientation_mask(OUT.A + (int64_t)r * MM * d, OUT.A + (int64_t)sk * MM * d, m, d);
-    const uint32_t sh = ((uint32_t)sig & top) ? ((uint32_t)sig ^ rev) : (uint32_t)sig;
-    EvalTerm Tk = stage_term<MODE, KM>(OUT, sk, m, gk_prev, gv_prev, rank, gscale, lds_dyn, wmax, qr, cm_s, cs_s, rare);
-    const double psk = dev_psum2(OUT, sk, m);
-    bool sm = true;
-    for (int i0 = 0; i0 < n && sm; i0 += kWave) {
-        const int i = i0 + lane;
-        cplx v = cmake(0, 0);
-        if (i < n) v = eval_cell<MODE, KM>(Tk, qr, cm_s, cs_s, B[i] ^ X ^ sh);
-        sm = wave_all(i >= n || !((psk * hypot(v.re, v.im)) > kApproxEps));
-    }
-    if (lane == 0) cneg[item] = sm ? 1 : 0;
-    if (mem_add && lane == 0) mem_add[grp_moff[g] + k] = sm ? 0 : 1;
-    if (sm) return;
+    const double* Ar = OUT.A + (int64_t)r * MM * d;
+    const int sig = wave_orientation(Ar, lane < m ? Ar[lane * d] : 1.0, OUT.A + (int64_t)sk * MM * d, m, d);
+    const EvalTerm T = stage_term<MODE, KM>(OUT, sk, m, gk_prev, gv_prev, rank, gscale, lds_dyn, wmax, qr, cm_s, cs_s);
     cplx* out = contrib + coff[g] + (int64_t)k * n;
-    for (int i = lane; i < n; i += kWave) {
-        const uint32_t bi = B[i] ^ X;
-        uint32_t x = bi ^ (uint32_t)sig;
-        bool cj = false;
-        if (x & top) {
-            cj = true;
-            x ^= rev;
-        }
-        const uint32_t y = x ^ sh ^ X;
-        cplx c = cmake(-0.0, -0.0);
-        if ((bset[y >> 5] >> (y & 31)) & 1u) {
-            const cplx v = eval_cell<MODE, KM>(Tk, qr, cm_s, cs_s, x);
-            c = cj ? cconj(v) : v;
-        }
-        out[i] = c;
-    }
+    for (int i = lane; i < n; i += kWave) out[i] = cmake(-0.0, -0.0);
+    const bool negl = eval_member<MODE, KM>(T, qr, cm_s, cs_s, B, n, m, (uint32_t)gxor[g], (uint32_t)sig,
+                                            wave_psum2(OUT, sk, m), [&](int i, cplx v) { out[i] = v; });
+    if (mem_add && lane == 0) mem_add[grp_moff[g] + k] = negl ? 0 : 1;
 }
 
 // Adds the member contributions of each large group into its root's table, one
-// lane per cell, members in order (the sum order of add_gtables).
+// lane per cell, members in order (the sum order of add_gtables): a serial chain of adds, fed
+// by kSumBatch loads in flight.
 __device__ __forceinline__ void k_group_sum(MG<64, 1> mg, int ng, const int* __restrict__ hoff, int nchunks,
-                                                 const int* __restrict__ ioff, const int64_t* __restrict__ coff,
+                                                 const int64_t* __restrict__ coff,
                                                  const int* __restrict__ grp_mcnt, const int* __restrict__ b2_n,
                                                  const int64_t* __restrict__ g_off, const int* __restrict__ surv,
                                                  const int* __restrict__ defer_k0, const cplx* __restrict__ contrib,
-                                                 const uint8_t* __restrict__ cneg, cplx* __restrict__ gv_out) {
+                                                 cplx* __restrict__ gv_out) {
     const int item = mg.bx;
     if (item >= nchunks) return;
     const int g = owner_of(hoff, ng, item);
@@ -2657,13 +2607,17 @@ __device__ __forceinline__ void k_group_sum(MG<64, 1> mg, int ng, const int* __r
     if (i >= n) return;
     const int nm = grp_mcnt[g];
     const cplx* cb = contrib + coff[g] + i;
-    const uint8_t* ng_ = cneg + ioff[g];
     cplx acc = gv_out[g_off[g] + i];
-    for (int k = defer_k0[g]; k < nm; k++) {
-        if (ng_[k]) continue;
-        const cplx c = cb[(int64_t)k * n];
-        acc = cadd(acc, c);
+    constexpr int kSumBatch = 16;
+    int k = defer_k0[g];
+    for (; k + kSumBatch <= nm; k += kSumBatch) {
+        cplx c[kSumBatch];
+#pragma unroll
+        for (int u = 0; u < kSumBatch; u++) c[u] = cb[(int64_t)(k + u) * n];
+#pragma unroll
+        for (int u = 0; u < kSumBatch; u++) acc = cadd(acc, c[u]);
     }
+    for (; k < nm; k++) acc = cadd(acc, cb[(int64_t)k * n]);
     gv_out[g_off[g] + i] = acc;
 }
 
