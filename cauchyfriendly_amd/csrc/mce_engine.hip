@@ -1651,9 +1651,15 @@ struct Engine {
         prof.mark(kPhEnum, st);
 
         // ---- measurement update
-        out.reserve(nslots);
+        // the last update keeps no terms: of its output pool only flags and shapes exist
+        if (skip) {
+            out.flags.reserve(nslots);
+            out.m.reserve(nslots);
+        } else {
+            out.reserve(nslots);
+            keys.reserve(nslots);
+        }
         gy.reserve((size_t)nslots * (2 + 2 * d));
-        keys.reserve(nslots);
         chain_key.reserve(nslots);
         chain_skey.reserve(nslots);
         chain_perm.reserve(nslots);
@@ -1661,15 +1667,19 @@ struct Engine {
         chain_off.reserve(16);
         mom_part.reserve((size_t)T * (1 + d + d * d) * 2 + 1);
         TermPool OUT = out.view();
-        // child rows in registers when the largest shape fits a compile-time bound
         const int mu_km = MM <= 8 ? 8 : MM <= 14 ? 14 : 0;
-        if (mu_km == 8) {
-            MCE_DISPATCH_D(d, MCE_RUN((k_mu_r<DD, 8>), dim3(ceil_div(nslots, 256)), dim3(256), 0, st, IN,
+        if (skip) {
+            MCE_DISPATCH_D(d, MCE_RUN(k_mu_last<DD>, dim3(ceil_div(nslots, kMuThreads)), dim3(kMuThreads), 0, st, IN,
+                                      np, slot_base.ptr, out.flags.ptr, out.m.ptr, nslots, dconst.ptr, gk[gcur].ptr,
+                                      gv[gcur].ptr, gy.ptr, chain_key.ptr));
+        } else if (mu_km == 8) {
+            // child rows in registers when the largest shape fits a compile-time bound
+            MCE_DISPATCH_D(d, MCE_RUN((k_mu_r<DD, 8>), dim3(ceil_div(nslots, kMuThreads)), dim3(kMuThreads), 0, st, IN,
                                                  np, slot_base.ptr, OUT, nslots, dconst.ptr, gk[gcur].ptr,
                                                  gv[gcur].ptr, gy.ptr, keys.ptr, chain_key.ptr, counters.ptr + 17));
         } else if (mu_km == 14 && d <= 5) {
             MCE_DISPATCH_D(d, if constexpr (DD <= 5) MCE_RUN(
-                                  (k_mu_r<DD, 14>), dim3(ceil_div(nslots, 256)), dim3(256), 0, st, IN, np,
+                                  (k_mu_r<DD, 14>), dim3(ceil_div(nslots, kMuThreads)), dim3(kMuThreads), 0, st, IN, np,
                                   slot_base.ptr, OUT, nslots, dconst.ptr, gk[gcur].ptr, gv[gcur].ptr, gy.ptr, keys.ptr,
                                   chain_key.ptr, counters.ptr + 17));
         } else {
@@ -1679,7 +1689,7 @@ struct Engine {
         }
         HIPCHK(hipGetLastError());
         if (ntan) {
-            tout.reserve(nslots);
+            if (!skip) tout.reserve(nslots);
             dg_slot.reserve((size_t)nslots * ntan);
             dfz_dev.reserve(ntan);
             MCE_DISPATCH_D(d, MCE_LAUNCH(k_mu_tan<DD>, dim3(ceil_div(nslots, 128)), dim3(128), 0, st, IN, tin.view(),

@@ -945,7 +945,7 @@ __device__ __forceinline__ void k_mu(MG<1024, 1> mg, TermPool IN, int np, const 
     OUT.lhp[s] = (int)lhp;
     OUT.bt_off[s] = IN.bt_off[P];
     OUT.bt_n[s] = IN.bt_n[P];
-    OUT.bt_sgn[s] = sc->skip ? 0 : (int)sg;
+    OUT.bt_sgn[s] = (int)sg;
     OUT.tid[s] = IN.tid[P];
     // moments: g and y_ei of this term (cache_moments, cauchy_estimator.hpp:307-338)
     {
@@ -962,7 +962,7 @@ __device__ __forceinline__ void k_mu(MG<1024, 1> mg, TermPool IN, int np, const 
     }
     int mnew = m;
     uint8_t fl = kValid | ((t != m) ? kIsNew : 0);
-    if (!sc->skip && !sc->first) {
+    if (!sc->first) {
         uint8_t* cm = OUT.cmap + (int64_t)s * MM;
         int8_t* cs = OUT.csmap + (int64_t)s * MM;
         if (t == m) {
@@ -987,31 +987,195 @@ __device__ __forceinline__ void k_mu(MG<1024, 1> mg, TermPool IN, int np, const 
     keys_out[s] = (uint32_t)(((mnew * sc->T) + IN.tid[P]) * 2 + ((t != m) ? 1 : 0));
 }
 
-// Child row r of slot (P, t) as k_mu builds it: parent row r below t and row r + 1
-// from t on, parent row m standing for the measurement-noise row (-mu_t, gamma).
-// Returns the row's p value; sets *horth when the parent row is H-orthogonal.
+// Rows of the parents of one block of output slots, staged in LDS by k_mu_r and k_mu_last.
+// Slot s of parent P is s - slot_base[P] in 0..m: 0 the parent itself, t + 1 its child t.
+// A child's row r is parent row src (r below t, r + 1 from t on; src == m is the
+// measurement-noise row) as mu_src - mu_t with mu_l = A_l / (H . A_l), so everything but a
+// subtraction depends on the parent's row alone: mu_l, rho_l = p_l |H . A_l| and whether the
+// row is H-orthogonal are formed once per parent and block here, where m + 1 threads each
+// formed all of them (a product with H, a division and D products per row and slot) out of
+// global memory.  Entry q holds row q - slot_base[P] of the parent that slot base0 + q belongs
+// to (the last slot of each parent stands empty): a block's slots and the other slots of its
+// first and last parent, at most 31 each.
+constexpr int kMuThreads = 256;
+constexpr int kMuRowCap = kMuThreads + 64;
 template <int D>
-__device__ inline double dev_child_row(const double* A, const double* p, const double* H, const double* mut,
-                                       double gamma, int m, int t, int r, double* row, bool* horth) {
+struct MuRows {
+    double mu[D][kMuRowCap];
+    double rho[kMuRowCap];
+    uint8_t cls[kMuRowCap];  // 0: H-orthogonal (mu holds A itself), 1: H . A > 0, 2: not
+    int base0, last;         // first slot of the first parent, last parent
+};
+
+// Largest i in [0, n) with base[i] <= x (base ascending, base[0] <= x), by a whole wavefront:
+// 64 probes a round, three rounds up to 262,144 entries, where a binary search has 18
+// dependent loads.
+__device__ __forceinline__ int wave_floor(const int* __restrict__ base, int n, int x) {
+    const int lane = threadIdx.x & 63;
+    int lo = 0, len = n;  // the answer lies in [lo, lo + len)
+    while (len > 1) {
+        const int step = (len + 63) >> 6;
+        const int i = lane * step;
+        const int cnt = __popcll(__ballot(i < len && base[lo + i] <= x));  // lane 0 always counts
+        lo += (cnt - 1) * step;
+        len = min(step, len - (cnt - 1) * step);
+    }
+    return lo;
+}
+
+// Stages the rows behind the block's slots [mg.bx * 256, + 256) and returns the parent of this
+// thread's slot (of the last slot for threads past the end).  All threads of the block.
+template <int D>
+__device__ __forceinline__ int mu_stage(MuRows<D>& R, const TermPool& IN, int np, const int* __restrict__ slot_base,
+                                        int s0, int nslots, const double* H) {
+    const int tid = threadIdx.x;
+    const int P0 = wave_floor(slot_base, np, s0);
+    auto parent = [&](int lo, int hi, int x) {
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (slot_base[mid] <= x) lo = mid;
+            else hi = mid - 1;
+        }
+        return lo;
+    };
+    const int sl = min(s0 + kMuThreads, nslots) - 1;
+    const int P = parent(P0, min(np - 1, P0 + kMuThreads - 1), min(s0 + tid, sl));
+    if (s0 + tid == sl) R.last = P;
+    if (tid == 0) R.base0 = slot_base[P0];
+    __syncthreads();
+    const int base0 = R.base0, Pl = R.last;
+    const int end = slot_base[Pl + 1];
+    const int MM = IN.MM;
+    for (int q = base0 + tid; q < end; q += kMuThreads) {
+        const int Q = parent(P0, Pl, q);
+        const int l = q - slot_base[Q];
+        if (l >= IN.m[Q] || q - base0 >= kMuRowCap) continue;
+        const double* A = IN.A + ((int64_t)Q * MM + l) * D;
+        double row[D];
+#pragma unroll
+        for (int k = 0; k < D; k++) row[k] = A[k];
+        const double pl = IN.p[(int64_t)Q * MM + l];
+        const double h = dev_dot<D>(H, row);
+        const int i = q - base0;
+        if (fabs(h) < kMuEps) {
+            R.cls[i] = 0;
+            R.rho[i] = pl;
+        } else {
+            const double r = 1.0 / h;
+            R.cls[i] = h > 0 ? 1 : 2;
+            R.rho[i] = pl * fabs(h);
+#pragma unroll
+            for (int k = 0; k < D; k++) row[k] *= r;
+        }
+#pragma unroll
+        for (int k = 0; k < D; k++) R.mu[k][i] = row[k];
+    }
+    __syncthreads();
+    return P;
+}
+
+// Masks of the parent's rows: integ has the rows that are not H-orthogonal, the result those
+// of them with H . A not positive.
+template <int D>
+__device__ __forceinline__ uint32_t mu_masks(const MuRows<D>& R, int i0, int m, uint32_t* integ) {
+    uint32_t in = 0, neg = 0;
+    for (int l = 0; l < m; l++) {
+        const int c = R.cls[i0 + l];
+        in |= (uint32_t)(c != 0) << l;
+        neg |= (uint32_t)(c == 2) << l;
+    }
+    *integ = in;
+    return neg;
+}
+
+// Row r of child t from the staged rows; returns its p.
+template <int D>
+__device__ __forceinline__ double mu_row(const MuRows<D>& R, int i0, const double* mut, double gamma, int m, int t,
+                                         int r, double* row, bool* horth) {
     const int src = (t < m && r >= t) ? r + 1 : r;
-    *horth = false;
     if (src == m) {
 #pragma unroll
-        for (int kk = 0; kk < D; kk++) row[kk] = 0.0 - mut[kk];
+        for (int k = 0; k < D; k++) row[k] = 0.0 - mut[k];
+        *horth = false;
         return gamma;
     }
-    const double* Ar = A + src * D;
-    const double h = dev_dot<D>(H, Ar);
-    if (fabs(h) < kMuEps) {
+    const int i = i0 + src;
+    *horth = R.cls[i] == 0;
 #pragma unroll
-        for (int kk = 0; kk < D; kk++) row[kk] = Ar[kk];
-        *horth = true;
-        return p[src];
+    for (int k = 0; k < D; k++) {
+        const double v = R.mu[k][i];
+        row[k] = *horth ? v : v - mut[k];
     }
-    const double rr = 1.0 / h;
+    return R.rho[i];
+}
+
+// row /= n1, to the same bits: the steps a double division takes (two Newton steps on the
+// estimate of 1 / n1, the product, one correction by its exact remainder; Markstein, IBM
+// J. Res. Dev. 34, 1990), with the estimate's part done once for the row's D quotients.
+// Outside the range where no step can overflow or lose a subnormal's bits the row is divided
+// as it stands.
+template <int D>
+__device__ __forceinline__ void div_row(double* row, double n1) {
+    bool plain = n1 > 1e-120 && n1 < 1e120;
 #pragma unroll
-    for (int kk = 0; kk < D; kk++) row[kk] = (Ar[kk] * rr) - mut[kk];
-    return p[src] * fabs(h);
+    for (int k = 0; k < D; k++) plain &= row[k] == 0.0 || fabs(row[k]) > 1e-150;
+    if (plain) {
+        double y = __builtin_amdgcn_rcp(n1);
+        y = __builtin_fma(__builtin_fma(-n1, y, 1.0), y, y);
+        y = __builtin_fma(__builtin_fma(-n1, y, 1.0), y, y);
+#pragma unroll
+        for (int k = 0; k < D; k++) {
+            const double q = row[k] * y;
+            const double v = __builtin_fma(__builtin_fma(-n1, q, row[k]), y, q);
+            row[k] = row[k] == 0.0 ? row[k] : v;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < D; k++) row[k] /= n1;
+    }
+}
+
+// g and -Re y, Im y of one slot (eval_g_yei, cauchy_term.hpp:312-401) from its sums over the
+// child rows: written where the moment sums read them.
+template <int D>
+__device__ __forceinline__ void mu_moment(const TermPool& IN, int P, bool first, int m, int t, uint32_t neg,
+                                          uint32_t lhp, double ygi, double rho_t, double zeta, const double* ty,
+                                          const double* cb, const uint32_t* __restrict__ gk_prev,
+                                          const cplx* __restrict__ gv_prev, double* __restrict__ g_out) {
+    cplx gpl, gmn;
+    if (first) {
+        gpl = cmake(1, 0);
+        gmn = cmake(1, 0);
+    } else {
+        const int phc = IN.phc[P];
+        const int top = 1 << (phc - 1), rev = (phc >= 32) ? -1 : ((1 << phc) - 1);
+        int lp = 0, lmv = 0, kq = 0;
+        for (int l = 0; l < m; l++) {
+            if (kq < phc) {
+                if (kq == t) {
+                    lmv |= (1 << kq);
+                    kq++;
+                    if (kq == phc) continue;
+                }
+                if ((neg >> l) & 1u) {
+                    lp |= (1 << kq);
+                    lmv |= (1 << kq);
+                }
+                kq++;
+            }
+        }
+        const int64_t go = IN.gp_off[P];
+        gpl = lookup_num(lp ^ (int)lhp, top, rev, gk_prev + go, gv_prev + go, IN.gp_n[P]);
+        gmn = lookup_num(lmv ^ (int)lhp, top, rev, gk_prev + go, gv_prev + go, IN.gp_n[P]);
+    }
+    const cplx g = cscale(csub(cdiv(gpl, cmake(ygi + rho_t, zeta)), cdiv(gmn, cmake(ygi - rho_t, zeta))), kInvTwoPi);
+    g_out[0] = g.re;
+    g_out[1] = g.im;
+#pragma unroll
+    for (int k = 0; k < D; k++) {
+        g_out[2 + 2 * k] = -ty[k];
+        g_out[3 + 2 * k] = cb[k];
+    }
 }
 
 // Measurement update streamed row by row (KM >= m, compile-time bound).  The same
@@ -1019,21 +1183,18 @@ __device__ inline double dev_child_row(const double* A, const double* p, const d
 // sums, is L1-normalised and written once; only the normalised first coordinates
 // are kept, for the coalignment filter.  When the filter finds a possible merge (a
 // rare case) the rows are rebuilt in memory and coaligned there, as k_mu does.
+// Bound by its double-precision arithmetic: the row's share that does not depend on the
+// child is staged (MuRows) and the normalisation's D divisions share a reciprocal.
 template <int D, int KM>
 __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const int* __restrict__ slot_base, TermPool OUT,
                                              int nslots, const StepConst* __restrict__ sc,
                                              const uint32_t* __restrict__ gk_prev, const cplx* __restrict__ gv_prev,
                                              double* __restrict__ gy, uint32_t* __restrict__ keys_out,
                                              uint32_t* __restrict__ chain_key, int* __restrict__ err) {
-    const int s = mg.bx * blockDim.x + threadIdx.x;
+    __shared__ MuRows<D> R;
+    const int s = mg.bx * kMuThreads + threadIdx.x;
+    const int P = mu_stage<D>(R, IN, np, slot_base, mg.bx * kMuThreads, nslots, sc->H);
     if (s >= nslots) return;
-    int lo = 0, hi = np - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (slot_base[mid] <= s) lo = mid;
-        else hi = mid - 1;
-    }
-    const int P = lo;
     const int MM = IN.MM;
     const int m = IN.m[P];
     if (m > KM) {
@@ -1042,18 +1203,11 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
     }
     const int ts = s - slot_base[P];
     const int t = (ts == 0) ? m : ts - 1;
-    const double* A = IN.A + (int64_t)P * MM * D;
-    const double* p = IN.p + (int64_t)P * MM;
+    const int i0 = slot_base[P] - R.base0;
     const double* b = IN.b + (int64_t)P * D;
     const double* H = sc->H;
-    uint32_t integ = 0, negs = 0;
-    for (int l = 0; l < m; l++) {
-        const double h = dev_dot<D>(H, A + l * D);
-        if (!(fabs(h) < kMuEps)) {
-            integ |= (1u << l);
-            if (!(h > 0)) negs |= (1u << l);
-        }
-    }
+    uint32_t integ;
+    const uint32_t negs = mu_masks<D>(R, i0, m, &integ);
     double* g_out = gy + (int64_t)s * (2 + 2 * D);
     if (t < m && !((integ >> t) & 1u)) {
         OUT.flags[s] = 0;
@@ -1065,18 +1219,9 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
     chain_key[s] = (uint32_t)IN.tid[P];
     const double zeta = sc->msmt - dev_dot<D>(H, b);
     double mut[D];
-    double rho_t;
-    if (t == m) {
 #pragma unroll
-        for (int kk = 0; kk < D; kk++) mut[kk] = 0.0;
-        rho_t = sc->gamma;
-    } else {
-        const double h = dev_dot<D>(H, A + t * D);
-        const double r = 1.0 / h;
-#pragma unroll
-        for (int kk = 0; kk < D; kk++) mut[kk] = A[t * D + kk] * r;
-        rho_t = p[t] * fabs(h);
-    }
+    for (int kk = 0; kk < D; kk++) mut[kk] = t == m ? 0.0 : R.mu[kk][i0 + t];
+    const double rho_t = t == m ? sc->gamma : R.rho[i0 + t];
     double cb[D];
 #pragma unroll
     for (int kk = 0; kk < D; kk++) cb[kk] = b[kk] + zeta * mut[kk];
@@ -1098,7 +1243,7 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
     OUT.lhp[s] = (int)lhp;
     OUT.bt_off[s] = IN.bt_off[P];
     OUT.bt_n[s] = IN.bt_n[P];
-    OUT.bt_sgn[s] = sc->skip ? 0 : (int)sg;
+    OUT.bt_sgn[s] = (int)sg;
     OUT.tid[s] = IN.tid[P];
     double* ob = OUT.b + (int64_t)s * D;
 #pragma unroll
@@ -1106,7 +1251,7 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
     double* oA = OUT.A + (int64_t)s * MM * D;
     double* op = OUT.p + (int64_t)s * MM;
     double* oq = OUT.q + (int64_t)s * MM;
-    const bool normalise = !sc->skip && !sc->first;
+    const bool normalise = !sc->first;
     // rows: moment contributions (eval_g_yei, cauchy_term.hpp:312-401), then
     // q <- p and the L1 normalisation (normalize_hps, cauchy_term.hpp:458-474)
     double ty[D];
@@ -1122,7 +1267,7 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
         if (r < m) {
             double row[D];
             bool ho;
-            double pr = dev_child_row<D>(A, p, H, mut, sc->gamma, m, t, r, row, &ho);
+            double pr = mu_row<D>(R, i0, mut, sc->gamma, m, t, r, row, &ho);
             if (ho) hf |= (1u << r);
             double dr = 0.0;
 #pragma unroll
@@ -1140,8 +1285,7 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
                 oq[r] = pr;
                 pr *= n1;
                 nan_p |= pr != pr;
-#pragma unroll
-                for (int kk = 0; kk < D; kk++) row[kk] /= n1;
+                div_row<D>(row, n1);
                 x0[r] = fabs(row[0]);
             }
 #pragma unroll
@@ -1149,42 +1293,7 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
             op[r] = pr;
         }
     }
-    {
-        cplx gpl, gmn;
-        if (sc->first) {
-            gpl = cmake(1, 0);
-            gmn = cmake(1, 0);
-        } else {
-            const int top = 1 << (phc - 1), rev = (phc >= 32) ? -1 : ((1 << phc) - 1);
-            int lp = 0, lmv = 0, kq = 0;
-            for (int l = 0; l < m; l++) {
-                if (kq < phc) {
-                    if (kq == t) {
-                        lmv |= (1 << kq);
-                        kq++;
-                        if (kq == phc) continue;
-                    }
-                    if ((neg >> l) & 1u) {
-                        lp |= (1 << kq);
-                        lmv |= (1 << kq);
-                    }
-                    kq++;
-                }
-            }
-            const int64_t go = IN.gp_off[P];
-            gpl = lookup_num(lp ^ (int)lhp, top, rev, gk_prev + go, gv_prev + go, IN.gp_n[P]);
-            gmn = lookup_num(lmv ^ (int)lhp, top, rev, gk_prev + go, gv_prev + go, IN.gp_n[P]);
-        }
-        const cplx g = cscale(csub(cdiv(gpl, cmake(ygi + rho_t, zeta)), cdiv(gmn, cmake(ygi - rho_t, zeta))),
-                              kInvTwoPi);
-        g_out[0] = g.re;
-        g_out[1] = g.im;
-#pragma unroll
-        for (int kk = 0; kk < D; kk++) {
-            g_out[2 + 2 * kk] = -ty[kk];
-            g_out[3 + 2 * kk] = cb[kk];
-        }
-    }
+    mu_moment<D>(IN, P, sc->first != 0, m, t, neg, lhp, ygi, rho_t, zeta, ty, cb, gk_prev, gv_prev, g_out);
     int mnew = m;
     uint8_t fl = kValid | ((t != m) ? kIsNew : 0);
     if (normalise && t != m) {
@@ -1206,7 +1315,7 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
             for (int r = 0; r < m; r++) {
                 double row[D];
                 bool ho;
-                op[r] = dev_child_row<D>(A, p, H, mut, sc->gamma, m, t, r, row, &ho);
+                op[r] = mu_row<D>(R, i0, mut, sc->gamma, m, t, r, row, &ho);
 #pragma unroll
                 for (int kk = 0; kk < D; kk++) oA[r * D + kk] = row[kk];
             }
@@ -1225,6 +1334,67 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
     OUT.flags[s] = fl;
     OUT.m[s] = mnew;
     keys_out[s] = (uint32_t)(((mnew * sc->T) + IN.tid[P]) * 2 + ((t != m) ? 1 : 0));
+}
+
+// A window's last update: its terms are summed into the moments and not kept, so only the
+// moment inputs, the shape and the chain key of each slot are formed; the rows are never
+// written, and the output pool holds nothing but flags and shapes.  The same operations in
+// the same order as k_mu and k_mu_r for any shape.
+template <int D>
+__device__ __forceinline__ void k_mu_last(MG<256, 4> mg, TermPool IN, int np, const int* __restrict__ slot_base,
+                                          uint8_t* __restrict__ flags, int* __restrict__ shape, int nslots,
+                                          const StepConst* __restrict__ sc, const uint32_t* __restrict__ gk_prev,
+                                          const cplx* __restrict__ gv_prev, double* __restrict__ gy,
+                                          uint32_t* __restrict__ chain_key) {
+    __shared__ MuRows<D> R;
+    const int s = mg.bx * kMuThreads + threadIdx.x;
+    const int P = mu_stage<D>(R, IN, np, slot_base, mg.bx * kMuThreads, nslots, sc->H);
+    if (s >= nslots) return;
+    const int m = IN.m[P];
+    const int ts = s - slot_base[P];
+    const int t = (ts == 0) ? m : ts - 1;
+    const int i0 = slot_base[P] - R.base0;
+    const double* b = IN.b + (int64_t)P * D;
+    uint32_t integ;
+    const uint32_t negs = mu_masks<D>(R, i0, m, &integ);
+    double* g_out = gy + (int64_t)s * (2 + 2 * D);
+    if (t < m && !((integ >> t) & 1u)) {
+        flags[s] = 0;
+        chain_key[s] = 15u;
+        for (int k = 0; k < 2 + 2 * D; k++) g_out[k] = 0.0;
+        return;
+    }
+    chain_key[s] = (uint32_t)IN.tid[P];
+    const double zeta = sc->msmt - dev_dot<D>(sc->H, b);
+    double mut[D], cb[D], ty[D];
+#pragma unroll
+    for (int k = 0; k < D; k++) {
+        mut[k] = t == m ? 0.0 : R.mu[k][i0 + t];
+        cb[k] = b[k] + zeta * mut[k];
+        ty[k] = 0.0;
+    }
+    const double rho_t = t == m ? sc->gamma : R.rho[i0 + t];
+    const int phc = IN.phc[P];
+    const uint32_t lhp = phc < m ? negs & ((1u << phc) - 1u) : negs;
+    double ygi = 0.0;
+    uint32_t neg = 0;
+    for (int r = 0; r < m; r++) {
+        double row[D];
+        bool ho;
+        const double pr = mu_row<D>(R, i0, mut, sc->gamma, m, t, r, row, &ho);
+        double dr = 0.0;
+#pragma unroll
+        for (int k = 0; k < D; k++) dr += row[k] * sc->root[k];
+        const double sgn = dr > 0 ? 1 : -1;
+        if (sgn < 0) neg |= (1u << r);
+        const double scl = pr * sgn;
+#pragma unroll
+        for (int k = 0; k < D; k++) ty[k] += scl * row[k];
+        if (!ho) ygi += pr * sgn;
+    }
+    mu_moment<D>(IN, P, sc->first != 0, m, t, neg, lhp, ygi, rho_t, zeta, ty, cb, gk_prev, gv_prev, g_out);
+    flags[s] = kValid | ((t != m) ? kIsNew : 0);
+    shape[s] = m;
 }
 
 // ------------------------------------------------------------------ moments

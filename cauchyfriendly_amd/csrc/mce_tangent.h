@@ -279,9 +279,13 @@ __global__ void k_mu_tan(TermPool IN, TanPool TI, int np, const int* __restrict_
     const double* H = sc->H;
     const double zeta = sc->msmt - dev_dot<D>(H, b);
     const bool first = sc->first != 0;
-    const bool post = !sc->skip && !first;
     // nominal parent-table lookup of this slot's g (independent of the direction)
-    const int phc = OUT.phc[s], lhp = OUT.lhp[s];
+    const int phc = IN.phc[Pp];
+    int lhp = 0;
+    for (int l = 0; l < m && l < phc; l++) {
+        const double h = dev_dot<D>(H, A + l * D);
+        if (!(fabs(h) < kMuEps) && !(h > 0)) lhp |= 1 << l;
+    }
     const int64_t go = IN.gp_off[Pp];
     const int gn = IN.gp_n[Pp];
     double mut[D], dmut[D], row[kMaxM * D], drow[kMaxM * D], rho[kMaxM], drho[kMaxM], An[kMaxM * D], n1s[kMaxM];
@@ -317,12 +321,6 @@ __global__ void k_mu_tan(TermPool IN, TanPool TI, int np, const int* __restrict_
             child_row_tan<D>(A, p, dA, dp, H, dH, mut, dmut, sc->gamma, dgamma, m, t, r, row + r * D, drow + r * D,
                              rho + r, drho + r, &horth);
             if (horth) hf |= 1u << r;
-        }
-        double* tb_ = TO.tb(s, kk);
-        double bo[D];
-        for (int k = 0; k < D; k++) {
-            bo[k] = b[k] + zeta * mut[k];
-            tb_[k] = db[k] + dzeta * mut[k] + zeta * dmut[k];
         }
         // g at the root point: signs of the child rows, ygi over the rows that are not
         // H-orthogonal, the two parent-table numerators
@@ -366,12 +364,15 @@ __global__ void k_mu_tan(TermPool IN, TanPool TI, int np, const int* __restrict_
         const cplx dD1 = cmake(dygi + drho_t, dzeta), dD2 = cmake(dygi - drho_t, dzeta);
         const cplx v = csub(dquot(gp, dgp, D1, dD1), dquot(gm, dgm, D2, dD2));
         dg[(int64_t)s * NP + kk] = cscale(v, kInvTwoPi);
+        if (sc->skip) continue;  // a window's last update keeps no terms: TO may be empty
+        double* tb_ = TO.tb(s, kk);
+        for (int k = 0; k < D; k++) tb_[k] = db[k] + dzeta * mut[k] + zeta * dmut[k];
         *TO.tc(s, kk) = dzeta;
         *TO.tdv(s, kk) = drho_t;
         double* oA = TO.tA(s, kk);
         double* op = TO.tp(s, kk);
         double* oq = TO.tq(s, kk);
-        if (!post) {
+        if (first) {
             for (int r = 0; r < m; r++) {
                 for (int k = 0; k < D; k++) oA[r * D + k] = drow[r * D + k];
                 op[r] = drho[r];
