@@ -16,6 +16,7 @@
 #include <coroutine>
 #include <functional>
 #include <initializer_list>
+#include <map>
 #include <mutex>
 #include <optional>
 #include <cstdio>
@@ -231,48 +232,70 @@ inline BatchSlot* bslot() { return nullptr; }
 
 #define MCE_RUN(K_, G_, B_, L_, S_, ...) mce_run<&K_>(bslot(), (G_), (B_), (L_), (S_), #K_, __VA_ARGS__)
 
-// Device blocks of up to kMaxBlock bytes come from a process-wide cache with one free list
-// per power-of-two size.  An estimator that outgrows its buffers, or a new estimator of a
-// batch, takes blocks that others gave back instead of calling hipMalloc, which holds a
-// device-wide lock and slows down as live allocations multiply (thousands of small
-// estimators stepped from many host threads otherwise spend most of their time there).
-// Blocks of up to kSlabMax bytes are carved from slabs of several hundred blocks and stay
-// with the process; larger ones are allocated one by one and freed when the cache holds more
-// than kMaxCached.  A block is given back only when no queued work can touch it: after the
-// streams of the engine that used it were synchronised.  Larger blocks bypass the cache.
+// Device blocks come from a process-wide cache.  An estimator that outgrows its buffers, or
+// a new estimator of a batch, takes blocks that others gave back instead of calling
+// hipMalloc, which holds a device-wide lock and slows down as live allocations multiply
+// (thousands of small estimators stepped from many host threads otherwise spend most of
+// their time there), and which takes from 0.04 to over 2 s for the 19 GiB of a five-window
+// bank of 5-state windows when they were freed just before.  A block is given back only when
+// no queued work can touch it: after the streams of the engine that used it were synchronised.
+//
+// Up to kMaxBlock there is one free list per power-of-two size; blocks of up to kSlabMax
+// bytes are carved from slabs of several hundred blocks and stay with the process.  Larger
+// blocks (sizes in eighths of a power of two, so at most an eighth over what was asked) are
+// kept by size, and a request takes the smallest that holds it and is at most a quarter
+// larger.  Unslabbed blocks are freed when the cache would hold more than kMaxCached, or less
+// than a quarter of the device's memory is free (other processes and allocators share it);
+// large ones also once they lay unused for kIdle while others came and went, and all of them
+// when an allocation fails.
 class BlockCache {
    public:
     static constexpr size_t kMinBlock = 256;
     static constexpr size_t kSlabMax = size_t(4) << 20;
     static constexpr size_t kMaxBlock = size_t(256) << 20;
-    static constexpr size_t kMaxCached = size_t(16) << 30;  // unslabbed blocks beyond this are freed
+    static constexpr size_t kMaxCached = size_t(48) << 30;
+    static constexpr std::chrono::seconds kIdle{10};
 
     static size_t block_size(size_t bytes) {
-        if (bytes > kMaxBlock) return bytes;
         size_t s = kMinBlock;
         while (s < bytes) s <<= 1;
+        if (bytes > kMaxBlock) {
+            const size_t unit = s >> 4;  // s / 2 < bytes <= s: eighths of s / 2
+            s = (bytes + unit - 1) / unit * unit;
+        }
         return s;
     }
     // Bytes of the slab that blocks of `bytes` (a block_size() value <= kSlabMax) are cut from.
     static size_t slab_size(size_t bytes) {
         return std::min<size_t>(size_t(256) << 20, std::max<size_t>(size_t(4) << 20, bytes * 512));
     }
-    // `bytes` is a block_size() value.
-    void* get(size_t bytes) {
-        if (bytes <= kMaxBlock) {
+    // `bytes` is a block_size() value, and on return the size of the block.
+    void* get(size_t& bytes) {
+        {
             std::lock_guard<std::mutex> lk(mu_);
-            auto& l = free_[cls(bytes)];
-            if (l.empty() && bytes <= kSlabMax) {
-                const size_t sb = slab_size(bytes);
-                char* slab = (char*)raw_alloc(sb, true);
-                slab_bytes_ += sb;
-                for (size_t off = sb; off >= bytes; off -= bytes) l.push_back(slab + off - bytes);
-            }
-            if (!l.empty()) {
-                void* p = l.back();
-                l.pop_back();
-                if (bytes > kSlabMax) cached_ -= bytes;
-                return p;
+            if (bytes > kMaxBlock) {
+                const auto it = large_.lower_bound(bytes);
+                if (it != large_.end() && it->first <= bytes + bytes / 4) {
+                    void* p = it->second.p;
+                    bytes = it->first;
+                    cached_ -= bytes;
+                    large_.erase(it);
+                    return p;
+                }
+            } else {
+                auto& l = free_[cls(bytes)];
+                if (l.empty() && bytes <= kSlabMax) {
+                    const size_t sb = slab_size(bytes);
+                    char* slab = (char*)raw_alloc(sb, true);
+                    slab_bytes_ += sb;
+                    for (size_t off = sb; off >= bytes; off -= bytes) l.push_back(slab + off - bytes);
+                }
+                if (!l.empty()) {
+                    void* p = l.back();
+                    l.pop_back();
+                    if (bytes > kSlabMax) cached_ -= bytes;
+                    return p;
+                }
             }
         }
         return raw_alloc(bytes, false);
@@ -280,27 +303,50 @@ class BlockCache {
     // The caller guarantees that no queued work reads or writes the block.
     void put(void* p, size_t bytes) {
         if (!p) return;
-        if (bytes <= kMaxBlock) {
+        std::vector<void*> gone;
+        {
+            size_t avail = 0, total = 0;
+            const bool room = bytes <= kMaxBlock || (hipMemGetInfo(&avail, &total) == hipSuccess && avail >= total / 4);
             std::lock_guard<std::mutex> lk(mu_);
             if (bytes <= kSlabMax) {
                 free_[cls(bytes)].push_back(p);
                 return;
             }
-            if (cached_ + bytes <= kMaxCached) {
-                free_[cls(bytes)].push_back(p);
+            const auto now = std::chrono::steady_clock::now();
+            if (bytes > kMaxBlock)
+                for (auto it = large_.begin(); it != large_.end();) {
+                    if (now - it->second.since < kIdle) {
+                        ++it;
+                        continue;
+                    }
+                    gone.push_back(it->second.p);
+                    cached_ -= it->first;
+                    it = large_.erase(it);
+                }
+            if (!room || cached_ + bytes > kMaxCached) {
+                gone.push_back(p);
+            } else {
+                if (bytes > kMaxBlock)
+                    large_.emplace(bytes, Idle{p, now});
+                else
+                    free_[cls(bytes)].push_back(p);
                 cached_ += bytes;
-                return;
             }
         }
-        (void)hipFree(p);
+        for (void* g : gone) (void)hipFree(g);
     }
 
    private:
+    struct Idle {
+        void* p;
+        std::chrono::steady_clock::time_point since;
+    };
     // `locked`: the caller holds mu_.
     void* raw_alloc(size_t bytes, bool locked) {
         void* p = nullptr;
         hipError_t e = hipMalloc(&p, bytes);
         if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
             if (locked) {
                 trim_unslabbed();
             } else {
@@ -321,11 +367,14 @@ class BlockCache {
             for (void* p : free_[c]) (void)hipFree(p);
             free_[c].clear();
         }
+        for (auto& [size, b] : large_) (void)hipFree(b.p);
+        large_.clear();
         cached_ = 0;
     }
     static int cls(size_t bytes) { return __builtin_ctzll(bytes); }
     std::mutex mu_;
     std::vector<void*> free_[64];
+    std::multimap<size_t, Idle> large_;
     size_t cached_ = 0, slab_bytes_ = 0;
 };
 
@@ -335,30 +384,14 @@ BlockCache& block_cache() {
 }
 
 // Allocations outgrown while an engine works on this host thread.  The engine gives them
-// back once its streams are idle: blocks of the cache's sizes at the end of the call, larger
-// ones (hipFree synchronises the whole device, which would stall every other estimator
-// stepped concurrently) when they add up to more than a bound or the engine goes.  Outside an
+// back to the block cache once its streams are idle, at the end of the call; outside an
 // engine they are given back at once, after a device synchronisation.
 struct Graveyard {
     std::vector<std::pair<void*, size_t>> blocks;
-    size_t bytes = 0, big_bytes = 0;
-    void add(void* p, size_t b) {
-        blocks.emplace_back(p, b);
-        bytes += b;
-        if (b > BlockCache::kMaxBlock) big_bytes += b;
-    }
-    // Gives back the cache-sized blocks, and the larger ones too if `all`.
-    void release(bool all) {
-        std::vector<std::pair<void*, size_t>> keep;
-        for (auto& [p, b] : blocks) {
-            if (all || b <= BlockCache::kMaxBlock)
-                block_cache().put(p, b);
-            else
-                keep.emplace_back(p, b);
-        }
-        blocks.swap(keep);
-        bytes = big_bytes = 0;
-        for (auto& [p, b] : blocks) bytes += b, big_bytes += b;
+    void add(void* p, size_t b) { blocks.emplace_back(p, b); }
+    void release() {
+        for (auto& [p, b] : blocks) block_cache().put(p, b);
+        blocks.clear();
     }
 };
 thread_local Graveyard* t_graveyard = nullptr;
@@ -394,7 +427,7 @@ struct DBuf {
             ptr = nullptr;
             cap = bytes = 0;
         }
-        const size_t b = BlockCache::block_size(nn * sizeof(T));
+        size_t b = BlockCache::block_size(nn * sizeof(T));
         ptr = (T*)block_cache().get(b);
         bytes = b;
         cap = b / sizeof(T);
@@ -603,7 +636,38 @@ struct ThreadStreams {
         HIPCHK(hipHostGetDevicePointer((void**)&total_dev, total, 0));
     }
 };
-thread_local ThreadStreams t_streams;
+// A host thread that ends hands its streams and slots to the next new one: a caller that
+// starts its threads anew for each call would otherwise leave two streams per thread behind
+// at every call.  Work still queued on them (a call that failed) runs before the next
+// owner's, in stream order.
+struct ThreadStreamsOwner : ThreadStreams {
+    static std::mutex& mu() {
+        static std::mutex* m = new std::mutex();  // never destroyed: threads may outlive static teardown
+        return *m;
+    }
+    static std::vector<ThreadStreams>& idle() {
+        static auto* v = new std::vector<ThreadStreams>();
+        return *v;
+    }
+    void init() {
+        if (st) return;
+        {
+            std::lock_guard<std::mutex> lk(mu());
+            if (!idle().empty()) {
+                static_cast<ThreadStreams&>(*this) = idle().back();
+                idle().pop_back();
+                return;
+            }
+        }
+        ThreadStreams::init();
+    }
+    ~ThreadStreamsOwner() {
+        if (!st) return;
+        std::lock_guard<std::mutex> lk(mu());
+        idle().push_back(*this);
+    }
+};
+thread_local ThreadStreamsOwner t_streams;
 
 // ---------------------------------------------------------------- engine
 struct Engine {
@@ -709,16 +773,14 @@ struct Engine {
     DBuf<cplx> contrib;
     Profiler prof;
     Graveyard graveyard;
-    static constexpr size_t kGraveyardBytes = size_t(4) << 30;  // released early beyond this
 
-    // Gives back the outgrown allocations once this engine's streams are idle: every one if
-    // `all`, else the cache-sized ones, and the larger ones beyond kGraveyardBytes.
-    void bury(bool all = true) {
+    // Gives back the outgrown allocations once this engine's streams are idle.
+    void bury() {
         if (graveyard.blocks.empty()) return;
         bind();
         HIPCHK(hipStreamSynchronize(st));
         HIPCHK(hipStreamSynchronize(st2));
-        graveyard.release(all || graveyard.big_bytes > kGraveyardBytes);
+        graveyard.release();
     }
 
     Engine(int num_steps, int d_, int cmcc_, int pncc_, int p_, const double* A0_, const double* p0_,
@@ -797,7 +859,7 @@ struct Engine {
         bind();
         (void)hipStreamSynchronize(st);
         (void)hipStreamSynchronize(st2);
-        graveyard.release(true);
+        graveyard.release();
         if (ev_mu) (void)hipEventDestroy(ev_mu);
         if (ev_c0) (void)hipEventDestroy(ev_c0);
         if (ev_c1) (void)hipEventDestroy(ev_c1);
@@ -1472,7 +1534,7 @@ struct Engine {
             GraveyardScope gs(&graveyard);
             r = co_await update_terms(msmt, Phi, Gamma, beta, Hrow, gamma, Bm, u);
         }
-        bury(false);
+        bury();
         co_return r;
     }
 
@@ -2951,7 +3013,7 @@ class BatchRunner {
         for (Job& jb : jobs) {
             jb.e->bs = nullptr;
             jb.e->prof.on = jb.prof_on;
-            jb.e->graveyard.release(jb.e->graveyard.big_bytes > Engine::kGraveyardBytes);
+            jb.e->graveyard.release();
         }
         if (profiling_) {
             unsigned long long b = 0;
