@@ -717,7 +717,7 @@ struct Engine {
     int ntan = 0;
     TanStore tin, tout;
     DBuf<cplx> dgv[2];
-    DBuf<cplx> dg_slot, dfz_dev;
+    DBuf<cplx> dg_slot, dg_part, dfz_dev;
     DBuf<double> dgscale_dev;
     DBuf<StepTan> dstan;
     DBuf<uint8_t> mem_add;
@@ -1631,7 +1631,7 @@ struct Engine {
                     {hist_mx.ptr, (sr + 2) * sizeof(int), 0}});
         // tangents first: k_tp_tan reads the parents before k_tp propagates them in place
         if (ntan)
-            MCE_DISPATCH_D(d, MCE_LAUNCH(k_tp_tan<DD>, dim3(ceil_div(np, 256)), dim3(256), 0, st, IN, tin.view(), np,
+            MCE_DISPATCH_D(d, MCE_LAUNCH(k_tp_tan<DD>, dim3(np), dim3(64), 0, st, IN, tin.view(), np,
                                          dconst.ptr, dstan.ptr));
         MCE_DISPATCH_D(d, MCE_RUN(k_tp<DD>, dim3(ceil_div(np, 256)), dim3(256), 0, st, IN, np, dconst.ptr,
                                              dcen_half.ptr, slots.ptr, btcap.ptr, counters.ptr + 8));
@@ -1754,10 +1754,13 @@ struct Engine {
             if (!skip) tout.reserve(nslots);
             dg_slot.reserve((size_t)nslots * ntan);
             dfz_dev.reserve(ntan);
-            MCE_DISPATCH_D(d, MCE_LAUNCH(k_mu_tan<DD>, dim3(ceil_div(nslots, 128)), dim3(128), 0, st, IN, tin.view(),
-                                         np, slot_base.ptr, OUT, tout.view(), nslots, dconst.ptr, dstan.ptr,
-                                         gk[gcur].ptr, gv[gcur].ptr, dgv[gcur].ptr, dg_slot.ptr));
-            MCE_LAUNCH(k_tan_colsum, dim3(ntan), dim3(256), 0, st, dg_slot.ptr, nslots, ntan, dfz_dev.ptr);
+            MCE_DISPATCH_D(d, MCE_LAUNCH(k_mu_tan<DD>, dim3(np), dim3(128), mu_tan_lds(MM, d, ntan), st, IN, tin.view(),
+                                         np, slot_base.ptr, OUT, tout.view(), dconst.ptr, dstan.ptr, gk[gcur].ptr,
+                                         gv[gcur].ptr, dgv[gcur].ptr, dg_slot.ptr));
+            const int nb = std::min(kTanSumBlocks, ceil_div(nslots, 64));
+            dg_part.reserve((size_t)nb * ntan);
+            MCE_LAUNCH(k_tan_colsum, dim3(nb), dim3(256), 0, st, dg_slot.ptr, nslots, ntan, dg_part.ptr);
+            MCE_LAUNCH(k_tan_colsum_finish, dim3(1), dim3(64), 0, st, dg_part.ptr, nb, ntan, dfz_dev.ptr);
         }
         prof.mark(kPhMu, st);
 
@@ -1880,7 +1883,7 @@ struct Engine {
         if (ntan) {
             dgv[nx].reserve((size_t)n * cells * ntan);
             tin.reserve(n);
-            MCE_DISPATCH_D(d, MCE_LAUNCH(k_gtable_first_tan<DD>, dim3(ceil_div(n, 64)), dim3(64), 0, st, OUT,
+            MCE_DISPATCH_D(d, MCE_LAUNCH(k_gtable_first_tan<DD>, dim3(n), dim3(256), 0, st, OUT,
                                          tout.view(), n, perm.ptr, gscale, dgscale_dev.ptr, dgv[nx].ptr, tin.view()));
         }
         HIPCHK(hipGetLastError());
@@ -2038,10 +2041,16 @@ struct Engine {
         }
         if (ntan) {
             dgv[nx].reserve(((size_t)cells_total + 1) * ntan);
-            MCE_LAUNCH(k_group_tan, dim3(ng), dim3(64), 0, st, OUT, tout.view(), ng, d, grp_moff.ptr, grp_mcnt.ptr,
-                       grp_m.ptr, mem_slots.ptr, mem_add.ptr, surv.ptr, gxor.ptr, b2arena.ptr, b2off.ptr, b2n.ptr,
-                       goff.ptr, gk[gcur].ptr, gv[gcur].ptr, dgv[gcur].ptr, gk[nx].ptr, gscale, dgscale_dev.ptr,
-                       dgv[nx].ptr);
+            auto launch_tan = [&](auto k, int waves) {
+                MCE_LAUNCH(k, dim3(ng), dim3(64 * waves), 0, st, OUT, tout.view(), ng, d, grp_moff.ptr, grp_mcnt.ptr,
+                           grp_m.ptr, mem_slots.ptr, mem_add.ptr, surv.ptr, gxor.ptr, b2arena.ptr, b2off.ptr, b2n.ptr,
+                           goff.ptr, gk[gcur].ptr, gv[gcur].ptr, dgv[gcur].ptr, gk[nx].ptr, gscale, dgscale_dev.ptr,
+                           dgv[nx].ptr);
+            };
+            if (ng < kTanOneWave)
+                launch_tan(k_group_tan<4>, 4);
+            else
+                launch_tan(k_group_tan<1>, 1);
         }
         prof.mark(kPhGEval, st);
 
@@ -2056,7 +2065,7 @@ struct Engine {
                                              surv.ptr, spos.ptr, grp_m.ptr, goff.ptr, b2n.ptr, NEXT));
         if (ntan) {
             tin.reserve(std::max(ng, 1));
-            MCE_DISPATCH_D(d, MCE_LAUNCH(k_compact_tan<DD>, dim3(ceil_div(ng, 256)), dim3(256), 0, st, tout.view(), ng,
+            MCE_DISPATCH_D(d, MCE_LAUNCH(k_compact_tan<DD>, dim3(ceil_div(ng, 4)), dim3(256), 0, st, tout.view(), ng,
                                          surv.ptr, spos.ptr, grp_m.ptr, tin.view()));
         }
         HIPCHK(hipGetLastError());
