@@ -705,6 +705,8 @@ struct Engine {
     // MCE_GEVAL_MODE=0..3 selects the g-table lookup mode (tuning; unsupported choices are ignored)
     int geval_mode_override = getenv("MCE_GEVAL_MODE") ? atoi(getenv("MCE_GEVAL_MODE")) : -1;
     // MCE_BIG_GROUP_MEMBERS: groups with more members add them one wavefront per member
+    // groups from which on one wavefront takes a group's tangents (k_group_tan)
+    int tan_one_wave = getenv("MCE_TAN_ONE_WAVE") ? atoi(getenv("MCE_TAN_ONE_WAVE")) : kTanOneWave;
     int big_group_members = getenv("MCE_BIG_GROUP_MEMBERS") ? std::max(0, atoi(getenv("MCE_BIG_GROUP_MEMBERS")))
                                                             : kBigGroupMembers;
     // MCE_ENUM_THREADS=64|128|256: lanes per parent in the TP cell enumerator
@@ -2047,7 +2049,7 @@ struct Engine {
                            goff.ptr, gk[gcur].ptr, gv[gcur].ptr, dgv[gcur].ptr, gk[nx].ptr, gscale, dgscale_dev.ptr,
                            dgv[nx].ptr);
             };
-            if (ng < kTanOneWave)
+            if (ng < tan_one_wave)
                 launch_tan(k_group_tan<4>, 4);
             else
                 launch_tan(k_group_tan<1>, 1);
