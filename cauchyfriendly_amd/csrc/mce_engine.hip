@@ -695,8 +695,7 @@ struct Engine {
     hipStream_t st = nullptr;
     hipStream_t st2 = nullptr;  // moment chains, overlapped with the reduction phase
     hipEvent_t ev_mu = nullptr, ev_c0 = nullptr, ev_c1 = nullptr;
-    DBuf<uint32_t> chain_key, chain_skey, chain_perm;
-    DBuf<int> chain_off;
+    DBuf<int> chain_rel, chain_len;
     int cur_T = 1;
     bool moments_pending = false;
     int max_gp_cells = 1;  // largest parent g-table of the current parents
@@ -730,7 +729,7 @@ struct Engine {
     DBuf<uint32_t> barena, b2arena, tmpk;
     DBuf<cplx> tmpv;
     DBuf<StepConst> dconst;
-    DBuf<double> dbpert, gy, mom_part, mom_out, mom_x;
+    DBuf<double> dbpert, gy, mom_part, mom_out;
     DBuf<uint8_t> dcombos;
     DBuf<int64_t> dcombo_off;
     DBuf<int> dcombo_cnt, dcen_half;
@@ -1454,35 +1453,20 @@ struct Engine {
     // cauchy_estimator.hpp:524-602 with eval_g_yei_after_ftr, cauchy_term.hpp:403-433), summed
     // in term order, and printed.  Without it fz is 1 after reduction.
     bool debug_after_ftr = false;
-    DBuf<double> dbg_gy, dbg_x, dbg_part;
-    DBuf<uint8_t> dbg_flags;
-    DBuf<uint32_t> dbg_chain;
-    DBuf<int> dbg_off;
+    DBuf<double> dbg_gy, dbg_part;
     Co<void> moments_after_ftr() {
         const int n = Nt;
         const int NC = 1 + d + d * d;
         TermPool P = in.view();
         dbg_gy.reserve((size_t)std::max(n, 1) * (2 + 2 * d));
-        dbg_flags.reserve(std::max(n, 1));
-        dbg_chain.reserve(std::max(n, 1));
-        dbg_off.reserve(2);
         dbg_part.reserve((size_t)NC * 2 + 1);
         std::vector<double> part((size_t)NC * 2 + 1, 0.0);
         if (n > 0) {
             MCE_DISPATCH_D(d, MCE_RUN(k_after_ftr_gy<DD>, dim3(ceil_div(n, 256)), dim3(256), 0, st, P, n, dconst.ptr,
                                       gk[gcur].ptr, gv[gcur].ptr, dbg_gy.ptr));
-            fill_multi({{dbg_flags.ptr, (size_t)n, kValid}});
-            MCE_RUN(k_iota, dim3(ceil_div(n, 256)), dim3(256), 0, st, dbg_chain.ptr, n);
-            const int off2[2] = {0, n};
-            upload(dbg_off.ptr, off2, sizeof(off2));
-            int ncp = 0, nyb = 0;
-            MCE_DISPATCH_D(d, (nyb = mom_blocks<DD>(), ncp = nyb * kSumCW / 2));
-            dbg_x.reserve((size_t)nyb * n * kSumCW);
             // one chain over the terms in order: the reference's sequential sums
-            MCE_DISPATCH_D(d, MCE_RUN(k_mom_terms<DD>, dim3(ceil_div((int64_t)n * ncp, 256)), dim3(256), 0, st,
-                                      dbg_gy.ptr, dbg_flags.ptr, dbg_chain.ptr, dbg_off.ptr, 1, n, dbg_x.ptr));
-            MCE_DISPATCH_D(d, MCE_RUN(k_mom_sum<DD>, dim3(1, nyb), dim3(256), 0, st, dbg_x.ptr, dbg_off.ptr, 1,
-                                      dbg_part.ptr, counters.ptr + 17));
+            MCE_DISPATCH_D(d, MCE_RUN(k_mom_sum<DD>, dim3(1, mom_blocks<DD>()), dim3(64 * kSumWaves), 0, st, dbg_gy.ptr,
+                                      (const int*)nullptr, 1, n, dbg_part.ptr, counters.ptr + 17));
             co_await rd(dbg_part.ptr, part.data(), (int)part.size());
         }
         fz = cmake(part[0], part[1]);
@@ -1724,32 +1708,34 @@ struct Engine {
             keys.reserve(nslots);
         }
         gy.reserve((size_t)nslots * (2 + 2 * d));
-        chain_key.reserve(nslots);
-        chain_skey.reserve(nslots);
-        chain_perm.reserve(nslots);
-        iota.reserve(nslots);
-        chain_off.reserve(16);
+        if (T > 1) {
+            chain_rel.reserve(np);
+            chain_len.reserve(T);
+            MCE_RUN(k_chain_pos, dim3(T), dim3(1024), 0, st, slots.ptr, dconst.ptr, sr, chain_rel.ptr, chain_len.ptr);
+        }
         mom_part.reserve((size_t)T * (1 + d + d * d) * 2 + 1);
         TermPool OUT = out.view();
         const int mu_km = MM <= 8 ? 8 : MM <= 14 ? 14 : 0;
         if (skip) {
             MCE_DISPATCH_D(d, MCE_RUN(k_mu_last<DD>, dim3(ceil_div(nslots, kMuThreads)), dim3(kMuThreads), 0, st, IN,
                                       np, slot_base.ptr, out.flags.ptr, out.m.ptr, nslots, dconst.ptr, gk[gcur].ptr,
-                                      gv[gcur].ptr, gy.ptr, chain_key.ptr));
+                                      gv[gcur].ptr, gy.ptr, chain_rel.ptr, chain_len.ptr));
         } else if (mu_km == 8) {
             // child rows in registers when the largest shape fits a compile-time bound
             MCE_DISPATCH_D(d, MCE_RUN((k_mu_r<DD, 8>), dim3(ceil_div(nslots, kMuThreads)), dim3(kMuThreads), 0, st, IN,
                                                  np, slot_base.ptr, OUT, nslots, dconst.ptr, gk[gcur].ptr,
-                                                 gv[gcur].ptr, gy.ptr, keys.ptr, chain_key.ptr, counters.ptr + 17));
+                                                 gv[gcur].ptr, gy.ptr, keys.ptr, chain_rel.ptr, chain_len.ptr,
+                                                 counters.ptr + 17));
         } else if (mu_km == 14 && d <= 5) {
             MCE_DISPATCH_D(d, if constexpr (DD <= 5) MCE_RUN(
                                   (k_mu_r<DD, 14>), dim3(ceil_div(nslots, kMuThreads)), dim3(kMuThreads), 0, st, IN, np,
                                   slot_base.ptr, OUT, nslots, dconst.ptr, gk[gcur].ptr, gv[gcur].ptr, gy.ptr, keys.ptr,
-                                  chain_key.ptr, counters.ptr + 17));
+                                  chain_rel.ptr, chain_len.ptr, counters.ptr + 17));
         } else {
             MCE_DISPATCH_D(d, MCE_RUN(k_mu<DD>, dim3(ceil_div(nslots, 256)), dim3(256), 0, st, IN, np,
                                                  slot_base.ptr, OUT, nslots, dconst.ptr, gk[gcur].ptr, gv[gcur].ptr,
-                                                 gy.ptr, keys.ptr, chain_key.ptr, counters.ptr + 17));
+                                                 gy.ptr, keys.ptr, chain_rel.ptr, chain_len.ptr,
+                                                 counters.ptr + 17));
         }
         HIPCHK(hipGetLastError());
         if (ntan) {
@@ -1766,25 +1752,14 @@ struct Engine {
         }
         prof.mark(kPhMu, st);
 
-        // ---- moments: slots in reference-thread chain order, then the chains on st2
-        MCE_RUN(k_iota, dim3(ceil_div(nslots, 256)), dim3(256), 0, st, iota.ptr, nslots);
-        sort_pairs(chain_key.ptr, chain_skey.ptr, iota.ptr, chain_perm.ptr, nslots, 0, 4);
-        MCE_RUN(k_chain_off, dim3(1), dim3(16), 0, st, chain_skey.ptr, nslots, T, chain_off.ptr);
+        // ---- moments: the chains' sums on st2
         if (!bs) {
             HIPCHK(hipEventRecord(ev_mu, st));
             HIPCHK(hipStreamWaitEvent(st2, ev_mu, 0));
         }
         if (prof.on) HIPCHK(hipEventRecord(ev_c0, st2));
-        {
-            int ncp = 0, nyb = 0;
-            MCE_DISPATCH_D(d, (nyb = mom_blocks<DD>(), ncp = nyb * kSumCW / 2));
-            mom_x.reserve((size_t)nyb * nslots * kSumCW);
-            MCE_DISPATCH_D(d, MCE_RUN(k_mom_terms<DD>, dim3(ceil_div((int64_t)nslots * ncp, 256)), dim3(256),
-                                                 0, st2, gy.ptr, out.flags.ptr, chain_perm.ptr, chain_off.ptr, T,
-                                                 nslots, mom_x.ptr));
-            MCE_DISPATCH_D(d, MCE_RUN(k_mom_sum<DD>, dim3(T, nyb), dim3(256), 0, st2, mom_x.ptr,
-                                                 chain_off.ptr, T, mom_part.ptr, counters.ptr + 17));
-        }
+        MCE_DISPATCH_D(d, MCE_RUN(k_mom_sum<DD>, dim3(T, mom_blocks<DD>()), dim3(64 * kSumWaves), 0, st2, gy.ptr,
+                                  chain_len.ptr, T, nslots, mom_part.ptr, counters.ptr + 17));
         HIPCHK(hipGetLastError());
         if (prof.on) HIPCHK(hipEventRecord(ev_c1, st2));
         cur_T = T;
@@ -1813,7 +1788,7 @@ struct Engine {
             iota.reserve(nslots);
             perm.reserve(nslots);
             skeys.reserve(nslots);
-            // iota still holds 0..nslots-1: the chain sort only read it
+            MCE_RUN(k_iota, dim3(ceil_div(nslots, 256)), dim3(256), 0, st, iota.ptr, nslots);
             sort_pairs(keys.ptr, skeys.ptr, iota.ptr, perm.ptr, nslots, 0, kGatherKeyBits);
             MCE_RUN(k_hist, dim3(std::min(ceil_div(nslots, 256), 1024)), dim3(256), 0, st, nslots, sr + 1, 0,
                                out.flags.ptr, out.m.ptr, (const int*)nullptr, (const uint32_t*)nullptr, hist.ptr);

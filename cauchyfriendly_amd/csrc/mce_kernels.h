@@ -5,7 +5,7 @@
 //   k_btab_simple      B-tables that need no enumeration (copy / identity / empty)
 //   k_btab_enum        time-propagation B-table by vertex enumeration, one block per parent
 //   k_mu               measurement update, one thread per output slot (parent x child)
-//   k_mom_terms/sum    fz / mean / covariance summands, then in-order sums per
+//   k_mom_sum          fz / mean / covariance summands and their in-order sums per
 //                      reference thread (second stream, overlapped with reduction)
 //   k_ftr_*            fast term reduction of all shape buckets: keys, components, groups
 //   k_group_btab       B-table of each reduction group's root, one wavefront per group
@@ -841,6 +841,64 @@ __device__ inline int dev_mu_coalign(double* A, double* p, double* q, uint8_t* c
     return ns;
 }
 
+// ------------------------------------------------------------------ moment chains
+// Moment sums run in the reference's exact order.  Reference thread t owns parents
+// i = t, t+T, ... of every shape bucket (cauchy_estimator.hpp:1575-1604) and adds,
+// per parent, the parent's own term before its children (cache_moments,
+// cauchy_estimator.hpp:307-338 and 1436-1468): chain t is the output slots (parent first) of
+// its parents in order.  The measurement update writes a slot's moment inputs at its chain's
+// position, so the sums read them as they come; one chain (T == 1) is the slots themselves.
+//
+// rel[i]: slots of chain t before parent i's, len[t]: slots of the chain.  One workgroup per
+// chain over its parents.  Sorting the slots by chain instead took three launches of a small
+// update and a radix sort of every slot of a large one.
+__device__ __forceinline__ void k_chain_pos(MG<1024, 1> mg, const int* __restrict__ slots,
+                                            const StepConst* __restrict__ sc, int sr, int* __restrict__ rel,
+                                            int* __restrict__ len) {
+    __shared__ int cum[kMaxM + 2];  // parents of the chain in the buckets before each
+    const int t = mg.bx, T = sc->T;
+    if (threadIdx.x == 0) {
+        int c = 0;
+        for (int b = 0; b < sr; b++) {
+            cum[b] = c;
+            const int n = sc->in_off[b + 1] - sc->in_off[b];
+            c += n > t ? (n - t - 1) / T + 1 : 0;
+        }
+        cum[sr] = c;
+    }
+    __syncthreads();
+    const int n = cum[sr];
+    int carry = 0;
+    for (int q0 = 0; q0 < n; q0 += blockDim.x) {
+        const int q = q0 + threadIdx.x;
+        int i = -1;
+        if (q < n) {
+            int b = 0;
+            while (cum[b + 1] <= q) b++;
+            i = sc->in_off[b] + t + T * (q - cum[b]);
+        }
+        int total;
+        const int x = block_excl_scan(i >= 0 ? slots[i] : 0, &total);
+        if (i >= 0) rel[i] = carry + x;
+        carry += total;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) len[t] = carry;
+}
+
+// First position of chain t.
+__device__ __forceinline__ int chain_begin(const int* __restrict__ len, int t) {
+    int o = 0;
+    for (int u = 0; u < t; u++) o += len[u];
+    return o;
+}
+
+// Position of slot s, the ts-th of parent P of chain t.
+__device__ __forceinline__ int64_t chain_pos(const StepConst* __restrict__ sc, const int* __restrict__ rel,
+                                             const int* __restrict__ len, int t, int P, int s, int ts) {
+    return sc->T > 1 ? chain_begin(len, t) + rel[P] + ts : s;
+}
+
 // ------------------------------------------------------------------ measurement update
 // cauchy_term.hpp:84-310 (msmt_update) + cache_moments inputs + MU coalignment,
 // one thread per output slot.  Slot t < m of parent P is its child t; slot m is
@@ -850,7 +908,7 @@ template <int D>
 __device__ __forceinline__ void k_mu(MG<1024, 1> mg, TermPool IN, int np, const int* __restrict__ slot_base, TermPool OUT, int nslots,
                      const StepConst* __restrict__ sc, const uint32_t* __restrict__ gk_prev,
                      const cplx* __restrict__ gv_prev, double* __restrict__ gy, uint32_t* __restrict__ keys_out,
-                     uint32_t* __restrict__ chain_key, int* __restrict__ err) {
+                     const int* __restrict__ chain_rel, const int* __restrict__ chain_len, int* __restrict__ err) {
     const int s = mg.bx * blockDim.x + threadIdx.x;
     if (s >= nslots) return;
     int lo = 0, hi = np - 1;
@@ -877,15 +935,13 @@ __device__ __forceinline__ void k_mu(MG<1024, 1> mg, TermPool IN, int np, const 
             if (!(h > 0)) negs |= (1u << l);
         }
     }
-    double* g_out = gy + (int64_t)s * (2 + 2 * D);
+    double* g_out = gy + chain_pos(sc, chain_rel, chain_len, IN.tid[P], P, s, ts) * (2 + 2 * D);
     if (t < m && !((integ >> t) & 1u)) {
         OUT.flags[s] = 0;
         keys_out[s] = kGatherKeyNone;
-        chain_key[s] = 15u;
         for (int k = 0; k < 2 + 2 * D; k++) g_out[k] = 0.0;
         return;
     }
-    chain_key[s] = (uint32_t)IN.tid[P];
     const double zeta = sc->msmt - dev_dot<D>(H, b);
     double mut[D];
     double rho_t;
@@ -1190,7 +1246,8 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
                                              int nslots, const StepConst* __restrict__ sc,
                                              const uint32_t* __restrict__ gk_prev, const cplx* __restrict__ gv_prev,
                                              double* __restrict__ gy, uint32_t* __restrict__ keys_out,
-                                             uint32_t* __restrict__ chain_key, int* __restrict__ err) {
+                                             const int* __restrict__ chain_rel, const int* __restrict__ chain_len,
+                                             int* __restrict__ err) {
     __shared__ MuRows<D> R;
     const int s = mg.bx * kMuThreads + threadIdx.x;
     const int P = mu_stage<D>(R, IN, np, slot_base, mg.bx * kMuThreads, nslots, sc->H);
@@ -1208,15 +1265,13 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
     const double* H = sc->H;
     uint32_t integ;
     const uint32_t negs = mu_masks<D>(R, i0, m, &integ);
-    double* g_out = gy + (int64_t)s * (2 + 2 * D);
+    double* g_out = gy + chain_pos(sc, chain_rel, chain_len, IN.tid[P], P, s, ts) * (2 + 2 * D);
     if (t < m && !((integ >> t) & 1u)) {
         OUT.flags[s] = 0;
         keys_out[s] = kGatherKeyNone;
-        chain_key[s] = 15u;
         for (int kk = 0; kk < 2 + 2 * D; kk++) g_out[kk] = 0.0;
         return;
     }
-    chain_key[s] = (uint32_t)IN.tid[P];
     const double zeta = sc->msmt - dev_dot<D>(H, b);
     double mut[D];
 #pragma unroll
@@ -1345,7 +1400,7 @@ __device__ __forceinline__ void k_mu_last(MG<256, 4> mg, TermPool IN, int np, co
                                           uint8_t* __restrict__ flags, int* __restrict__ shape, int nslots,
                                           const StepConst* __restrict__ sc, const uint32_t* __restrict__ gk_prev,
                                           const cplx* __restrict__ gv_prev, double* __restrict__ gy,
-                                          uint32_t* __restrict__ chain_key) {
+                                          const int* __restrict__ chain_rel, const int* __restrict__ chain_len) {
     __shared__ MuRows<D> R;
     const int s = mg.bx * kMuThreads + threadIdx.x;
     const int P = mu_stage<D>(R, IN, np, slot_base, mg.bx * kMuThreads, nslots, sc->H);
@@ -1357,14 +1412,12 @@ __device__ __forceinline__ void k_mu_last(MG<256, 4> mg, TermPool IN, int np, co
     const double* b = IN.b + (int64_t)P * D;
     uint32_t integ;
     const uint32_t negs = mu_masks<D>(R, i0, m, &integ);
-    double* g_out = gy + (int64_t)s * (2 + 2 * D);
+    double* g_out = gy + chain_pos(sc, chain_rel, chain_len, IN.tid[P], P, s, ts) * (2 + 2 * D);
     if (t < m && !((integ >> t) & 1u)) {
         flags[s] = 0;
-        chain_key[s] = 15u;
         for (int k = 0; k < 2 + 2 * D; k++) g_out[k] = 0.0;
         return;
     }
-    chain_key[s] = (uint32_t)IN.tid[P];
     const double zeta = sc->msmt - dev_dot<D>(sc->H, b);
     double mut[D], cb[D], ty[D];
 #pragma unroll
@@ -1398,22 +1451,11 @@ __device__ __forceinline__ void k_mu_last(MG<256, 4> mg, TermPool IN, int np, co
 }
 
 // ------------------------------------------------------------------ moments
-// Moment sums in the reference's exact order.  Reference thread t owns parents
-// i = t, t+T, ... of every shape bucket (cauchy_estimator.hpp:1575-1604) and adds,
-// per parent, the parent's own term before its children (cache_moments,
-// cauchy_estimator.hpp:307-338 and 1436-1468).  `chain` lists the output slots in
-// exactly that order (slots are parent-first), so chain t is one contiguous range
-// [chain_off[t], chain_off[t+1]) of chain positions.
-//
-// Two kernels: k_mom_terms writes every summand of every chain position (fully
-// parallel), k_mom_sum adds them in order, one lane per double of a component.
-// Summands are grouped in blocks of kSumCW doubles: X[(yb * npos + pos) * kSumCW + c]
-// holds double yb * kSumCW + c (component / 2, real or imaginary part) of position
-// pos.  Padding and slots without a term hold +0.0: an in-order sum that starts at
-// +0.0 never becomes -0.0, so adding +0.0 leaves it unchanged.
-constexpr int kSumCW = 8;     // doubles per summand block (lanes of the adding wave)
-constexpr int kSumTP = 288;   // positions per LDS tile (tile = 12 doubles per loader thread)
-constexpr int kSumDepth = 3;  // tiles in flight in loader registers
+constexpr int kSumCW = 16;    // doubles (twice the components) one workgroup sums
+constexpr int kSumTP = 224;   // positions per LDS tile
+constexpr int kSumWaves = 8;  // the adding wave and seven that form the summands
+static_assert(kSumTP % 32 == 0, "the adding wave takes a full tile 32 positions at a time");
+constexpr int kSumDepth = 3;  // tiles whose inputs are in flight in registers
 
 template <int D>
 __host__ __device__ constexpr int mom_blocks() {
@@ -1423,7 +1465,7 @@ __host__ __device__ constexpr int mom_blocks() {
 // Moments after term reduction (debug mode), cauchy_term.hpp:403-433 (eval_g_yei_after_ftr)
 // over every parent term: the sign vector of its hyperplanes at the root point (bit l set
 // where A_l . root <= 0), y_j = -(sum_l (p_l s_l) A_lj) + i b_j, and g its own g-table's value
-// at that sign vector.  Writes (g, y) per term in the layout k_mom_terms reads.
+// at that sign vector.  Writes (g, y) per term in the layout k_mom_sum reads.
 template <int D>
 __device__ __forceinline__ void k_after_ftr_gy(MG<1024, 1> mg, const TermPool P, int n,
                                                const StepConst* __restrict__ sc, const uint32_t* __restrict__ gk,
@@ -1463,147 +1505,138 @@ __device__ __forceinline__ void k_after_ftr_gy(MG<1024, 1> mg, const TermPool P,
     }
 }
 
-// Products with the reference's operations: g, g*y_j and the negated (g*y_j)*y_k
-// (the reference subtracts the latter; a - b == a + (-b) exactly).
+// In-order sums of g, g*y_j and the negated (g*y_j)*y_k over each chain (the reference
+// subtracts the latter; a - b == a + (-b) exactly), with the reference's operations.  Grid
+// (T, mom_blocks): a workgroup sums kSumCW doubles of chain blockIdx.x.  Seven waves form the
+// summands of a tile of positions out of the slots' (g, y) and leave them in a two-tile LDS
+// ring, with the inputs of the next kSumDepth tiles in flight; wave 0 adds, a lane per
+// double, bound by the latency of dependent double-precision additions (the last
+// update of a 5-state window, 1.45M slots in 8 chains of 62 doubles: 2.0 ms; 1.0 ms of summands
+// written to memory and read back and 3.1 ms of sums before, whose adding wave waited for LDS
+// reads under a condition).
+// Slots without a term hold zeros and add +-0.0, which leaves a sum that starts at +0.0
+// unchanged; padding is +0.0.  part[t][c] receives the sum of chain t, and part[T * NC2] the
+// measurement update's error bits (*mu_err), so one copy brings both back.  `len` is not read
+// when T == 1: the chain is all n slots.
 template <int D>
-__device__ __forceinline__ void k_mom_terms(MG<1024, 1> mg, const double* __restrict__ gy, const uint8_t* __restrict__ flags,
-                            const uint32_t* __restrict__ chain, const int* __restrict__ chain_off, int T, int nslots,
-                            double* __restrict__ X) {
+__device__ __forceinline__ void k_mom_sum(MG<64 * kSumWaves, 2> mg, const double* __restrict__ gy,
+                                          const int* __restrict__ len, int T, int n, double* __restrict__ part,
+                                          const int* __restrict__ mu_err) {
     constexpr int NS = 2 + 2 * D;
     constexpr int NC = 1 + D + D * D;
-    constexpr int NCP = mom_blocks<D>() * kSumCW / 2;  // padded components per position
-    const int64_t i = (int64_t)mg.bx * blockDim.x + threadIdx.x;
-    const int pos = (int)(i / NCP);
-    const int cc = (int)(i - (int64_t)pos * NCP);
-    if (pos >= nslots) return;
-    const int npos = chain_off[T];
-    if (pos >= npos) return;
-    const uint32_t s = chain[pos];
-    double2 out = make_double2(0.0, 0.0);
-    if (cc < NC && (flags[s] & kValid)) {
-        const double* rec = gy + (int64_t)s * NS;
-        const cplx g = cmake(rec[0], rec[1]);
-        cplx x;
-        if (cc == 0) {
-            x = g;
-        } else if (cc <= D) {
-            x = cmul(g, cmake(rec[2 + 2 * (cc - 1)], rec[3 + 2 * (cc - 1)]));
-        } else {
-            const int j = (cc - 1 - D) / D, kk = (cc - 1 - D) % D;
-            const cplx gyj = cmul(g, cmake(rec[2 + 2 * j], rec[3 + 2 * j]));
-            const cplx q = cmul(gyj, cmake(rec[2 + 2 * kk], rec[3 + 2 * kk]));
-            x = cmake(-q.re, -q.im);
-        }
-        out = make_double2(x.re, x.im);
-    }
-    const int c2 = 2 * cc;
-    const int yb = c2 / kSumCW, c = c2 % kSumCW;
-    *reinterpret_cast<double2*>(X + ((int64_t)yb * npos + pos) * kSumCW + c) = out;
-}
-
-// In-order sums.  Grid (T, mom_blocks), 256 threads: wave 0 adds, lane c < kSumCW
-// owning double blockIdx.y * kSumCW + c; waves 1-3 stream the chain's summand block
-// through a two-tile LDS ring, holding kSumDepth tiles in registers so that the
-// loads of a tile are in flight while the tiles before it are added.  part[t][c2]
-// receives the sum of chain t.
-template <int D>
-// part[T * NC2] also receives the measurement update's error bits (*mu_err), so one copy
-// brings both back.
-__device__ __forceinline__ void k_mom_sum(MG<256, 1> mg, const double* __restrict__ X, const int* __restrict__ chain_off,
-                                                 int T, double* __restrict__ part, const int* __restrict__ mu_err) {
-    constexpr int NC2 = 2 * (1 + D + D * D);
-    constexpr int TE = kSumTP * kSumCW;          // doubles per tile
-    constexpr int NL = 192;                      // loader threads
-    constexpr int PER = TE / NL;                 // doubles per loader thread per tile
-    static_assert(PER * NL == TE, "a tile is an exact multiple of the loader threads");
-    __shared__ double ring[2][TE];
+    constexpr int CB = kSumCW / 2;                        // components of the workgroup
+    constexpr int PT = 64 * (kSumWaves - 1) / CB;         // positions the producers take at once
+    constexpr int PER = kSumTP / PT;                      // ... and times per tile
+    static_assert(PER * PT == kSumTP, "a tile is an exact multiple of the producers");
+    __shared__ __align__(16) double ring[2][kSumTP * kSumCW];
     const int t = mg.bx;
     const int yb = mg.by;
     const int tid = threadIdx.x;
-    if (t == 0 && yb == 0 && tid == 0) part[T * NC2] = (double)mu_err[0];
-    const int npos = chain_off[T];
-    const int beg = chain_off[t], end = chain_off[t + 1];
-    const int ntiles = (end - beg + kSumTP - 1) / kSumTP;
-    const double* Xb = X + ((int64_t)yb * npos + beg) * kSumCW;  // this chain's block, tile 0 first
-    const int64_t lim = (int64_t)(end - beg) * kSumCW;           // doubles of the chain
-    const bool loader = __builtin_amdgcn_readfirstlane(tid >> 6) != 0;  // wave 0 adds
-    const int l = tid - 64;
-    double rg[kSumDepth][PER];
-
-    // Loads are unconditional (address clamped into the chain) so that no load is
-    // skipped and the wait for the oldest tile stays exact; values past the chain's
-    // end are replaced by +0.0 when the tile is stored to LDS, not at load time,
-    // so the loads stay in flight until then.
-    auto gload = [&](double (&r)[PER], int tile) {
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int64_t o = (int64_t)tile * TE + l + NL * q;
-            r[q] = Xb[o < lim ? o : lim - 1];
-        }
-    };
-    auto lstore = [&](const double (&r)[PER], int tile, double* dst) {
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int64_t o = (int64_t)tile * TE + l + NL * q;
-            dst[l + NL * q] = o < lim ? r[q] : 0.0;
-        }
-    };
+    if (t == 0 && yb == 0 && tid == 0) part[(int64_t)T * 2 * NC] = (double)mu_err[0];
+    const int beg = T > 1 ? chain_begin(len, t) : 0;
+    const int cnt = T > 1 ? len[t] : n;
+    const int ntiles = (cnt + kSumTP - 1) / kSumTP;
+    const bool adder = __builtin_amdgcn_readfirstlane(tid >> 6) == 0;
     // LDS-only barrier: global loads stay in flight across it
     auto lds_barrier = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     };
-
-    // The two roles run separate loops; each performs exactly nsteps + 1 barriers.
-    // The step count is padded to a multiple of kSumDepth so that every unrolled
-    // step is unconditional (the compiler then keeps the later tiles' loads in
-    // flight); padded tiles hold +0.0 only.
+    // The two roles run separate loops; each performs exactly nsteps + 1 barriers.  The step
+    // count is padded to a multiple of kSumDepth so that every unrolled step is unconditional
+    // (the compiler then keeps the later tiles' loads in flight).
     const int nsteps = (ntiles + kSumDepth - 1) / kSumDepth * kSumDepth;
-    double acc = 0.0;
-    const int lane = tid & 63;
-    if (loader) {
+    if (!adder) {
+        const int l = tid - 64;
+        const int c = l % CB, p0 = l / CB;
+        const int cc = yb * CB + c;
+        // operands of this thread's component: g, y_j where jo, y_k where ko
+        const bool live = cc < NC, jo = live && cc > 0, ko = live && cc > D;
+        const int j = !jo ? 0 : ko ? (cc - 1 - D) / D : cc - 1, k = ko ? (cc - 1 - D) % D : 0;
+        const double* base = gy + (int64_t)beg * NS;
+        double2 rg[kSumDepth][PER], rj[kSumDepth][PER], rk[kSumDepth][PER];
+        // Loads are unconditional (position clamped into the chain) so that no load is
+        // skipped and the wait for the oldest tile stays exact.
+        auto load = [&](int u, int tile) {
+#pragma unroll
+            for (int q = 0; q < PER; q++) {
+                const int pos = min(tile * kSumTP + q * PT + p0, cnt - 1);
+                const double* rec = base + (int64_t)pos * NS;
+                rg[u][q] = *(const double2*)rec;
+                rj[u][q] = *(const double2*)(rec + 2 + 2 * j);
+                rk[u][q] = *(const double2*)(rec + 2 + 2 * k);
+            }
+        };
+        auto form = [&](int u, int tile, double* dst) {
+#pragma unroll
+            for (int q = 0; q < PER; q++) {
+                const int pos = q * PT + p0;
+                cplx x = cmake(rg[u][q].x, rg[u][q].y);
+                const cplx xj = cmul(x, cmake(rj[u][q].x, rj[u][q].y));
+                if (jo) x = xj;
+                const cplx xk = cmul(x, cmake(rk[u][q].x, rk[u][q].y));
+                if (ko) x = cmake(-xk.re, -xk.im);
+                if (!live || tile * kSumTP + pos >= cnt) x = cmake(0.0, 0.0);
+                *(double2*)(dst + pos * kSumCW + 2 * c) = make_double2(x.re, x.im);
+            }
+        };
         if (nsteps > 0) {
 #pragma unroll
-            for (int j = 0; j < kSumDepth; j++) gload(rg[j], j);
-            lstore(rg[0], 0, ring[0]);
-            gload(rg[0], kSumDepth);
+            for (int u = 0; u < kSumDepth; u++) load(u, u);
+            form(0, 0, ring[0]);
+            load(0, kSumDepth);
         }
         lds_barrier();
         for (int k0 = 0; k0 < nsteps; k0 += kSumDepth) {
 #pragma unroll
             for (int u = 0; u < kSumDepth; u++) {
-                const int k = k0 + u;
+                const int s = k0 + u;
                 // u is a compile-time index once the loop is unrolled
-                lstore(rg[(u + 1) % kSumDepth], k + 1, ring[(k + 1) & 1]);
-                gload(rg[(u + 1) % kSumDepth], k + 1 + kSumDepth);
+                form((u + 1) % kSumDepth, s + 1, ring[(s + 1) & 1]);
+                load((u + 1) % kSumDepth, s + 1 + kSumDepth);
                 lds_barrier();
             }
         }
     } else {
+        const int lane = tid;
+        double acc = 0.0;
         lds_barrier();
-        for (int k = 0; k < nsteps; k++) {
-            if (lane < kSumCW) {
-                const double* src = ring[k & 1] + lane;
-                double cur[16], nxt[16];
+        for (int s = 0; s < nsteps; s++) {
+            if (lane < kSumCW && s < ntiles) {
+                const double* src = ring[s & 1] + lane;
+                const int left = cnt - s * kSumTP;
+                double ev[16], od[16];
+                auto take = [&](double (&v)[16], int blk) {
 #pragma unroll
-                for (int q = 0; q < 16; q++) cur[q] = src[q * kSumCW];
-                for (int r0 = 0; r0 < kSumTP; r0 += 16) {
-                    if (r0 + 16 < kSumTP) {
+                    for (int q = 0; q < 16; q++) v[q] = src[(blk * 16 + q) * kSumCW];
+                };
+                auto add = [&](const double (&v)[16]) {
 #pragma unroll
-                        for (int q = 0; q < 16; q++) nxt[q] = src[(r0 + 16 + q) * kSumCW];
+                    for (int q = 0; q < 16; q++) acc += v[q];
+                };
+                if (left >= kSumTP) {
+                    // reads of the next 16 summands are always in flight, none of them under
+                    // a condition, so the additions wait for nothing but each other
+                    take(ev, 0);
+                    for (int r = 0; r < kSumTP / 16; r += 2) {
+                        take(od, r + 1);
+                        add(ev);
+                        take(ev, min(r + 2, kSumTP / 16 - 1));
+                        add(od);
                     }
-#pragma unroll
-                    for (int q = 0; q < 16; q++) acc += cur[q];
-#pragma unroll
-                    for (int q = 0; q < 16; q++) cur[q] = nxt[q];
+                } else {
+                    for (int r = 0; r * 16 < left; r++) {
+                        take(ev, r);
+                        add(ev);
+                    }
                 }
             }
             lds_barrier();
         }
+        const int c2 = yb * kSumCW + lane;
+        if (lane < kSumCW && c2 < 2 * NC) part[(int64_t)t * 2 * NC + c2] = acc;
     }
-    const int c2 = yb * kSumCW + lane;
-    if (!loader && lane < kSumCW && c2 < NC2) part[(int64_t)t * NC2 + c2] = acc;
 }
 
 // Histogram of small integer values privatised in LDS (nbins <= 64).  mode 0: valid
@@ -2938,19 +2971,6 @@ __device__ __forceinline__ void k_prof_sum(MG<1024, 1> mg, int n, const int* __r
         v = (unsigned long long)max(a[i], 0) * (unsigned long long)(b ? max(b[i], 0) : 1);
     for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_down(v, o, kWave);
     if ((threadIdx.x & (kWave - 1)) == 0 && v) atomicAdd(acc, v);
-}
-
-// Start of each reference thread's chain in the sorted chain keys (T+1 entries).
-__device__ __forceinline__ void k_chain_off(MG<1024, 1> mg, const uint32_t* __restrict__ skeys, int n, int T, int* __restrict__ off) {
-    const int t = threadIdx.x;
-    if (t > T) return;
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (skeys[mid] < (uint32_t)t) lo = mid + 1;
-        else hi = mid;
-    }
-    off[t] = lo;
 }
 
 // ------------------------------------------------------------------ small helpers
