@@ -681,11 +681,6 @@ struct Engine {
     double gscale = 0;
     std::vector<int> in_count;  // per-shape term counts of the parent pool
     // largest hyperplane count among the parent pool's terms (0 when it is empty)
-    int largest_shape() const {
-        for (int m = (int)in_count.size() - 1; m > 0; m--)
-            if (in_count[m] > 0) return m;
-        return 0;
-    }
     // diagnostics of the last update
     bool have_diag = false;
     std::vector<double> diag_mom;
@@ -2189,6 +2184,9 @@ struct Engine {
     DBuf<CpdfTerm1D> cpdf_cache;
     // relative-system scratch (held by the primary estimator of a pair)
     DBuf<double> rs_mom, rs_sums, rs_part;
+    DBuf<RsysStep> rs_steps;
+    DBuf<RsysTerm> rs_terms;
+    DBuf<double2> rs_shares;
     DBuf<uint8_t> rs_keep;
     DBuf<int> rs_idx, rs_cnt;
     DBuf<int> c2_mc, c2_err;
@@ -2378,13 +2376,13 @@ struct Grid2DShape {
     }
 };
 
-static void launch_grid_2d(hipStream_t st, const Cpdf2D& C, int n, const Grid2DShape& g, const int* idx,
-                           const double* px, const double* py, int npts, double* part, int* err) {
+static void launch_grid_2d(hipStream_t st, const Cpdf2D& C, int n, const Grid2DShape& g, const double* px,
+                           const double* py, int npts, double* part, int* err) {
     const dim3 grid(ceil_div(npts, kGridLanes * g.points), g.chunks), block(kGridLanes * kGridWaves);
     if (g.points == 2)
-        MCE_LAUNCH((k_cpdf2d_grid<2>), grid, block, 0, st, C, n, g.terms, idx, px, py, npts, part, err);
+        MCE_LAUNCH((k_cpdf2d_grid<2>), grid, block, 0, st, C, n, g.terms, px, py, npts, part, err);
     else
-        MCE_LAUNCH((k_cpdf2d_grid<1>), grid, block, 0, st, C, n, g.terms, idx, px, py, npts, part, err);
+        MCE_LAUNCH((k_cpdf2d_grid<1>), grid, block, 0, st, C, n, g.terms, px, py, npts, part, err);
 }
 
 int Engine::cpdf_2d(int i1, int i2, double lox, double hix, double resx, double loy, double hiy, double resy,
@@ -2448,7 +2446,7 @@ int Engine::cpdf_2d(int i1, int i2, double lox, double hix, double resx, double 
                                              cpdf_direct.ptr, c2_err.ptr));
         MCE_LAUNCH(k_sum_fixed, dim3(1), dim3(1024), 0, st, cpdf_direct.ptr, Nt, cpdf_sum.ptr);
         if (npts > 1) {
-            launch_grid_2d(st, C, Nt, shape, nullptr, c2_px.ptr + 1, c2_py.ptr + 1, npts - 1, cpdf_part.ptr, c2_err.ptr);
+            launch_grid_2d(st, C, Nt, shape, c2_px.ptr + 1, c2_py.ptr + 1, npts - 1, cpdf_part.ptr, c2_err.ptr);
             MCE_LAUNCH(k_cpdf1d_finish, dim3(ceil_div(npts - 1, kFinishPoints)), dim3(kFinishPoints * kFinishSlices), 0, st, cpdf_part.ptr,
                                nchunks, npts - 1, 1.0, cpdf_y.ptr + 1);
             HIPCHK(hipGetLastError());
@@ -2515,10 +2513,6 @@ static int64_t rsys_2d(Engine& P, Engine& S, const double* Trel, double eps, dou
     GraveyardScope gs(&P.graveyard);
     hipStream_t st = P.st;
     HIPCHK(hipStreamSynchronize(S.st));
-    P.c2_mc.reserve(npairs);
-    P.c2_b2.reserve(2 * npairs);
-    P.c2_wall.reserve(npairs * (CM + 1));
-    P.c2_cell.reserve(npairs * CM);
     P.rs_mom.reserve(npairs * 14);
     P.rs_keep.reserve(npairs);
     P.rs_idx.reserve(npairs);
@@ -2526,31 +2520,25 @@ static int64_t rsys_2d(Engine& P, Engine& S, const double* Trel, double eps, dou
     P.rs_sums.reserve(14);
     P.rs_part.reserve(14 * kColSlices);
     P.c2_err.reserve(1);
-    Cpdf2D C;
-    C.MM = CM;
-    C.mc = P.c2_mc.ptr;
-    C.b2 = P.c2_b2.ptr;
-    C.wall = P.c2_wall.ptr;
-    C.cell = P.c2_cell.ptr;
+    Cpdf2D C{CM, nullptr, nullptr, nullptr, nullptr};
     TermPool PI = P.in.view(), SI = S.in.view();
+    auto pairs = [&](auto kernel, int64_t n, const int* idx) {
+        MCE_LAUNCH(kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, PI, SI, ns, n, d, idx, P.rs_steps.ptr,
+                   P.rs_terms.ptr, P.rs_steps.ptr + (size_t)np * (P.MM + 1), P.rs_terms.ptr + np, P.rs_shares.ptr, R, C,
+                   P.rs_mom.ptr, P.rs_keep.ptr);
+    };
     if (npairs > 0) {
-        const unsigned blocks = (unsigned)((npairs + 127) / 128);
-        // per-lane arrays sized by the pairs' largest row count: the smaller the bound,
-        // the smaller each lane's private memory
-        const int KM = P.largest_shape() + S.largest_shape();
-        HIPCHK(hipMemsetAsync(P.c2_err.ptr, 0, sizeof(int), st));
-#define MCE_RSYS(K_)                                                                                             \
-    MCE_DISPATCH_D(d, MCE_LAUNCH((k_rsys_pairs<DD, K_>), dim3(blocks), dim3(128), 0, st, PI, np,         \
-                                         P.gk[P.gcur].ptr, P.gv[P.gcur].ptr, SI, ns, S.gk[S.gcur].ptr,           \
-                                         S.gv[S.gcur].ptr, R, C, P.rs_mom.ptr, P.rs_keep.ptr, P.c2_err.ptr))
-        if (KM <= 16) {
-            MCE_RSYS(16);
-        } else if (KM <= 24) {
-            MCE_RSYS(24);
-        } else {
-            MCE_RSYS(kMaxM);
-        }
-#undef MCE_RSYS
+        // both terms' tables with the primary's estimator (the two may be one)
+        P.rs_steps.reserve((size_t)np * (P.MM + 1) + (size_t)ns * (S.MM + 1));
+        P.rs_terms.reserve((size_t)np + ns);
+        P.rs_shares.reserve((size_t)ns * S.MM);
+        RsysStep* ssteps = P.rs_steps.ptr + (size_t)np * (P.MM + 1);
+        RsysTerm* sterms = P.rs_terms.ptr + np;
+        MCE_LAUNCH(k_rsys_terms, dim3(np), dim3(64), 0, st, PI, np, d, -1.0, P.gk[P.gcur].ptr, P.gv[P.gcur].ptr, R,
+                   P.rs_steps.ptr, P.rs_terms.ptr, (double2*)nullptr);
+        MCE_LAUNCH(k_rsys_terms, dim3(ns), dim3(64), 0, st, SI, ns, d, 1.0, S.gk[S.gcur].ptr, S.gv[S.gcur].ptr, R,
+                   ssteps, sterms, P.rs_shares.ptr);
+        pairs(k_rsys_pairs<false>, npairs, nullptr);
         MCE_LAUNCH(k_colsum_part, dim3(kColSlices, 14), dim3(256), 0, st, P.rs_mom.ptr, npairs,
                            P.rs_part.ptr);
         MCE_LAUNCH(k_colsum_finish, dim3(1), dim3(64), 0, st, P.rs_part.ptr, 14, P.rs_sums.ptr);
@@ -2567,14 +2555,12 @@ static int64_t rsys_2d(Engine& P, Engine& S, const double* Trel, double eps, dou
         HIPCHK(hipGetLastError());
     }
     double sums[14] = {0};
-    int nkeep = 0, pair_err = 0;
+    int nkeep = 0;
     if (npairs > 0) {
         HIPCHK(hipMemcpyAsync(sums, P.rs_sums.ptr, sizeof(sums), hipMemcpyDeviceToHost, st));
         HIPCHK(hipMemcpyAsync(&nkeep, P.rs_cnt.ptr, sizeof(int), hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(&pair_err, P.c2_err.ptr, sizeof(int), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
     }
-    if (pair_err) throw std::runtime_error("a relative term has more rows than the pair kernel was launched for");
     // finalize_rel_sys_moments (cauchy_prediction.hpp:288-304)
     nf = cmake(sums[0], sums[1]);
     const cplx ifz = cmake(0.0, nf.re);
@@ -2612,7 +2598,13 @@ static int64_t rsys_2d(Engine& P, Engine& S, const double* Trel, double eps, dou
         HIPCHK(hipMemcpyAsync(P.c2_px.ptr, px.data(), npts * sizeof(double), hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(P.c2_py.ptr, py.data(), npts * sizeof(double), hipMemcpyHostToDevice, st));
         HIPCHK(hipMemsetAsync(P.c2_err.ptr, 0, sizeof(int), st));
-        launch_grid_2d(st, C, nkeep, shape, P.rs_idx.ptr, P.c2_px.ptr, P.c2_py.ptr, npts, P.cpdf_part.ptr, P.c2_err.ptr);
+        P.c2_mc.reserve(nkeep);
+        P.c2_b2.reserve(2 * (size_t)nkeep);
+        P.c2_wall.reserve((size_t)nkeep * (CM + 1));
+        P.c2_cell.reserve((size_t)nkeep * CM);
+        C = Cpdf2D{CM, P.c2_mc.ptr, P.c2_b2.ptr, P.c2_wall.ptr, P.c2_cell.ptr};
+        pairs(k_rsys_pairs<true>, nkeep, P.rs_idx.ptr);
+        launch_grid_2d(st, C, nkeep, shape, P.c2_px.ptr, P.c2_py.ptr, npts, P.cpdf_part.ptr, P.c2_err.ptr);
         MCE_LAUNCH(k_cpdf1d_finish, dim3(ceil_div(npts, kFinishPoints)), dim3(kFinishPoints * kFinishSlices), 0, st, P.cpdf_part.ptr, nchunks, npts,
                            1.0, P.cpdf_y.ptr);
         HIPCHK(hipGetLastError());

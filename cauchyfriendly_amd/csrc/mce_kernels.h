@@ -3570,7 +3570,6 @@ constexpr int kGridLanes = 64;
 constexpr int kGridWaves = 4;
 template <int P>
 __global__ void __launch_bounds__(kGridLanes* kGridWaves) k_cpdf2d_grid(Cpdf2D C, int n, int chunk_terms,
-                                                                        const int* __restrict__ idx,
                                                                         const double* __restrict__ px,
                                                                         const double* __restrict__ py, int npts,
                                                                         double* __restrict__ part,
@@ -3593,8 +3592,7 @@ __global__ void __launch_bounds__(kGridLanes* kGridWaves) k_cpdf2d_grid(Cpdf2D C
         acc[j] = 0.0;
     }
     bool singular = false;
-    for (int tt = t0; tt < t1; tt++) {
-        const int64_t t = idx ? idx[tt] : tt;
+    for (int64_t t = t0; t < t1; t++) {
         const int u = C.mc[t];
         if (u <= 0) continue;
         const Wall2D* __restrict__ W = C.wall + t * (MM + 1);
@@ -3700,273 +3698,259 @@ struct RsysArgs {
 
 __device__ inline double sgn_d(double x) { return (double)((x > 0) - (x < 0)); }
 
-template <int D, int K>
-__global__ void k_rsys_pairs(TermPool P, int np, const uint32_t* __restrict__ pkeys, const cplx* __restrict__ pvals,
-                             TermPool S, int ns, const uint32_t* __restrict__ skeys, const cplx* __restrict__ svals,
-                             RsysArgs R, Cpdf2D C, double* __restrict__ mom, uint8_t* __restrict__ keep,
-                             int* __restrict__ err) {
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= (int64_t)np * ns) return;
-    const int tp = (int)(q / ns), ts = (int)(q % ns);
-    const int mp = P.m[tp], ms = S.m[ts];
-    const int m = mp + ms;
-    // K bounds the rows of every pair (the two pools' largest shapes); a pair above it
-    // is reported, never evaluated
-    if (m > K) {
-        atomicOr(err, 2);
-        keep[q] = 0;
-        return;
-    }
-    const double* Ap = P.A + (int64_t)tp * P.MM * D;
-    const double* As = S.A + (int64_t)ts * S.MM * D;
-    // per-lane arrays, sized by K: the merged rows are compacted into a2 / p2 in place
-    double a2[2 * K], p2[K], th[2 * K];
-    int8_t cmap[K], csm[K], fidx[K];
-    bool F[K];
-    // A_2d = A_rel Trel^T (matmatmul with the second operand transposed), p_2d = p_rel
-    for (int i = 0; i < m; i++) {
-        const bool pr = i < mp;
-        const double* ar = pr ? Ap + i * D : As + (i - mp) * D;
-        const double sg = pr ? -1.0 : 1.0;
-        for (int k = 0; k < 2; k++) {
-            double acc = 0.0;
-            for (int j = 0; j < D; j++) acc += (ar[j] * sg) * R.T[k * D + j];
-            a2[2 * i + k] = acc;
-        }
-        p2[i] = pr ? P.p[(int64_t)tp * P.MM + i] : S.p[(int64_t)ts * S.MM + (i - mp)];
-    }
-    double b2[2];
-    {
-        double br[kMaxD];
-        for (int j = 0; j < D; j++) br[j] = S.b[(int64_t)ts * D + j] - P.b[(int64_t)tp * D + j];
-        for (int k = 0; k < 2; k++) {
-            double acc = 0.0;
-            for (int j = 0; j < D; j++) acc += R.T[k * D + j] * br[j];
-            b2[k] = acc;
-        }
-    }
-    // zero rows marked, the others L1-normalised in place; +/- equal rows merged
-    for (int r = 0; r < m; r++) {
-        const double f0 = fabs(a2[2 * r]), f1 = fabs(a2[2 * r + 1]);
-        if (f0 < kMuEps && f1 < kMuEps) {
-            cmap[r] = csm[r] = fidx[r] = kZeroHpMarker;
-            F[r] = false;
+// A pair's rows are its two terms' rows, so everything about a row is formed once per term
+// (k_rsys_terms), where one thread per pair formed all of it in private memory: u angles, 2 u
+// sines and cosines, a sort and u^2 sums and merge tests (u rows): 119 ms for two 5-state
+// estimators of two steps, 4.6 ms in the two passes below.  A row vanishes on a line through the origin, at angle th in [0, pi]; going
+// round, its side flips there and nowhere else within half a turn.  So a term's lines in order,
+// with its Re gamma sums and g value before each, are all that the cells of a pair need: the
+// cells lie between the merged lines of both terms, sums add and g values multiply.
+struct RsysStep {
+    double th, s, c;    // the line's angle (infinity after the last line), sin, cos
+    double a0, a1;      // its row, L1-normalised
+    double g1, g2;      // Re gamma of the term's rows before the line
+    double gre, gim, gabs;  // the term's g value before the line, and its modulus
+};
+struct RsysTerm {
+    double ty0, ty1;  // the rows' shares of Re y at bar_nu, summed
+    cplx g;           // the term's g value there
+};
+
+// One wavefront per term; sg: -1 for the primary's rows, +1 for the secondary's.
+// steps: [term][MM + 1]; shares ([term][MM], may be null): every row's share of Re y.
+__global__ __launch_bounds__(64) void k_rsys_terms(TermPool P, int n, int d, double sg,
+                                                   const uint32_t* __restrict__ keys, const cplx* __restrict__ vals,
+                                                   RsysArgs R, RsysStep* __restrict__ steps,
+                                                   RsysTerm* __restrict__ terms, double2* __restrict__ shares) {
+    __shared__ double ty[2][kMaxM];
+    __shared__ double th[kMaxM], sn[kMaxM], cs[kMaxM], a0s[kMaxM], a1s[kMaxM], bp[kMaxM];
+    __shared__ int row[kMaxM];
+    const int t = blockIdx.x;
+    if (t >= n) return;
+    const int r = threadIdx.x;
+    const int MM = P.MM;
+    const int m = P.m[t];
+    const int mask = (1 << m) - 1, top = 1 << (m - 1);
+    double a0 = 0, a1 = 0, p = 0, ang = 0, c = 1, s = 0, beta = 0;
+    bool zero = true, neg_nu = false, neg = false;
+    if (r < m) {
+        const double* A = P.A + ((int64_t)t * MM + r) * d;
+        for (int j = 0; j < d; j++) a0 += (A[j] * sg) * R.T[j];
+        for (int j = 0; j < d; j++) a1 += (A[j] * sg) * R.T[d + j];
+        p = P.p[(int64_t)t * MM + r];
+        // rows that vanish under Trel keep the side of bar_nu, the others are L1-normalised
+        const double f0 = fabs(a0), f1 = fabs(a1);
+        zero = f0 < kMuEps && f1 < kMuEps;
+        double ds = 0.0;
+        if (zero) {
+            for (int j = 0; j < d; j++) ds += (A[j] * sg) * R.nu[j];
         } else {
             const double sa = f0 + f1;
-            a2[2 * r] /= sa;
-            a2[2 * r + 1] /= sa;
-            p2[r] *= sa;
-            F[r] = true;
+            a0 /= sa;
+            a1 /= sa;
+            p *= sa;
+            ds = a0 * R.nu2[0] + a1 * R.nu2[1];
+            const bool flat = fabs(a0) < fabs(a1);
+            ang = flat ? atan2(-a0 / a1, 1.0) : atan2(1.0, -a1 / a0);
+            if (ang < 0) ang += kPi;
+            sincos(ang, &s, &c);
+            beta = a0 * s - a1 * c > 0 ? 1.0 : -1.0;  // the row's side before its line
         }
+        const double sgi = sgn_d(ds);
+        neg_nu = sgi < 0;
+        neg = zero ? ds < 0 : beta < 0;
+        ty[0][r] = a0 * (p * sgi);
+        ty[1][r] = a1 * (p * sgi);
+        if (shares) shares[(int64_t)t * MM + r] = make_double2(ty[0][r], ty[1][r]);
     }
-    const uint32_t* pk = pkeys + P.gp_off[tp];
-    const cplx* pv = pvals + P.gp_off[tp];
-    const int pn = P.gp_n[tp];
-    const uint32_t* sk = skeys + S.gp_off[ts];
-    const cplx* sv_ = svals + S.gp_off[ts];
-    const int sn_ = S.gp_n[ts];
-    // moment contribution: the cell of bar_nu (Trel bar_nu in 2D, bar_nu on zero rows);
-    // taken before the merge, which leaves a2 and p2 as they are until the compaction
-    {
-        double ty0 = 0.0, ty1 = 0.0;
-        int encp = 0, encs = 0;
-        for (int i = 0; i < m; i++) {
-            double ds;
-            if (F[i]) {
-                ds = a2[2 * i] * R.nu2[0] + a2[2 * i + 1] * R.nu2[1];
-            } else {
-                const bool pr = i < mp;
-                const double* ar = pr ? Ap + i * D : As + (i - mp) * D;
-                const double sg = pr ? -1.0 : 1.0;
-                ds = 0.0;
-                for (int j = 0; j < D; j++) ds += (ar[j] * sg) * R.nu[j];
-            }
-            const double sgi = sgn_d(ds);
-            ty0 += a2[2 * i] * (p2[i] * sgi);
-            ty1 += a2[2 * i + 1] * (p2[i] * sgi);
-            if (sgi < 0) {
-                if (i < mp) encp |= 1 << i;
-                else encs |= 1 << (i - mp);
-            }
+    const int enc_nu = (int)__ballot(neg_nu), enc0 = (int)__ballot(neg);
+    const bool line = r < m && !zero;
+    const int u = __popcll(__ballot(line));
+    // the lines in order of their angles (of the rows, where equal)
+    int rank = 0;
+    for (int q = 0; q < m; q++) {
+        const double o = __shfl(ang, q, kWave);
+        const bool lq = __shfl((int)line, q, kWave) != 0;
+        rank += lq && (o < ang || (o == ang && q < r));
+    }
+    if (line) {
+        th[rank] = ang;
+        sn[rank] = s;
+        cs[rank] = c;
+        a0s[rank] = a0;
+        a1s[rank] = a1;
+        bp[rank] = beta * p;
+        row[rank] = r;
+    }
+    __syncthreads();
+    const uint32_t* pk = keys + P.gp_off[t];
+    const cplx* pv = vals + P.gp_off[t];
+    const int pn = P.gp_n[t];
+    if (r <= u) {
+        // before line r: lines 0 .. r-1 crossed
+        int enc = enc0;
+        double g1 = 0.0, g2 = 0.0;
+        for (int j = 0; j < u; j++) {
+            const double w = j < r ? bp[j] : -bp[j];
+            g1 += a0s[j] * w;
+            g2 += a1s[j] * w;
+            if (j < r) enc ^= 1 << row[j];
         }
-        const cplx gp = lookup_num(encp, 1 << (mp - 1), (1 << mp) - 1, pk, pv, pn);
-        const cplx gs = lookup_num(encs, 1 << (ms - 1), (1 << ms) - 1, sk, sv_, sn_);
-        const cplx g = cmul(gp, gs);
+        const cplx g = lookup_num(enc, top, mask, pk, pv, pn);
+        RsysStep o;
+        const bool end = r == u;
+        o.th = end ? __builtin_inf() : th[r];
+        o.s = end ? 0.0 : sn[r];
+        o.c = end ? 1.0 : cs[r];
+        o.a0 = end ? 0.0 : a0s[r];
+        o.a1 = end ? 0.0 : a1s[r];
+        o.g1 = g1;
+        o.g2 = g2;
+        o.gre = g.re;
+        o.gim = g.im;
+        o.gabs = hypot(g.re, g.im);
+        steps[(int64_t)t * (MM + 1) + r] = o;
+    }
+    if (r == 0) {
+        RsysTerm o;
+        o.ty0 = o.ty1 = 0.0;
+        for (int j = 0; j < m; j++) {
+            o.ty0 += ty[0][j];
+            o.ty1 += ty[1][j];
+        }
+        o.g = lookup_num(enc_nu, top, mask, pk, pv, pn);
+        terms[t] = o;
+    }
+}
+
+// One thread per pair walks the lines of both terms in order: per line one 80-byte step of
+// either term, two sums, a product and the cell it closes, in registers.  Lines whose rows
+// agree within kCoalignEps up to sign, the last line with the first included, bound no cell
+// between them.  First (CELLS false) every pair's moments and whether the approximation keeps
+// it; then (CELLS true) the cells of the n kept pairs idx[0 .. n), which the grid reads.  The
+// cells are 80 bytes each in separate stretches per lane, and writing them bounds the second
+// pass, so pairs that are dropped write none: 2.6 + 1.9 ms, where one pass that wrote every
+// pair's took 19.8 ms.  The first is bound by the latency of the steps' loads.
+template <bool CELLS>
+__global__ __launch_bounds__(256) void k_rsys_pairs(TermPool P, TermPool S, int ns, int64_t n, int d,
+                                                    const int* __restrict__ idx,
+                                                    const RsysStep* __restrict__ psteps,
+                                                    const RsysTerm* __restrict__ pterms,
+                                                    const RsysStep* __restrict__ ssteps,
+                                                    const RsysTerm* __restrict__ sterms,
+                                                    const double2* __restrict__ sshares, RsysArgs R, Cpdf2D C,
+                                                    double* __restrict__ mom, uint8_t* __restrict__ keep) {
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const int64_t q = CELLS ? idx[k] : k;
+    const int tp = (int)(q / ns), ts = (int)(q % ns);
+    double b2[2] = {0.0, 0.0};
+    for (int j = 0; j < d; j++) {
+        const double br = S.b[(int64_t)ts * d + j] - P.b[(int64_t)tp * d + j];
+        b2[0] += R.T[j] * br;
+        b2[1] += R.T[d + j] * br;
+    }
+    if constexpr (!CELLS) {
+        const RsysTerm a = pterms[tp], b = sterms[ts];
+        const cplx g = cmul(a.g, b.g);
+        // one sum over the primary's rows, then the secondary's: the covariance, a difference
+        // of far larger numbers, shows its rounding
+        double ty0 = a.ty0, ty1 = a.ty1;
+        const int ms = S.m[ts];
+        for (int j = 0; j < ms; j++) {
+            const double2 v = sshares[(int64_t)ts * S.MM + j];
+            ty0 += v.x;
+            ty1 += v.y;
+        }
         const cplx y0 = cmake(-ty0, b2[0]), y1 = cmake(-ty1, b2[1]);
         // component c of pair q at mom[c * npairs + q] (column-major: contiguous column sums)
-        const int64_t npq = (int64_t)np * ns;
         const cplx gy0 = cmul(g, y0), gy1 = cmul(g, y1);
         const cplx c00 = cmul(gy0, y0), c01 = cmul(gy0, y1), c10 = cmul(gy1, y0), c11 = cmul(gy1, y1);
         const double v[14] = {g.re,   g.im,   gy0.re, gy0.im, gy1.re, gy1.im, c00.re,
                               c00.im, c01.re, c01.im, c10.re, c10.im, c11.re, c11.im};
 #pragma unroll
-        for (int c = 0; c < 14; c++) mom[c * npq + q] = v[c];
+        for (int c = 0; c < 14; c++) mom[c * n + q] = v[c];
     }
-    int u = 0;
-    for (int r = 0; r < m; r++) {
-        if (!F[r]) continue;
-        cmap[r] = u;
-        csm[r] = 1;
-        fidx[r] = r;
-        double w = p2[r];
-        for (int j = r + 1; j < m; j++) {
-            if (!F[j]) continue;
-            const bool pos = (fabs(a2[2 * r] - a2[2 * j]) < kCoalignEps) && (fabs(a2[2 * r + 1] - a2[2 * j + 1]) < kCoalignEps);
-            if (pos) {
-                cmap[j] = u;
-                csm[j] = 1;
-                F[j] = false;
-                fidx[j] = r;
-                w += p2[j];
-                continue;
-            }
-            const bool neg = (fabs(a2[2 * r] + a2[2 * j]) < kCoalignEps) && (fabs(a2[2 * r + 1] + a2[2 * j + 1]) < kCoalignEps);
-            if (neg) {
-                cmap[j] = u;
-                csm[j] = -1;
-                F[j] = false;
-                fidx[j] = r;
-                w += p2[j];
-            }
-        }
-        p2[u] = w;  // u <= r: no later read of the merge touches index u
-        u++;
-    }
-    {
-        int k = 0;
-        for (int r = 0; r < m; r++)
-            if (fidx[r] == r) {  // k <= r
-                a2[2 * k] = a2[2 * r];
-                a2[2 * k + 1] = a2[2 * r + 1];
-                k++;
-            }
-    }
-    // cell data over a half turn; rowof[i] is the compacted row whose line lies at th[i]
-    int8_t rowof[2 * K];
-    for (int r = 0; r < u; r++) {
-        const double x0 = a2[2 * r], x1 = a2[2 * r + 1];
-        double px, py;
-        if (fabs(x0) < fabs(x1)) {
-            px = 1.0;
-            py = -x0 / x1;
-        } else {
-            px = -x1 / x0;
-            py = 1.0;
-        }
-        double t1 = atan2(py, px);
-        if (t1 < 0) t1 += kPi;
-        th[2 * r] = t1;
-        th[2 * r + 1] = t1 + kPi;
-        rowof[2 * r] = rowof[2 * r + 1] = (int8_t)r;
-    }
-    for (int a = 1; a < 2 * u; a++) {
-        const double v = th[a];
-        const int8_t rv = rowof[a];
-        int b = a - 1;
-        while (b >= 0 && th[b] > v) {
-            th[b + 1] = th[b];
-            rowof[b + 1] = rowof[b];
-            b--;
-        }
-        th[b + 1] = v;
-        rowof[b + 1] = rv;
-    }
-    // The key bits of the original rows as a function of the compacted rows' sides: a zero
-    // row's bit is fixed by bar_nu; row j on compacted row k = cmap[j] has its bit set when
-    // k's side is negative and csm[j] = 1, or positive and csm[j] = -1.  With every side
-    // positive the bits are enc_fix | enc_pos; turning row k negative flips the bits hit[k].
-    uint32_t hit[K];
-    for (int k = 0; k < u; k++) hit[k] = 0;
-    int enc_fix = 0, enc_pos = 0;
-    for (int j = 0; j < m; j++) {
-        if (cmap[j] == kZeroHpMarker) {
-            const bool pr = j < mp;
-            const double* ar = pr ? Ap + j * D : As + (j - mp) * D;
-            const double sg = pr ? -1.0 : 1.0;
-            double ip = 0.0;
-            for (int k = 0; k < D; k++) ip += (ar[k] * sg) * R.nu[k];
-            if (ip < 0) enc_fix |= 1 << j;
-        } else {
-            hit[cmap[j]] |= 1u << j;
-            if (csm[j] < 0) enc_pos |= 1 << j;
-        }
-    }
-    // sides at the first cell's midpoint, then one crossing per cell: cell c lies between
-    // th[c] and th[c + 1], so moving into it crosses the line at th[c] and flips its row.
-    // Rows closer in angle than the merge tolerance were merged, so every midpoint is far
-    // from every line compared with the rounding of its dot products, and the flips give
-    // the sides a dot product at each midpoint gives.
-    uint32_t negb = 0;
-    int encv = 0;
-    if (u > 0) {
-        const double t = (th[1] + th[0]) / 2.0;
-        const double ptx = cos(t), pty = sin(t);
-        for (int j = 0; j < u; j++)
-            if (!(a2[2 * j] * ptx + a2[2 * j + 1] * pty > 0)) {
-                negb |= 1u << j;
-                encv ^= (int)hit[j];
-            }
-    }
-    // the g-integral terms a_j p_j (the products the sums below take, formed once)
-    for (int j = 0; j < u; j++) {
-        a2[2 * j] *= p2[j];
-        a2[2 * j + 1] *= p2[j];
-    }
-    const int MM = C.MM;
-    const int64_t co = q * MM;
-    const int mpmask = (1 << mp) - 1;
-    double total = 0.0;
+    const RsysStep* pp = psteps + (int64_t)tp * (P.MM + 1);
+    const RsysStep* ps = ssteps + (int64_t)ts * (S.MM + 1);
+    RsysStep A = *pp, B = *ps;
+    const int64_t w0 = k * (C.MM + 1), c0 = k * C.MM;
+    double total = 0.0, g1 = 0.0, g2 = 0.0;
     bool keep_term = false;
-    double s_hi = 0.0, c_hi = 0.0;  // sin / cos of the previous cell's upper edge
-    // a crossing usually changes the key of one estimator's term only: the other
-    // term's g value is the previous cell's (same key, same table)
-    int key_p = -1, key_s = -1;
-    cplx gp = cmake(0, 0), gs = cmake(0, 0);
-    for (int c = 0; c < u; c++) {
-        if (c > 0) {
-            const int k = rowof[c];
-            negb ^= 1u << k;
-            encv ^= (int)hit[k];
+    int u = 0;
+    // takes cell u between the lower and the upper line, both terms' states being those in it
+    auto cell = [&](double s1, double c1, double s2, double c2) {
+        g1 = A.g1 + B.g1;
+        g2 = A.g2 + B.g2;
+        if constexpr (CELLS) {
+            const cplx g = cmul(cmake(A.gre, A.gim), cmake(B.gre, B.gim));
+            C.wall[w0 + u] = wall2d(s1, c1, s2, c2, g1, g2, g);
+            C.cell[c0 + u] = Cell2D{g1, g2, g};
+        } else {
+            // the approximation's bound on the cell's contribution
+            const double den1 = g1 * (g1 * c1 + g2 * s1);
+            const double den2 = g1 * (g1 * c2 + g2 * s2);
+            if (fabs(den1) < 1e-14 || fabs(den2) < 1e-14) keep_term = true;
+            const double gr = A.gabs * B.gabs;
+            total += fabs((gr * s2) / den2) + fabs((gr * s1) / den1);
         }
-        const int enc = enc_fix | (enc_pos ^ encv);
-        if ((enc & mpmask) != key_p) {
-            key_p = enc & mpmask;
-            gp = lookup_num(key_p, 1 << (mp - 1), mpmask, pk, pv, pn);
+        u++;
+    };
+    auto coaligned = [](double x0, double x1, double y0, double y1) {
+        return (fabs(x0 - y0) < kCoalignEps && fabs(x1 - y1) < kCoalignEps) ||
+               (fabs(x0 + y0) < kCoalignEps && fabs(x1 + y1) < kCoalignEps);
+    };
+    double fs = 0, fc = 1, fa0 = 0, fa1 = 0;  // the first line
+    double ls = 0, lc = 1, la0 = 0, la1 = 0;  // the line the open cell begins at
+    bool open = false;
+    bool fromA = A.th <= B.th;
+    while (fmin(A.th, B.th) < __builtin_inf()) {
+        const double s = fromA ? A.s : B.s, c = fromA ? A.c : B.c;
+        const double a0 = fromA ? A.a0 : B.a0, a1 = fromA ? A.a1 : B.a1;
+        if (open) {
+            cell(ls, lc, s, c);
+        } else {
+            fs = s;
+            fc = c;
+            fa0 = a0;
+            fa1 = a1;
         }
-        if ((enc >> mp) != key_s) {
-            key_s = enc >> mp;
-            gs = lookup_num(key_s, 1 << (ms - 1), (1 << ms) - 1, sk, sv_, sn_);
-        }
-        const cplx g = cmul(gp, gs);
-        double g1re = 0.0, g2re = 0.0;
-        for (int j = 0; j < u; j++) {
-            const double svd = ((negb >> j) & 1u) ? -1.0 : 1.0;
-            g1re -= a2[2 * j] * svd;
-            g2re -= a2[2 * j + 1] * svd;
-        }
-        // a cell's lower edge is the previous cell's upper edge: same argument, same value
-        const double s1 = c > 0 ? s_hi : sin(th[c]), c1 = c > 0 ? c_hi : cos(th[c]);
-        const double s2 = sin(th[c + 1]), c2 = cos(th[c + 1]);
-        s_hi = s2;
-        c_hi = c2;
-        C.wall[co + q + c] = wall2d(s1, c1, s2, c2, g1re, g2re, g);
-        C.cell[co + c] = Cell2D{g1re, g2re, g};
-        if (c == u - 1) {
-            const double r = g1re * c2 + g2re * s2;
-            C.wall[co + q + u] = Wall2D{c2, s2, r, r * r, 0.0, 0.0};
-        }
-        // the approximation's bound on the cell's contribution
-        const double den1 = g1re * (g1re * c1 + g2re * s1);
-        const double den2 = g1re * (g1re * c2 + g2re * s2);
-        if (fabs(den1) < 1e-14 || fabs(den2) < 1e-14) keep_term = true;
-        const double gr = hypot(g.re, g.im);
-        total += fabs((gr * s2) / den2) + fabs((gr * s1) / den1);
+        open = true;
+        ls = s;
+        lc = c;
+        la0 = a0;
+        la1 = a1;
+        // cross the line and those coaligned with it
+        double n0, n1, nt;
+        do {
+            const RsysStep N = *(fromA ? ++pp : ++ps);
+            if (fromA) A = N;
+            else B = N;
+            fromA = A.th <= B.th;
+            n0 = fromA ? A.a0 : B.a0;
+            n1 = fromA ? A.a1 : B.a1;
+            nt = fromA ? A.th : B.th;
+        } while (nt < __builtin_inf() && coaligned(n0, n1, la0, la1));
     }
-    C.mc[q] = u;
-    C.b2[2 * q] = b2[0];
-    C.b2[2 * q + 1] = b2[1];
-    total *= (2 * R.norm_fact);
-    keep[q] = (keep_term || !(fabs(total) < R.eps)) ? 1 : 0;
+    if (open) {
+        // the last cell ends at the first line's other half, or, where that is coaligned with
+        // the last line, has ended there
+        const bool ended = u > 0 && coaligned(la0, la1, fa0, fa1);
+        const double es = ended ? ls : -fs, ec = ended ? lc : -fc;
+        if (!ended) cell(ls, lc, es, ec);
+        if constexpr (CELLS) {
+            const double r = g1 * ec + g2 * es;
+            C.wall[w0 + u] = Wall2D{ec, es, r, r * r, 0.0, 0.0};
+        }
+    }
+    if constexpr (CELLS) {
+        C.mc[k] = u;
+        C.b2[2 * k] = b2[0];
+        C.b2[2 * k + 1] = b2[1];
+    } else {
+        total *= (2 * R.norm_fact);
+        keep[k] = (keep_term || !(fabs(total) < R.eps)) ? 1 : 0;
+    }
 }
 
 // Partial sums of the columns of a column-major n x cols array: block (b, c) adds the
