@@ -872,17 +872,12 @@ struct Engine {
         bury();
         GraveyardScope gs(&graveyard);
         in.reserve(1);
-        std::vector<double> A(MM * d, 0.0), pp(MM, 0.0);
-        memcpy(A.data(), A0.data(), d * d * sizeof(double));
-        memcpy(pp.data(), p0.data(), d * sizeof(double));
-        copy_sync(in.A.ptr, A.data(), MM * d * sizeof(double), hipMemcpyHostToDevice);
-        copy_sync(in.p.ptr, pp.data(), MM * sizeof(double), hipMemcpyHostToDevice);
-        copy_sync(in.b.ptr, b0.data(), d * sizeof(double), hipMemcpyHostToDevice);
-        int mm = d, zero = 0;
-        int64_t z64 = 0;
-        copy_sync(in.m.ptr, &mm, sizeof(int), hipMemcpyHostToDevice);
-        copy_sync(in.gp_n.ptr, &zero, sizeof(int), hipMemcpyHostToDevice);
-        copy_sync(in.gp_off.ptr, &z64, sizeof(int64_t), hipMemcpyHostToDevice);
+        FirstTerm f{};
+        std::copy(A0.begin(), A0.end(), f.A);
+        std::copy(p0.begin(), p0.end(), f.p);
+        std::copy(b0.begin(), b0.end(), f.b);
+        MCE_LAUNCH(k_first_term, dim3(1), dim3(64), 0, st, in.view(), d, f);
+        HIPCHK(hipStreamSynchronize(st));
         in_count.assign(sr, 0);
         in_count[d] = 1;
         Nt = 1;

@@ -308,6 +308,24 @@ __device__ __forceinline__ int block4_excl_scan(int v, int* total, int* wsum) {
     return before + x - v;
 }
 
+// ------------------------------------------------------------------ first term
+// The term a window starts from (setup_first_term, cauchy_term.hpp:772-785), by value with
+// the launch: one launch and one wait per reset, where a copy per field waited seven times.
+struct FirstTerm {
+    double A[kMaxD * kMaxD], p[kMaxD], b[kMaxD];
+};
+__global__ __launch_bounds__(64) void k_first_term(TermPool P, int d, FirstTerm f) {
+    const int t = threadIdx.x;
+    for (int i = t; i < P.MM * d; i += 64) P.A[i] = i < d * d ? f.A[i] : 0.0;
+    for (int i = t; i < P.MM; i += 64) P.p[i] = i < d ? f.p[i] : 0.0;
+    if (t < d) P.b[t] = f.b[t];
+    if (t == 0) {
+        P.m[0] = d;
+        P.gp_n[0] = 0;
+        P.gp_off[0] = 0;
+    }
+}
+
 // ------------------------------------------------------------------ time propagation
 // cauchy_term.hpp:435-531 (time_prop, normalize_hps, tp_coalign), with the B-table
 // mode decision of cauchy_estimator.hpp:678-708 (serial) / 1614-1637 (threaded).
@@ -3701,7 +3719,7 @@ __device__ inline double sgn_d(double x) { return (double)((x > 0) - (x < 0)); }
 // A pair's rows are its two terms' rows, so everything about a row is formed once per term
 // (k_rsys_terms), where one thread per pair formed all of it in private memory: u angles, 2 u
 // sines and cosines, a sort and u^2 sums and merge tests (u rows): 119 ms for two 5-state
-// estimators of two steps, 4.6 ms in the two passes below.  A row vanishes on a line through the origin, at angle th in [0, pi]; going
+// estimators of three steps, 4.6 ms in the two passes below.  A row vanishes on a line through the origin, at angle th in [0, pi]; going
 // round, its side flips there and nowhere else within half a turn.  So a term's lines in order,
 // with its Re gamma sums and g value before each, are all that the cells of a pair need: the
 // cells lie between the merged lines of both terms, sums add and g values multiply.
