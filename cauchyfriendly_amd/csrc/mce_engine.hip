@@ -735,7 +735,7 @@ struct Engine {
     // reduction
     DBuf<uint64_t> fkeys, fskeys;
     DBuf<uint32_t> fidx, fsidx;
-    DBuf<int> rootpos, memrank, big_comp, Fc, dboff, gbase_dev;
+    DBuf<int> rootpos, memrank, big_comp, Fc, ford, dboff, gbase_dev;
     DBuf<int64_t> gval, groff;
     std::vector<int> h_boff;
     // groups (all buckets of an update)
@@ -2106,6 +2106,65 @@ struct Engine {
         HIPCHK(hipGetLastError());
     }
 
+    // The reduction alone, of n terms given by the caller (shape ascending; b n x d, p and the
+    // flattened A's first entries n x MM): each term's root and its place among the root's
+    // members.  Works in the buffers of the next update's outputs.
+    void reduce_given(int n, const int* shape, const double* b, const double* p, const double* A, int* root,
+                      int* place) {
+        bind();
+        bury();
+        GraveyardScope gs(&graveyard);
+        std::vector<int> off(sr + 1, 0);
+        for (int i = 0; i < n; i++) {
+            if (shape[i] < 1 || shape[i] > MM || (i && shape[i] < shape[i - 1]))
+                throw std::runtime_error("shapes must ascend within 1.." + std::to_string(MM));
+            off[shape[i] + 1]++;
+        }
+        for (int m = 0; m < sr; m++) off[m + 1] += off[m];
+        StepConst sc{};
+        for (int i = 0; i < d; i++) {
+            sc.order[i] = g_search_order[i];
+            if (sc.order[i] < 0 || sc.order[i] >= d) throw std::runtime_error("search ordering outside the state");
+        }
+        bool nan_p = false;
+        std::vector<double> rows((size_t)n * MM * d, 0.0);
+        std::vector<uint32_t> slots(n);
+        for (int i = 0; i < n; i++) {
+            slots[i] = i;
+            for (int k = 0; k < shape[i]; k++) {
+                rows[(size_t)i * MM * d + k] = A[(size_t)i * MM + k];
+                nan_p |= std::isnan(p[(size_t)i * MM + k]);
+            }
+        }
+        out.reserve(n);
+        perm.reserve(n);
+        for (DBuf<int>* v : {&grp_root, &grp_moff, &grp_mcnt, &grp_m, &mem_slots}) v->reserve(n);
+        const int flag = nan_p;
+        upload(dconst.ptr, &sc, sizeof(sc));
+        fill_multi({{counters.ptr, 32 * sizeof(int), 0}});
+        copy_sync(counters.ptr + kCtrNanP, &flag, sizeof(int), hipMemcpyHostToDevice);
+        copy_sync(out.A.ptr, rows.data(), rows.size() * sizeof(double), hipMemcpyHostToDevice);
+        copy_sync(out.b.ptr, b, (size_t)n * d * sizeof(double), hipMemcpyHostToDevice);
+        copy_sync(out.p.ptr, p, (size_t)n * MM * sizeof(double), hipMemcpyHostToDevice);
+        copy_sync(perm.ptr, slots.data(), (size_t)n * sizeof(uint32_t), hipMemcpyHostToDevice);
+        std::vector<int> first;
+        const int ng = run_sync(reduce_all(out.view(), off, first));
+        std::vector<int> gr(ng), go(ng), gn(ng), mem(n);
+        copy_sync(gr.data(), grp_root.ptr, ng * sizeof(int), hipMemcpyDeviceToHost);
+        copy_sync(go.data(), grp_moff.ptr, ng * sizeof(int), hipMemcpyDeviceToHost);
+        copy_sync(gn.data(), grp_mcnt.ptr, ng * sizeof(int), hipMemcpyDeviceToHost);
+        copy_sync(mem.data(), mem_slots.ptr, n * sizeof(int), hipMemcpyDeviceToHost);
+        for (int i = 0; i < n; i++) root[i] = place[i] = -1;
+        for (int g = 0; g < ng; g++) {
+            root[gr[g]] = gr[g];
+            for (int k = 0; k < gn[g]; k++) {
+                const int s = mem[go[g] + k];
+                root[s] = gr[g];
+                place[s] = k;
+            }
+        }
+    }
+
     // Fast term reduction of every shape bucket at once.  off[m] is the first gathered
     // position of shape m; fills the reduction groups (shape ascending, roots ascending,
     // members ascending per root) and gbase_of[m], the first group of shape m.
@@ -2129,8 +2188,9 @@ struct Engine {
         gval.reserve(N);
         groff.reserve(N);
         gbase_dev.reserve(sr + 1);
-        big_comp.reserve(waves);  // at most one per wavefront
-        Fc.reserve((size_t)(chunked ? kFtrChunks : 1) * N);
+        big_comp.reserve(waves + sr);  // at most one per wavefront and one per shape
+        Fc.reserve((size_t)(chunked ? kFtrChunks : kFtrArrays) * N);
+        ford.reserve((size_t)kFtrOrders * N);
         const dim3 g1(ceil_div(std::max(N, sr + 1), 256)), b1(256);
         int* nbig = counters.ptr + kCtrBigComp;
         MCE_DISPATCH_D(d, MCE_RUN(k_ftr_keys<DD>, g1, b1, 0, st, OUT, perm.ptr, N, boff, sr, dconst.ptr,
@@ -2139,11 +2199,11 @@ struct Engine {
         MCE_DISPATCH_D(d, MCE_RUN(k_ftr_comp<DD>, dim3(ceil_div(waves, 4)), b1, 0, st, OUT, perm.ptr, N, boff,
                                   dconst.ptr, fskeys.ptr, fsidx.ptr, rootpos.ptr, memrank.ptr, gval.ptr, nbig,
                                   big_comp.ptr));
-        // a workgroup takes 8 listed components at a time, and at most one is listed per wavefront
+        // a workgroup takes 8 listed components at a time, and hardly more than one is listed per wavefront
         const int bigb = std::max(1, std::min(1024, waves / 16));
         MCE_DISPATCH_D(d, MCE_RUN(k_ftr_comp_big<DD>, dim3(bigb), dim3(kCompThreads), 0, st, OUT, perm.ptr, N,
                                   boff, dconst.ptr, fskeys.ptr, fsidx.ptr, rootpos.ptr, memrank.ptr, gval.ptr, nbig,
-                                  big_comp.ptr, Fc.ptr));
+                                  big_comp.ptr, Fc.ptr, ford.ptr));
         scan_i64_excl(gval.ptr, groff.ptr, N);
         MCE_RUN(k_ftr_emit, g1, b1, 0, st, N, boff, sr, perm.ptr, gval.ptr, groff.ptr, rootpos.ptr, memrank.ptr,
                 grp_root.ptr, grp_moff.ptr, grp_mcnt.ptr, grp_m.ptr, mem_slots.ptr, gbase_dev.ptr);
@@ -4051,6 +4111,25 @@ int mce_term(void* handle, int shape, int idx, int* info, double* A, double* p, 
         return -1;
     }
 }
+
+int mce_reduce_terms(void* handle, int n, const int* shape, const double* b, const double* p, const double* A,
+                     int* root, int* place) {
+    try {
+        if (n > 0) ((Handle*)handle)->eng->reduce_given(n, shape, b, p, A, root, place);
+        return 0;
+    } catch (const std::exception& ex) {
+        set_err("mce_reduce_terms", ex);
+        return -1;
+    }
+}
+
+unsigned long long mce_reduction_key(int d, int m, const double* b, const double* p, const double* A) {
+    int order[kMaxD];
+    for (int a = 0; a < kMaxD; a++) order[a] = a;
+    return ftr_key(b, p, A, d, m, order, true);
+}
+
+unsigned long long mce_reduction_link(int d, int m) { return ftr_link(d, m); }
 
 void mce_set_random_draws(void* handle, const double* root_point, const double* b_pert_8xmax) {
     Engine* e = ((Handle*)handle)->eng;

@@ -1724,12 +1724,13 @@ __device__ __forceinline__ void k_fill_multi(MG<1024, 1> mg, FillArgs f) {
 // sorted by one number that every compared quantity enters instead (k_ftr_keys): two terms
 // that reduce differ by at most a known bound in it, so every reduction stays inside a run of
 // sorted neighbours that are no further apart than that bound, a component.  Components are
-// almost always the reduction groups themselves.  The greedy pass then runs inside each
-// component, with the reference's own comparisons on the terms' values (ftr_edge), so
-// what reduces with what is unchanged: the sort only decides which pairs are compared.
+// the reduction groups themselves unless scales come near the tolerances.  The greedy pass then
+// runs inside each component, with the reference's own comparisons on the terms' values
+// (ftr_edge), so what reduces with what is unchanged: the sort only decides which pairs are
+// compared.
 //   k_ftr_keys      sort key of each term
 //   k_ftr_comp      components of up to one wavefront: greedy pass, chunk merge, member ranks
-//   k_ftr_comp_big  the others, one workgroup each
+//   k_ftr_comp_big  the others, a wavefront or a workgroup each
 //   k_ftr_emit      reduction groups and member lists, after a scan over the roots
 // 718k terms of a 2-state, 20-hyperplane window: the pair search, its edge lists and the
 // resolution rounds took 78 ms per window (3.3 ms per pair pass, 1.2 ms per edge pass).
@@ -1753,16 +1754,64 @@ __device__ inline int ftr_chunk_of(int l, int n) {
     return c > kFtrChunks - 1 ? kFtrChunks - 1 : c;
 }
 
-// Sort key: shape, then s = sum_k w_k f(x_k) over the d coordinates of b, the m scales p and
-// the first m entries of A in magnitude, in units of 2^-26.  f(x) = x / (1 + |x|) never moves
-// two numbers further apart than they were and w_k <= 1, so terms that reduce, each of whose
-// compared quantities differ by at most kReductionEps, differ by at most (d + 2m) 1e-8 in s.
-// |s| < 70 keeps the key in kFtrKeyBits bits.  The w_k are spread over [0.5, 1) so that terms
-// that only exchange values get different keys.
+// Sort key: shape, then the sum over the d coordinates of b, the m scales p and the first m
+// entries of A in magnitude of w_k x_k, each x_k in whole units of 2^-kFtrFracBits and each
+// w_k in whole 1024ths of [1/2, 1), in units of 2^-26 on a ring of 2^kFtrValueBits.  All of it is
+// integer arithmetic, so two keys are as far apart as their terms whatever the terms' magnitude:
+// states in metres are told apart as well as states of order one, where a key that squashes large
+// numbers together sees thousands of distinct terms as one component.  (A 2-state window of 8
+// steps whose scales were all 1e5: 9296 of 13842 terms in components of up to 4102 with the
+// squashed key, whose roots a workgroup takes one by one; 2373 in 3 here, as in units of one.)
+// The w_k are spread over [1/2, 1) so that terms that only exchange values get different keys.
 constexpr int kFtrValueBits = 34;
 constexpr int kFtrKeyBits = kFtrValueBits + 5;
-// A NaN in p compares as equal to anything (ftr_edge), which no finite key can express: when
-// the measurement update saw one, p is left out of every key.
+constexpr uint64_t kFtrValueMask = ((uint64_t)1 << kFtrValueBits) - 1;
+constexpr int kFtrFracBits = 32;
+constexpr int kFtrDropBits = kFtrFracBits + 10 - 26;  // from units of 2^-kFtrFracBits / 1024 to 2^-26
+__host__ __device__ constexpr uint32_t ftr_weight(int k) {  // k + 1 golden ratios, the 9 bits after the point
+    return 512u + (((uint32_t)(k + 1) * 0x9E3779B9u) >> 23);
+}
+// Compared quantities of terms that reduce differ by at most kReductionEps = 42.9 units, those
+// of b by at most 2^-26 = 64 units (b + kReductionEps is rounded, which adds up to half of b's last
+// place where that is below 2^-25, and nothing but b itself is inside the window of a larger b).
+// From 2^28 on they only reduce if they are equal, and any function of their bits will do.
+__host__ __device__ inline uint64_t ftr_units(double x) {
+    if (fabs(x) < (double)(1 << 28)) return (uint64_t)(int64_t)floor(x * (double)((uint64_t)1 << kFtrFracBits));
+    union {
+        double d;
+        uint64_t u;
+    } v = {x};
+    return v.u * 0x9E3779B97F4A7C15ull;
+}
+// A NaN in p compares as equal to anything (ftr_edge), which no key can express: when the
+// measurement update saw one, p is left out of every key.
+__host__ __device__ inline uint64_t ftr_key(const double* b, const double* p, const double* A, int d, int m,
+                                            const int* order, bool with_p) {
+    uint64_t v = 0;
+    for (int a = 0; a < d; a++) v += ftr_weight(a) * ftr_units(b[order[a]]);
+    for (int k = 0; k < m; k++) {
+        if (with_p) v += ftr_weight(d + 2 * k) * ftr_units(p[k]);
+        v += ftr_weight(d + 2 * k + 1) * ftr_units(fabs(A[k]));
+    }
+    return ((uint64_t)m << kFtrValueBits) | ((v >> kFtrDropBits) & kFtrValueMask);
+}
+// Largest distance of the keys of two terms of shape m that reduce.  n weights in a row add up to
+// at most 768 n + 512.
+__host__ __device__ constexpr uint64_t ftr_link(int d, int m) {
+    return (((768u * d + 512u) * 64u + (768u * 2u * m + 512u) * 43u) >> kFtrDropBits) + 1u;
+}
+constexpr bool ftr_weights_bounded() {
+    for (int i = 0; i <= kMaxD; i++) {
+        uint32_t sum = 0;
+        for (int n = 1; i + n <= kMaxD + 2 * kMaxM; n++) {
+            sum += ftr_weight(i + n - 1);
+            if (sum > 768u * n + 512u) return false;
+        }
+    }
+    return true;
+}
+static_assert(ftr_weights_bounded(), "ftr_link relies on it");
+
 template <int D>
 __device__ __forceinline__ void k_ftr_keys(MG<256, 1> mg, const TermPool OUT, const uint32_t* __restrict__ perm, int n,
                                            const int* __restrict__ boff, int nb, const StepConst* __restrict__ sc,
@@ -1770,40 +1819,34 @@ __device__ __forceinline__ void k_ftr_keys(MG<256, 1> mg, const TermPool OUT, co
                                            uint32_t* __restrict__ idx) {
     const int p = mg.bx * blockDim.x + threadIdx.x;
     if (p >= n) return;
-    const int m = bucket_of(boff, nb, p);
     const int64_t s = perm[p];
-    const double* b = OUT.b + s * D;
-    const double* pp = OUT.p + s * OUT.MM;
-    const double* A = OUT.A + s * OUT.MM * D;
-    auto weight = [](int k) {
-        const double t = (k + 1) * 0.6180339887498949;
-        return 0.5 + 0.5 * (t - floor(t));
-    };
-    auto squash = [](double x) {  // f(|x|); a NaN counts as infinite
-        const double u = fmin(fabs(x), 1e300);
-        return u / (1.0 + u);
-    };
-    double v = 128.0;
-#pragma unroll
-    for (int a = 0; a < D; a++) {
-        const double x = b[sc->order[a]];
-        v += weight(a) * copysign(squash(x), x);
-    }
-    const bool with_p = *nan_p == 0;
-    for (int k = 0; k < m; k++) {
-        if (with_p) v += weight(D + 2 * k) * copysign(squash(pp[k]), pp[k]);
-        v += weight(D + 2 * k + 1) * squash(A[k]);
-    }
-    keys[p] = ((uint64_t)m << kFtrValueBits) | (uint64_t)(v * (double)(1 << 26));
+    keys[p] = ftr_key(OUT.b + s * D, OUT.p + s * OUT.MM, OUT.A + s * OUT.MM * D, D, bucket_of(boff, nb, p), sc->order,
+                      *nan_p == 0);
     idx[p] = (uint32_t)p;
 }
 
-// Whether sorted neighbours belong to one component: same shape, and keys no further apart
-// than (d + 2m) 1e-8 in units of 2^-26, rounded up (two keys are floors of their values).
+__device__ __forceinline__ int ftr_shape(uint64_t key) { return (int)(key >> kFtrValueBits); }
+
+// Whether sorted neighbours belong to one component.
 template <int D>
 __device__ __forceinline__ bool ftr_linked(uint64_t prev, uint64_t cur) {
-    const int m = (int)(cur >> kFtrValueBits);
-    return (int)(prev >> kFtrValueBits) == m && cur - prev <= (uint64_t)((int)(0.672 * (D + 2 * m)) + 3);
+    const int m = ftr_shape(cur);
+    return ftr_shape(prev) == m && cur - prev <= ftr_link(D, m);
+}
+
+// Whether two keys of shape m are near enough for their terms to reduce.
+template <int D>
+__device__ __forceinline__ bool ftr_near(uint64_t a, uint64_t b, int m) {
+    const uint64_t x = (a - b) & kFtrValueMask;
+    return x <= ftr_link(D, m) || kFtrValueMask + 1 - x <= ftr_link(D, m);
+}
+
+// Whether the last and the first key of a shape are neighbours on the ring: the run at the
+// bucket's end goes on at its beginning.  (They are different runs: one around the whole ring
+// would need 2^kFtrValueBits / ftr_link terms of a shape, which no device holds.)
+template <int D>
+__device__ __forceinline__ bool ftr_joined(uint64_t first, uint64_t last) {
+    return ((first - last) & kFtrValueMask) <= ftr_link(D, ftr_shape(first)) && first != last;
 }
 
 // Whether term si (earlier) claims term sj (later) of shape m, term_reduction.hpp:89-276:
@@ -1849,8 +1892,9 @@ __device__ inline bool ftr_edge(const TermPool& O, int64_t si, int64_t sj, int m
 
 // Components that begin in the first kCompOwn of 64 sorted positions are reduced by the
 // wavefront that looks at these 64, a lane per term; the next wavefront begins kCompOwn
-// positions on.  A component that does not end inside the 64 goes to big_list (at most one
-// per wavefront).  No list of all components is made or counted.
+// positions on.  A component that does not end inside the 64, or that goes on at its bucket's
+// beginning, goes to big_list (at most one of the former per wavefront, one of the latter per
+// shape).  No list of all components is made or counted.
 //
 // Greedy pass: the least unclaimed term of a component is a root and claims every later
 // unclaimed term that ftr_edge accepts.  In a bucket above kFtrChunkTerms terms each chunk c
@@ -1860,31 +1904,42 @@ __device__ inline bool ftr_edge(const TermPool& O, int64_t si, int64_t sj, int m
 // merges never leave a component.
 constexpr int kCompOwn = 48;
 // Reduces the components that begin in the first `own` of the 64 sorted positions from `base`
-// (< n).  Returns the position of the one that does not end inside the 64, or -1.
+// (< n).  Returns the lanes at which those to be listed begin.
 template <int D>
-__device__ __forceinline__ int ftr_comp_wave(const TermPool& OUT, const uint32_t* __restrict__ perm, int n,
-                                             const int* __restrict__ boff, const StepConst* __restrict__ sc,
-                                             const uint64_t* __restrict__ skeys, const uint32_t* __restrict__ sidx,
-                                             int* __restrict__ rootpos, int* __restrict__ rank,
-                                             int64_t* __restrict__ gval, int base, int own_starts) {
+__device__ __forceinline__ uint64_t ftr_comp_wave(const TermPool& OUT, const uint32_t* __restrict__ perm, int n,
+                                                  const int* __restrict__ boff, const StepConst* __restrict__ sc,
+                                                  const uint64_t* __restrict__ skeys,
+                                                  const uint32_t* __restrict__ sidx, int* __restrict__ rootpos,
+                                                  int* __restrict__ rank, int64_t* __restrict__ gval, int base,
+                                                  int own_starts) {
     const int lane = wave_lane();
     const int r = base + lane;
     const bool in = r < n;
     const uint64_t q = in ? skeys[r] : 0;
-    const bool start = !(in && r > 0 && ftr_linked<D>(skeys[r - 1], q));  // past the end: a start
+    const uint64_t before = in && r > 0 ? skeys[r - 1] : 0;
+    const uint64_t beyond = base + kWave < n ? skeys[base + kWave] : 0;
+    const bool start = !(in && r > 0 && ftr_linked<D>(before, q));  // past the end: a start
     const uint64_t starts = __ballot(start);
     const uint64_t upto = starts & (~0ull >> (kWave - 1 - lane));
     const int sb = upto ? kWave - 1 - __clzll((long long)upto) : -1;
     const uint64_t after = lane == kWave - 1 ? 0ull : starts >> (lane + 1);
     const int se = after ? lane + __ffsll((unsigned long long)after) : kWave;
-    const bool ends = base + kWave >= n || !ftr_linked<D>(skeys[base + kWave - 1], skeys[base + kWave]);
+    const int m = ftr_shape(q);
+    // the first and the last term of a bucket (no shape is 0) whose ends are joined
+    const uint64_t down = __shfl_down(q, 1, kWave);
+    const bool head = in && ftr_shape(before) != m, tail = in && ftr_shape(lane == kWave - 1 ? beyond : down) != m;
+    const bool joined = (head || tail) && ftr_joined<D>(skeys[boff[m]], skeys[boff[m + 1] - 1]);
+    const uint64_t heads = __ballot(head && joined), tails = __ballot(tail && joined);
+    const bool ends = base + kWave >= n || !ftr_linked<D>(__shfl(q, kWave - 1, kWave), beyond);
     const bool own = in && sb >= 0 && sb < own_starts;
-    const bool mine = own && (se < kWave || ends);
-    const uint64_t open_start = __ballot(own && !mine && lane == sb);
+    const bool closed = se < kWave || ends;
+    const bool from_end = own && ((heads >> sb) & 1u), goes_on = own && ((tails >> (se - 1)) & 1u);
+    // a bucket's last run takes in its first one
+    const bool mine = own && closed && !from_end && !goes_on;
+    const uint64_t listed = __ballot(own && lane == sb && !from_end && (!closed || goes_on));
     const int size = mine ? se - sb : 1;
     const uint64_t seg = mine ? ((se == kWave ? ~0ull : (1ull << se) - 1ull) & ~((1ull << sb) - 1ull)) : 0ull;
     const int p = mine ? (int)sidx[r] : INT_MAX;
-    const int m = (int)(q >> kFtrValueBits);
     const int beg = mine ? boff[m] : 0, end = mine ? boff[m + 1] : 0;
     const int slot = mine ? (int)perm[p] : 0;
     const int last = mine ? se - 1 : lane;
@@ -1955,7 +2010,7 @@ __device__ __forceinline__ int ftr_comp_wave(const TermPool& OUT, const uint32_t
         rank[p] = less;
         gval[p] = ((int64_t)(f0 == lane) << 32) | (uint32_t)cnt;
     }
-    return open_start ? base + __ffsll((unsigned long long)open_start) - 1 : -1;
+    return listed;
 }
 
 template <int D>
@@ -1967,21 +2022,52 @@ __device__ __forceinline__ void k_ftr_comp(MG<256, 1> mg, const TermPool OUT, co
                                            int* __restrict__ big_list) {
     const int base = (mg.bx * (blockDim.x / kWave) + threadIdx.x / kWave) * kCompOwn;
     if (base >= n) return;
-    const int open = ftr_comp_wave<D>(OUT, perm, n, boff, sc, skeys, sidx, rootpos, rank, gval, base, kCompOwn);
-    if (open >= 0 && wave_lane() == 0) big_list[atomicAdd(big_count, 1)] = open;
+    const uint64_t listed =
+        ftr_comp_wave<D>(OUT, perm, n, boff, sc, skeys, sidx, rootpos, rank, gval, base, kCompOwn);
+    if ((listed >> wave_lane()) & 1u) big_list[atomicAdd(big_count, 1)] = base + wave_lane();
 }
 
+// LDS of one wavefront for a component of any size: up to kWave terms that may become roots
+// together (key, b on the first two search axes, slot, place in term order, which of them each
+// one claims; in the order of their keys, who they are and the entries with keys near theirs),
+// and a sort pass's digit counts.
+struct FtrLds {
+    uint64_t key[kWave], row[kWave];
+    double b0[kWave], b1[kWave];
+    int slot[kWave], idx[kWave];
+    int who[kWave], lo[kWave], hi[kWave];
+    int base[kWave], cnt[kWave];
+};
+
 // The component that begins at sorted position r0 and ends before r1, of any size, by T
-// threads: one wavefront, or (T > 64) a workgroup with T / 64 words of LDS in wred and wsum.
-// F: the flag arrays, indexed by sorted position.
+// threads: one wavefront, or (T > 64) a workgroup.  Positions beyond the bucket's end stand for
+// those from its beginning on (a component across the ring's zero).
+//
+// The terms are brought into term order.  Then the first kWave unclaimed ones are taken at a
+// time: which of them claims which follows from the pairs among them, and every later term looks
+// at those roots among them whose keys are near its own, with most of what tells them apart in
+// LDS.  The first time a single one is taken: a long window's largest components are one group.
+// At last a stable sort by root leaves each group's members together and in order.  Bound by the
+// latency of a pass's dependent loads and barriers, so a pass serves 64 roots.  Components whose
+// terms all differ are few, but where the scales come near the tolerances, or rounding at
+// large ones exceeds it, they hold thousands: with a pass and two barriers per root, and ranks by
+// comparing all pairs, a 2-state window of 8 steps with scales of 1e-5 took 125 ms (10.0 ms here),
+// with 1e6 66 ms (3.6 ms, most of it the key's), with 1 3.6 ms (3.6 ms).
+//
+// F: kFtrArrays arrays of n ints (8 where a bucket is reduced in chunks), O: kFtrOrders;
+// the component has its own positions in each.
+constexpr int kFtrArrays = 3;
+constexpr int kFtrOrders = 3;
 template <int D, int T>
 __device__ __forceinline__ void ftr_comp_many(const TermPool& OUT, const uint32_t* __restrict__ perm, int n,
                                               const int* __restrict__ boff, const StepConst* __restrict__ sc,
                                               const uint64_t* __restrict__ skeys, const uint32_t* __restrict__ sidx,
                                               int* __restrict__ rootpos, int* __restrict__ rank,
-                                              int64_t* __restrict__ gval, int* __restrict__ F, int r0, int r1,
-                                              unsigned long long* wred, int* wsum) {
+                                              int64_t* __restrict__ gval, int* F, int* O, int r0, int r1, FtrLds* lds,
+                                              int* wsum) {
+    constexpr int kWaves = T / kWave;
     const int lane = wave_lane(), t = T == kWave ? lane : (int)threadIdx.x, w = t / kWave;
+    FtrLds& L = lds[0];
     auto sync = [&]() {
         if constexpr (T == kWave) {
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
@@ -1989,17 +2075,6 @@ __device__ __forceinline__ void ftr_comp_many(const TermPool& OUT, const uint32_
         } else {
             __syncthreads();
         }
-    };
-    // the minimum over all threads; what they wrote to F before is visible afterwards
-    auto least = [&](unsigned long long v) {
-        for (int o = kWave / 2; o > 0; o >>= 1) v = min(v, (unsigned long long)__shfl_xor(v, o, kWave));
-        sync();
-        if constexpr (T > kWave) {
-            if (lane == 0) wred[w] = v;
-            __syncthreads();
-            for (int k = 0; k < T / kWave; k++) v = min(v, wred[k]);
-        }
-        return v;
     };
     // set flags before this thread's, and of all threads
     auto count = [&](bool flag, int* total) {
@@ -2010,7 +2085,7 @@ __device__ __forceinline__ void ftr_comp_many(const TermPool& OUT, const uint32_
             if (lane == 0) wsum[w] = all;
             __syncthreads();
             all = 0;
-            for (int k = 0; k < T / kWave; k++) {
+            for (int k = 0; k < kWaves; k++) {
                 x += k < w ? wsum[k] : 0;
                 all += wsum[k];
             }
@@ -2018,29 +2093,200 @@ __device__ __forceinline__ void ftr_comp_many(const TermPool& OUT, const uint32_
         *total = all;
         return x;
     };
-    const int m = (int)(skeys[r0] >> kFtrValueBits);
+    // the sum over all threads; what they wrote before is visible afterwards
+    auto sum = [&](int v) {
+        for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+        sync();
+        if constexpr (T > kWave) {
+            if (lane == 0) wsum[w] = v;
+            __syncthreads();
+            v = 0;
+            for (int k = 0; k < kWaves; k++) v += wsum[k];
+        }
+        return v;
+    };
+    const uint64_t key0 = skeys[r0];
+    const int m = ftr_shape(key0);
     const int beg = boff[m], end = boff[m + 1], nbk = end - beg;
-    const int nc = nbk > kFtrChunkTerms ? kFtrChunks : 1;
-    for (int c = 0; c < nc; c++)
-        for (int r = r0 + t; r < r1; r += T) F[(int64_t)c * n + r] = r;
+    const int nc = nbk > kFtrChunkTerms ? kFtrChunks : 1, per = nbk / kFtrChunks;
+    const int size = r1 - r0;
+    // entry e of the component, and of its stretch of an array
+    auto at = [&](int e) { return r0 + e < end ? r0 + e : r0 + e - nbk; };
+    auto dist = [&](int e) { return (skeys[at(e)] - key0) & kFtrValueMask; };  // ascending
+    // Stable sort of the entries of a by of(entry) < 2^bits, 6 bits a pass, through b; returns
+    // the one that holds the result.
+    auto sort = [&](int* a, int* b, int bits, auto of) {
+        for (int shift = 0; shift < bits; shift += 6) {
+            sync();
+            if (t < kWave) L.base[t] = 0;
+            sync();
+            for (int i = t; i < size; i += T) atomicAdd(&L.base[(of(a[at(i)]) >> shift) & 63], 1);
+            sync();
+            if (t < kWave) {
+                const int c = L.base[t];
+                L.base[t] = wave_incl_scan(c) - c;
+            }
+            for (int i0 = 0; i0 < size; i0 += T) {
+                const bool in = i0 + t < size;
+                const int e = in ? a[at(i0 + t)] : 0;
+                const int dg = in ? (of(e) >> shift) & 63 : 0;
+                uint64_t same = __ballot(in);
+                for (int k = 0; k < 6; k++) {
+                    const uint64_t set = __ballot((dg >> k) & 1);
+                    same &= (dg >> k) & 1 ? set : ~set;
+                }
+                const int before = __popcll(same & ((1ull << lane) - 1ull));
+                lds[w].cnt[lane] = 0;
+                sync();
+                if (in && before == 0) lds[w].cnt[dg] = __popcll(same);
+                sync();
+                if (in) {
+                    int o = L.base[dg] + before;
+                    for (int k = 0; k < w; k++) o += lds[k].cnt[dg];
+                    b[at(o)] = e;
+                }
+                sync();
+                if (t < kWave)
+                    for (int k = 0; k < kWaves; k++) L.base[t] += lds[k].cnt[t];
+                sync();
+            }
+            int* const was = a;
+            a = b;
+            b = was;
+        }
+        sync();
+        return a;
+    };
+    auto bits_of = [](int x) { return 32 - __clz(x); };
+
+    // P: the entries in term order, place: each one's place in it.  Equal keys are in order
+    // already, the sort was stable.
+    int* const place = O + 2 * (int64_t)n;
+    for (int e = t; e < size; e += T) O[at(e)] = e;
+    const bool in_order = r1 <= end && key0 == skeys[r1 - 1];
+    int* const P = in_order ? O : sort(O, O + n, bits_of(nbk - 1), [&](int e) { return (int)sidx[at(e)] - beg; });
+    sync();
+    for (int i = t; i < size; i += T) {
+        place[at(P[at(i)])] = i;
+        for (int c = 0; c < nc; c++) F[(int64_t)c * n + at(i)] = i;
+    }
+    auto term = [&](int i) { return (int)sidx[at(P[at(i)])]; };
+    // whether a term with x0 and x1 on the first search axes may be claimed by candidate i
+    const int a0 = sc->order[0], a1 = sc->order[D > 1 ? 1 : 0];
+    auto window = [&](int i, double x0, double x1) {
+        const double ep = kReductionEps, v0 = L.b0[i], v1 = L.b1[i];
+        return x0 > v0 - ep && x0 <= v0 + ep && x1 > v1 - ep && x1 <= v1 + ep;
+    };
+    sync();
+    if (t <= nc) {  // places of the chunks' first terms
+        int lo = t == nc ? size : 0, hi = t == 0 ? 0 : size;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (term(mid) - beg < t * per) lo = mid + 1;
+            else hi = mid;
+        }
+        L.base[t] = lo;
+    }
+    sync();
+    int roots = 0;  // with one chunk: of the component
     for (int c = 0; c < nc; c++) {
         int* Fc = F + (int64_t)c * n;
-        for (int last = -1;;) {
-            unsigned long long v = ~0ull;
-            for (int r = r0 + t; r < r1; r += T) {
-                const int p = (int)sidx[r];
-                if (p > last && Fc[r] == r && ftr_chunk_of(p - beg, nbk) == c)
-                    v = min(v, ((unsigned long long)p << 32) | (unsigned)r);
+        const int cb = L.base[c], ce = L.base[c + 1];
+        int left = ce - cb;  // neither roots nor claimed
+        int most = 1;
+        for (int next = cb; left > 0; most = kWave) {
+            // the first unclaimed terms, at most `most`
+            int k = 0;
+            for (; next < ce && k < most; next += T) {
+                const int i = next + t;
+                const bool un = i < ce && Fc[at(i)] == i;
+                int found;
+                const int x = k + count(un, &found);
+                if (un && x < most) {
+                    const int slot = (int)perm[term(i)];
+                    L.idx[x] = i;
+                    L.slot[x] = slot;
+                    L.key[x] = skeys[at(P[at(i)])];
+                    L.b0[x] = OUT.b[(int64_t)slot * D + a0];
+                    L.b1[x] = OUT.b[(int64_t)slot * D + a1];
+                }
+                k += found;
             }
-            v = least(v);
-            if (v == ~0ull) break;
-            const int rr = (int)(v & 0xffffffffu);
-            last = (int)(v >> 32);
-            const int64_t rs = perm[last];
-            for (int r = r0 + t; r < r1; r += T) {
-                const int p = (int)sidx[r];
-                if (p > last && Fc[r] == r && ftr_edge<D>(OUT, rs, perm[p], m, sc, perm, beg, end)) Fc[r] = rr;
+            k = min(k, most);
+            sync();
+            next = L.idx[k - 1] + 1;
+            // the entries near each, and which of them claims which later one
+            if (t < k) {
+                const uint64_t d = (L.key[t] - key0) & kFtrValueMask, link = ftr_link(D, m);
+                int place_of = 0;
+                for (int i = 0; i < k; i++) {
+                    const uint64_t di = (L.key[i] - key0) & kFtrValueMask;
+                    place_of += di < d || (di == d && i < t);
+                }
+                int lo = 0, hi = most == 1 ? 0 : size;
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (dist(mid) + link < d) lo = mid + 1;
+                    else hi = mid;
+                }
+                L.who[place_of] = t;
+                L.lo[place_of] = lo;
+                hi = size;
+                while (lo < hi && most > 1) {
+                    const int mid = (lo + hi) >> 1;
+                    if (dist(mid) <= d + link) lo = mid + 1;
+                    else hi = mid;
+                }
+                L.hi[place_of] = hi;
             }
+            for (int i = w; i < k; i += kWaves) {
+                const bool e = lane > i && lane < k && window(i, L.b0[lane], L.b1[lane]) &&
+                               ftr_near<D>(L.key[i], L.key[lane], m) &&
+                               ftr_edge<D>(OUT, L.slot[i], L.slot[lane], m, sc, perm, beg, end);
+                const uint64_t row = __ballot(e);
+                if (lane == 0) L.row[i] = row;
+            }
+            sync();
+            uint64_t is_root = 0, claimed = 0;
+            for (int i = 0; i < k; i++) {
+                if ((claimed >> i) & 1u) continue;
+                is_root |= 1ull << i;
+                claimed |= L.row[i];
+            }
+            // the earliest root that has an edge to a term claims it; those near entry e are
+            // the ones from the first that ends beyond it to the last that begins at or before it
+            auto beyond = [&](const int* ends, int e) {
+                int lo = 0, hi = k;
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (ends[mid] <= e) lo = mid + 1;
+                    else hi = mid;
+                }
+                return lo;
+            };
+            int fewer = 0;
+            for (int e = t; e < size; e += T) {
+                const int j = place[at(e)];
+                if (j <= L.idx[0] || Fc[at(j)] != j) continue;
+                int s = beyond(L.hi, e);
+                const int send = beyond(L.lo, e);
+                if (s >= send) continue;
+                const int64_t slot = perm[sidx[at(e)]];
+                const double x0 = OUT.b[slot * D + a0], x1 = OUT.b[slot * D + a1];
+                int f = j;
+                for (; s < send; s++) {
+                    const int i = L.who[s];
+                    if (((is_root >> i) & 1u) && L.idx[i] < f && window(i, x0, x1) &&
+                        ftr_edge<D>(OUT, L.slot[i], slot, m, sc, perm, beg, end))
+                        f = L.idx[i];
+                }
+                if (f < j) {
+                    Fc[at(j)] = f;
+                    fewer += j < ce;
+                }
+            }
+            left -= sum(fewer) + __popcll(is_root);
+            roots += __popcll(is_root);
         }
     }
     for (int lvl = 0; nc > 1 && lvl < 3; lvl++) {
@@ -2049,108 +2295,92 @@ __device__ __forceinline__ void ftr_comp_many(const TermPool& OUT, const uint32_
             const int rt = k << (lvl + 1), cm = rt + (1 << lvl);
             int* F1 = F + (int64_t)rt * n;
             const int* F2 = F + (int64_t)cm * n;
-            for (int r = r0 + t; r < r1; r += T) {
-                if ((int)sidx[r] - beg < cm * (nbk / kFtrChunks)) continue;
-                const int f2 = F2[r];
-                if (f2 != r && F1[r] == r) F1[r] = F1[f2] == f2 ? f2 : F1[f2];
+            for (int i = t; i < size; i += T) {
+                if (term(i) - beg < cm * per) continue;
+                const int f2 = F2[at(i)];
+                if (f2 != i && F1[at(i)] == i) F1[at(i)] = F1[at(f2)] == f2 ? f2 : F1[at(f2)];
             }
         }
+    }
+    if (nc > 1) {
+        sync();
+        roots = 0;
+        for (int i = t; i < size; i += T) roots += F[at(i)] == i;
+        roots = sum(roots);
+    }
+    if (roots == 1) {
+        const int pf = term(0);
+        for (int i = t; i < size; i += T) {
+            const int p = term(i);
+            rootpos[p] = pf;
+            rank[p] = max(i - 1, 0);
+            gval[p] = i == 0 ? ((int64_t)1 << 32) | (uint32_t)(size - 1) : 0;
+        }
+        sync();
+        return;
+    }
+    // groups: a root and its members, all later than it, in order
+    int* Q = P == O ? O + n : O;
+    int* const G = F + 2 * (int64_t)n;  // where each root's group begins
+    for (int i = t; i < size; i += T) Q[at(i)] = i;
+    Q = sort(Q, F + n, bits_of(size - 1), [&](int i) { return F[at(i)]; });
+    sync();
+    for (int x = t; x < size; x += T)
+        if (F[at(Q[at(x)])] == Q[at(x)]) G[at(Q[at(x)])] = x;
+    sync();
+    for (int x = t; x < size; x += T) {
+        const int i = Q[at(x)], f = F[at(i)], g = G[at(f)];
+        const int p = term(i), pf = term(f);
+        rootpos[p] = pf;
+        rank[p] = i == f ? 0 : x - g - 1;
+        if (i != f) gval[p] = 0;
+        if (x + 1 == size || F[at(Q[at(x + 1)])] != f) gval[pf] = ((int64_t)1 << 32) | (uint32_t)(x - g);
     }
     sync();
-    // members of each root and their ranks.  In term order (equal keys: the sort is stable):
-    // one prefix count per root, unless roots are many; else every pair of terms is compared.
-    const bool in_order = skeys[r0] == skeys[r1 - 1];
-    const int most = (r1 - r0) / kWave;
-    bool done = false;
-    for (int last = -1, k = 0; in_order && k <= most; k++) {
-        unsigned long long v = ~0ull;
-        for (int r = r0 + t; r < r1; r += T)
-            if (F[r] == r && r > last) {
-                v = (unsigned long long)r;
-                break;
-            }
-        v = least(v);
-        done = v == ~0ull;
-        if (done) break;
-        last = (int)v;
-        int before = 0;
-        for (int b = r0; b < r1; b += T) {
-            const int r = b + t;
-            const bool mem = r < r1 && r != last && F[r] == last;
-            int tot;
-            const int x = count(mem, &tot);
-            if (mem) {
-                const int p = (int)sidx[r];
-                rootpos[p] = (int)sidx[last];
-                rank[p] = before + x;
-                gval[p] = 0;
-            }
-            before += tot;
-        }
-        if (t == 0) {
-            const int p = (int)sidx[last];
-            rootpos[p] = p;
-            rank[p] = 0;
-            gval[p] = ((int64_t)1 << 32) | (uint32_t)before;
-        }
-    }
-    if (done) return;
-    for (int b = r0 + w * kWave; b < r1; b += T) {
-        const int r = b + lane;
-        const int f0 = r < r1 ? F[r] : -1, p = r < r1 ? (int)sidx[r] : 0;
-        int cnt = 0, less = 0;
-        for (int q0 = r0; q0 < r1; q0 += kWave) {
-            const int nq = min(kWave, r1 - q0);
-            const int fq = lane < nq ? F[q0 + lane] : -1, pq = lane < nq ? (int)sidx[q0 + lane] : 0;
-            for (int k = 0; k < nq; k++) {
-                const int fk = __shfl(fq, k, kWave), pk = __shfl(pq, k, kWave);
-                const int q = q0 + k;
-                cnt += fk == r && q != r;
-                less += fk == f0 && q != f0 && pk < p;
-            }
-        }
-        if (r < r1) {
-            rootpos[p] = (int)sidx[f0];
-            rank[p] = less;
-            gval[p] = ((int64_t)(f0 == r) << 32) | (uint32_t)cnt;
-        }
-    }
 }
 
 // The listed components.  Most only straddled the end of their wavefront's positions: a
 // wavefront takes each and reduces it as above from its own first position.  Up to
 // kCompWave terms it goes through them 64 at a time; a workgroup takes what is larger.
 // Long windows of few states have components of thousands of terms that all reduce into one
-// (16269 in a 10-step window of 2 states).  The F arrays (8 of n ints when a bucket is reduced
-// in chunks, else one) belong to these components alone.
+// (16269 in a 10-step window of 2 states).  The arrays F and O belong to these components alone.
 constexpr int kCompWave = 1024;
 constexpr int kCompThreads = 512;
 template <int D>
 __device__ __forceinline__ void k_ftr_comp_big(MG<kCompThreads, 1> mg, const TermPool OUT,
                                                const uint32_t* __restrict__ perm, int n, const int* __restrict__ boff,
                                                const StepConst* __restrict__ sc, const uint64_t* __restrict__ skeys,
-                                               const uint32_t* __restrict__ sidx, int* __restrict__ rootpos,
-                                               int* __restrict__ rank, int64_t* __restrict__ gval,
-                                               const int* __restrict__ big_count, const int* __restrict__ big_list,
-                                               int* __restrict__ F) {
+                                               const uint32_t* __restrict__ sidx,
+                                               int* __restrict__ rootpos, int* __restrict__ rank,
+                                               int64_t* __restrict__ gval, const int* __restrict__ big_count,
+                                               const int* __restrict__ big_list, int* F, int* O) {
     constexpr int kWaves = kCompThreads / kWave;
-    __shared__ unsigned long long wred[kWaves];
     __shared__ int wsum[kWaves];
     __shared__ int2 large[kWaves];
+    __shared__ FtrLds lds[kWaves];
     const int lane = wave_lane(), w = threadIdx.x / kWave;
     const int count = *big_count;
     for (int e0 = mg.bx * kWaves; e0 < count; e0 += mg.gx * kWaves) {
         int r0 = -1, r1 = -1;
-        if (e0 + w < count)
-            r0 = ftr_comp_wave<D>(OUT, perm, n, boff, sc, skeys, sidx, rootpos, rank, gval, big_list[e0 + w], 1);
+        if (e0 + w < count && (ftr_comp_wave<D>(OUT, perm, n, boff, sc, skeys, sidx, rootpos, rank, gval,
+                                                big_list[e0 + w], 1) & 1u))
+            r0 = big_list[e0 + w];
         if (r0 >= 0) {
-            for (int b = r0 + 1; r1 < 0; b += kWave) {  // ends: positions past n stop it
-                const int r = b + lane;
-                const uint64_t stop = __ballot(r >= n || !ftr_linked<D>(skeys[r - 1], skeys[r]));
-                if (stop) r1 = min(n, b + __ffsll((unsigned long long)stop) - 1);
-            }
+            auto run_end = [&](int b) {  // positions past n stop it
+                for (;; b += kWave) {
+                    const int r = b + lane;
+                    const uint64_t stop = __ballot(r >= n || !ftr_linked<D>(skeys[r - 1], skeys[r]));
+                    if (stop) return min(n, b + __ffsll((unsigned long long)stop) - 1);
+                }
+            };
+            r1 = run_end(r0 + 1);
+            const int m = ftr_shape(skeys[r0]);
+            const int beg = boff[m];
+            if (r1 == boff[m + 1] && ftr_joined<D>(skeys[beg], skeys[r1 - 1])) r1 += run_end(beg + 1) - beg;
+        }
+        if (r0 >= 0) {
             if (r1 - r0 <= kCompWave) {
-                ftr_comp_many<D, kWave>(OUT, perm, n, boff, sc, skeys, sidx, rootpos, rank, gval, F, r0, r1, nullptr,
+                ftr_comp_many<D, kWave>(OUT, perm, n, boff, sc, skeys, sidx, rootpos, rank, gval, F, O, r0, r1, lds + w,
                                         nullptr);
                 r0 = -1;
             }
@@ -2160,8 +2390,8 @@ __device__ __forceinline__ void k_ftr_comp_big(MG<kCompThreads, 1> mg, const Ter
         __syncthreads();
         for (int e = 0; e < kWaves; e++)
             if (large[e].x >= 0)
-                ftr_comp_many<D, kCompThreads>(OUT, perm, n, boff, sc, skeys, sidx, rootpos, rank, gval, F, large[e].x,
-                                               large[e].y, wred, wsum);
+                ftr_comp_many<D, kCompThreads>(OUT, perm, n, boff, sc, skeys, sidx, rootpos, rank, gval, F, O,
+                                               large[e].x, large[e].y, lds, wsum);
     }
 }
 

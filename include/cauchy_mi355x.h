@@ -372,6 +372,19 @@ long long mce_terms_generated(void* handle);
 int mce_term(void* handle, int shape, int idx, int* info, double* A, double* p, double* b, unsigned int* keys,
              double* gvals);
 
+/* Term reduction alone, of n terms given by the caller: shape[n] (1 .. the estimator's largest,
+ * ascending), b (n x d), p and the first entries of each term's flattened A (both n x largest
+ * shape).  root[i] receives the term that term i reduces into (itself if it stays), place[i] its
+ * place among that root's members (-1 for a root).  Between updates only; the estimator's terms
+ * are left alone.  Returns 0, or -1 (message in mce_last_error). */
+int mce_reduce_terms(void* handle, int n, const int* shape, const double* b, const double* p, const double* A,
+                     int* root, int* place);
+
+/* Host code: the key by which the reduction of a term of shape m (1 .. 20) sorts, states in their
+ * own order, and the largest distance, modulo 2^34, of the keys of two such terms that reduce. */
+unsigned long long mce_reduction_key(int d, int m, const double* b, const double* p, const double* A);
+unsigned long long mce_reduction_link(int d, int m);
+
 /* Replaces the construction-time random draws: root point (d) and the 8 x max_shape
  * perturbation vectors of the cell enumerator. */
 void mce_set_random_draws(void* handle, const double* root_point, const double* b_pert_8xmax);

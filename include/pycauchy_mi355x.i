@@ -81,6 +81,9 @@ import_array();
 %ignore pycauchy_batch_single_step_ltiv;
 %ignore pycauchy_batch_single_step_ltiv_merged;
 %ignore pycauchy_batch_single_step_nonlin;
+%ignore mce_reduce_terms;
+%ignore mce_reduction_key;
+%ignore mce_reduction_link;
 %ignore mce_estimator_create;
 %ignore mce_estimator_step;
 %ignore mce_estimator_moments;

@@ -1607,6 +1607,20 @@ int oracle_term(void* h, int shape, int idx, int* info, double* A, double* p, do
     return 0;
 }
 
+// The reduction alone, of n terms of shape m (b n x d, p and the flattened A's first m entries
+// n x m): F[i] is the term that term i reduces into, or i.
+void oracle_reduce(int n, int d, int m, const double* b, const double* p, const double* A, int* F) {
+    std::vector<Term> T(n);
+    for (int i = 0; i < n; i++) {
+        T[i].m = m;
+        T[i].b.assign(b + (size_t)i * d, b + (size_t)(i + 1) * d);
+        T[i].p.assign(p + (size_t)i * m, p + (size_t)(i + 1) * m);
+        T[i].A.assign(A + (size_t)i * m, A + (size_t)(i + 1) * m);
+    }
+    const std::vector<int> f = fast_term_reduction(T, d, m);
+    std::copy(f.begin(), f.end(), F);
+}
+
 int oracle_set_tr_search_idxs_ordering(const int* ordering, int n) {
     if (n > 12) return 1;
     for (int i = 0; i < n; i++) g_search_order[i] = ordering[i];
