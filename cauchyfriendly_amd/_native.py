@@ -141,6 +141,8 @@ def lib():
     L.mce_last_update.restype = ct.c_int
     L.mce_last_update.argtypes = [ct.c_void_p, _dp, _ip]
     L.mce_shape_range.restype = ct.c_int
+    L.mce_trim_device_memory.restype = ct.c_longlong
+    L.mce_trim_device_memory.argtypes = []
     L.mce_terms_generated.restype = ct.c_longlong
     L.mce_terms_generated.argtypes = [ct.c_void_p]
     L.mce_shape_range.argtypes = [ct.c_void_p]

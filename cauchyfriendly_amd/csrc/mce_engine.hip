@@ -244,15 +244,17 @@ inline BatchSlot* bslot() { return nullptr; }
 // bytes are carved from slabs of several hundred blocks and stay with the process.  Larger
 // blocks (sizes in eighths of a power of two, so at most an eighth over what was asked) are
 // kept by size, and a request takes the smallest that holds it and is at most a quarter
-// larger.  Unslabbed blocks are freed when the cache would hold more than kMaxCached, or less
-// than a quarter of the device's memory is free (other processes and allocators share it);
-// large ones also once they lay unused for kIdle while others came and went, and all of them
-// when an allocation fails.
+// larger.  Blocks between the two sizes are freed beyond kMaxMid of them, large ones beyond
+// kMaxCached of both and while less than a quarter of the device's memory is free (other
+// processes and allocators share it), and once they lay unused for kIdle: every block that is
+// taken or given back, of any size, frees those that did.  A process that makes no more calls
+// keeps what it has until it asks for it (trim).  All of them are freed when an allocation fails.
 class BlockCache {
    public:
     static constexpr size_t kMinBlock = 256;
     static constexpr size_t kSlabMax = size_t(4) << 20;
     static constexpr size_t kMaxBlock = size_t(256) << 20;
+    static constexpr size_t kMaxMid = size_t(16) << 30;
     static constexpr size_t kMaxCached = size_t(48) << 30;
     static constexpr std::chrono::seconds kIdle{10};
 
@@ -272,17 +274,24 @@ class BlockCache {
     // `bytes` is a block_size() value, and on return the size of the block.
     void* get(size_t& bytes) {
         {
+            Gone gone;  // freed before anything is allocated
             std::lock_guard<std::mutex> lk(mu_);
+            void* p = nullptr;
             if (bytes > kMaxBlock) {
                 const auto it = large_.lower_bound(bytes);
                 if (it != large_.end() && it->first <= bytes + bytes / 4) {
-                    void* p = it->second.p;
+                    p = it->second.p;
                     bytes = it->first;
-                    cached_ -= bytes;
+                    large_bytes_ -= bytes;
                     large_.erase(it);
-                    return p;
                 }
-            } else {
+            }
+            sweep(gone);
+            if (p) return p;
+        }
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            if (bytes <= kMaxBlock) {
                 auto& l = free_[cls(bytes)];
                 if (l.empty() && bytes <= kSlabMax) {
                     const size_t sb = slab_size(bytes);
@@ -293,7 +302,7 @@ class BlockCache {
                 if (!l.empty()) {
                     void* p = l.back();
                     l.pop_back();
-                    if (bytes > kSlabMax) cached_ -= bytes;
+                    if (bytes > kSlabMax) mid_bytes_ -= bytes;
                     return p;
                 }
             }
@@ -303,37 +312,31 @@ class BlockCache {
     // The caller guarantees that no queued work reads or writes the block.
     void put(void* p, size_t bytes) {
         if (!p) return;
-        std::vector<void*> gone;
-        {
-            size_t avail = 0, total = 0;
-            const bool room = bytes <= kMaxBlock || (hipMemGetInfo(&avail, &total) == hipSuccess && avail >= total / 4);
-            std::lock_guard<std::mutex> lk(mu_);
-            if (bytes <= kSlabMax) {
-                free_[cls(bytes)].push_back(p);
-                return;
-            }
-            const auto now = std::chrono::steady_clock::now();
-            if (bytes > kMaxBlock)
-                for (auto it = large_.begin(); it != large_.end();) {
-                    if (now - it->second.since < kIdle) {
-                        ++it;
-                        continue;
-                    }
-                    gone.push_back(it->second.p);
-                    cached_ -= it->first;
-                    it = large_.erase(it);
-                }
-            if (!room || cached_ + bytes > kMaxCached) {
-                gone.push_back(p);
+        Gone gone;
+        size_t avail = 0, total = 0;
+        const bool room = bytes <= kMaxBlock || (hipMemGetInfo(&avail, &total) == hipSuccess && avail >= total / 4);
+        std::lock_guard<std::mutex> lk(mu_);
+        sweep(gone);
+        if (bytes <= kSlabMax) {
+            free_[cls(bytes)].push_back(p);
+        } else if (bytes <= kMaxBlock) {
+            if (mid_bytes_ + bytes > kMaxMid) {
+                gone.blocks.push_back(p);
             } else {
-                if (bytes > kMaxBlock)
-                    large_.emplace(bytes, Idle{p, now});
-                else
-                    free_[cls(bytes)].push_back(p);
-                cached_ += bytes;
+                free_[cls(bytes)].push_back(p);
+                mid_bytes_ += bytes;
             }
+        } else if (!room || mid_bytes_ + large_bytes_ + bytes > kMaxCached) {
+            gone.blocks.push_back(p);
+        } else {
+            large_.emplace(bytes, Idle{p, std::chrono::steady_clock::now()});
+            large_bytes_ += bytes;
         }
-        for (void* g : gone) (void)hipFree(g);
+    }
+    // Frees every cached block that was allocated by itself; returns their bytes.
+    size_t trim() {
+        std::lock_guard<std::mutex> lk(mu_);
+        return trim_unslabbed();
     }
 
    private:
@@ -341,6 +344,27 @@ class BlockCache {
         void* p;
         std::chrono::steady_clock::time_point since;
     };
+    // Blocks to free once the lock is gone: hipFree waits for the device.
+    struct Gone {
+        std::vector<void*> blocks;
+        ~Gone() {
+            for (void* p : blocks) (void)hipFree(p);
+        }
+    };
+    // Takes out the large blocks that lay unused for kIdle.  Needs mu_.
+    void sweep(Gone& gone) {
+        if (large_.empty()) return;
+        const auto now = std::chrono::steady_clock::now();
+        for (auto it = large_.begin(); it != large_.end();) {
+            if (now - it->second.since < kIdle) {
+                ++it;
+                continue;
+            }
+            gone.blocks.push_back(it->second.p);
+            large_bytes_ -= it->first;
+            it = large_.erase(it);
+        }
+    }
     // `locked`: the caller holds mu_.
     void* raw_alloc(size_t bytes, bool locked) {
         void* p = nullptr;
@@ -362,20 +386,22 @@ class BlockCache {
     }
     // Frees the cached blocks that were allocated one by one (hipFree synchronises the
     // device); the lists it empties belong to classes above kSlabMax.  Needs mu_.
-    void trim_unslabbed() {
+    size_t trim_unslabbed() {
         for (int c = cls(kSlabMax) + 1; c < 64; c++) {
             for (void* p : free_[c]) (void)hipFree(p);
             free_[c].clear();
         }
         for (auto& [size, b] : large_) (void)hipFree(b.p);
         large_.clear();
-        cached_ = 0;
+        const size_t freed = mid_bytes_ + large_bytes_;
+        mid_bytes_ = large_bytes_ = 0;
+        return freed;
     }
     static int cls(size_t bytes) { return __builtin_ctzll(bytes); }
     std::mutex mu_;
     std::vector<void*> free_[64];
     std::multimap<size_t, Idle> large_;
-    size_t cached_ = 0, slab_bytes_ = 0;
+    size_t mid_bytes_ = 0, large_bytes_ = 0, slab_bytes_ = 0;
 };
 
 BlockCache& block_cache() {
@@ -4111,6 +4137,8 @@ int mce_term(void* handle, int shape, int idx, int* info, double* A, double* p, 
         return -1;
     }
 }
+
+long long mce_trim_device_memory(void) { return (long long)block_cache().trim(); }
 
 int mce_reduce_terms(void* handle, int n, const int* shape, const double* b, const double* p, const double* A,
                      int* root, int* place) {

@@ -154,6 +154,12 @@ class GpuEstimator:
         _native.lib().mce_estimator_reset(self.h)
 
 
+def trim_device_memory():
+    """Frees the device memory that closed estimators gave back and that is kept for the next
+    ones, for other allocators in the process; returns the bytes."""
+    return int(_native.lib().mce_trim_device_memory())
+
+
 def run_system(sysobj, num_steps=None, seed=None, collect_terms=False):
     """Runs one GPU estimator over a System's measurement record (num_steps time steps)."""
     steps = sysobj.num_steps if num_steps is None else num_steps

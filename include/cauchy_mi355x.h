@@ -372,6 +372,11 @@ long long mce_terms_generated(void* handle);
 int mce_term(void* handle, int shape, int idx, int* info, double* A, double* p, double* b, unsigned int* keys,
              double* gvals);
 
+/* Frees the device memory that estimators gave back and that is kept for the next ones (all but
+ * the slabs of small blocks); returns the bytes.  For hosts that share the device with another
+ * allocator.  Live estimators are left alone. */
+long long mce_trim_device_memory(void);
+
 /* Term reduction alone, of n terms given by the caller: shape[n] (1 .. the estimator's largest,
  * ascending), b (n x d), p and the first entries of each term's flattened A (both n x largest
  * shape).  root[i] receives the term that term i reduces into (itself if it stays), place[i] its

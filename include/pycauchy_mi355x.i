@@ -81,6 +81,7 @@ import_array();
 %ignore pycauchy_batch_single_step_ltiv;
 %ignore pycauchy_batch_single_step_ltiv_merged;
 %ignore pycauchy_batch_single_step_nonlin;
+%ignore mce_trim_device_memory;
 %ignore mce_reduce_terms;
 %ignore mce_reduction_key;
 %ignore mce_reduction_link;
