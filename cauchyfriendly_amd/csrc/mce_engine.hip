@@ -2603,10 +2603,12 @@ static int64_t rsys_2d(Engine& P, Engine& S, const double* Trel, double eps, dou
     P.c2_err.reserve(1);
     Cpdf2D C{CM, nullptr, nullptr, nullptr, nullptr};
     TermPool PI = P.in.view(), SI = S.in.view();
-    auto pairs = [&](auto kernel, int64_t n, const int* idx) {
+    auto pairs = [&](auto kernel, auto near_kernel, int64_t n, const int* idx) {
         MCE_LAUNCH(kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, PI, SI, ns, n, d, idx, P.rs_steps.ptr,
                    P.rs_terms.ptr, P.rs_steps.ptr + (size_t)np * (P.MM + 1), P.rs_terms.ptr + np, P.rs_shares.ptr, R, C,
                    P.rs_mom.ptr, P.rs_keep.ptr);
+        MCE_LAUNCH(near_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 2048)), dim3(256), 0, st, PI, SI, ns, n, d, idx,
+                   P.gk[P.gcur].ptr, P.gv[P.gcur].ptr, S.gk[S.gcur].ptr, S.gv[S.gcur].ptr, R, C, P.rs_keep.ptr);
     };
     if (npairs > 0) {
         // both terms' tables with the primary's estimator (the two may be one)
@@ -2619,7 +2621,7 @@ static int64_t rsys_2d(Engine& P, Engine& S, const double* Trel, double eps, dou
                    P.rs_steps.ptr, P.rs_terms.ptr, (double2*)nullptr);
         MCE_LAUNCH(k_rsys_terms, dim3(ns), dim3(64), 0, st, SI, ns, d, 1.0, S.gk[S.gcur].ptr, S.gv[S.gcur].ptr, R,
                    ssteps, sterms, P.rs_shares.ptr);
-        pairs(k_rsys_pairs<false>, npairs, nullptr);
+        pairs(k_rsys_pairs<false>, k_rsys_near<false>, npairs, nullptr);
         MCE_LAUNCH(k_colsum_part, dim3(kColSlices, 14), dim3(256), 0, st, P.rs_mom.ptr, npairs,
                            P.rs_part.ptr);
         MCE_LAUNCH(k_colsum_finish, dim3(1), dim3(64), 0, st, P.rs_part.ptr, 14, P.rs_sums.ptr);
@@ -2684,7 +2686,7 @@ static int64_t rsys_2d(Engine& P, Engine& S, const double* Trel, double eps, dou
         P.c2_wall.reserve((size_t)nkeep * (CM + 1));
         P.c2_cell.reserve((size_t)nkeep * CM);
         C = Cpdf2D{CM, P.c2_mc.ptr, P.c2_b2.ptr, P.c2_wall.ptr, P.c2_cell.ptr};
-        pairs(k_rsys_pairs<true>, nkeep, P.rs_idx.ptr);
+        pairs(k_rsys_pairs<true>, k_rsys_near<true>, nkeep, P.rs_idx.ptr);
         launch_grid_2d(st, C, nkeep, shape, P.c2_px.ptr, P.c2_py.ptr, npts, P.cpdf_part.ptr, P.c2_err.ptr);
         MCE_LAUNCH(k_cpdf1d_finish, dim3(ceil_div(npts, kFinishPoints)), dim3(kFinishPoints * kFinishSlices), 0, st, P.cpdf_part.ptr, nchunks, npts,
                            1.0, P.cpdf_y.ptr);

@@ -4072,13 +4072,21 @@ __global__ __launch_bounds__(64) void k_rsys_terms(TermPool P, int n, int d, dou
 }
 
 // One thread per pair walks the lines of both terms in order: per line one 80-byte step of
-// either term, two sums, a product and the cell it closes, in registers.  Lines whose rows
-// agree within kCoalignEps up to sign, the last line with the first included, bound no cell
-// between them.  First (CELLS false) every pair's moments and whether the approximation keeps
+// either term, two sums, a product and the cell it closes, in registers.  Lines that are the
+// same, the last and the first included, bound no cell between them.  Rows that agree within
+// kCoalignEps up to sign count as one, the first of them in row order; where neighbouring lines
+// agree so far but differ by more than kSameLine, the pair is left to k_rsys_near (keep 2, or -1
+// cells).  First (CELLS false) every pair's moments and whether the approximation keeps
 // it; then (CELLS true) the cells of the n kept pairs idx[0 .. n), which the grid reads.  The
 // cells are 80 bytes each in separate stretches per lane, and writing them bounds the second
 // pass, so pairs that are dropped write none: 2.6 + 1.9 ms, where one pass that wrote every
 // pair's took 19.8 ms.  The first is bound by the latency of the steps' loads.
+constexpr double kSameLine = 1e-12;
+constexpr uint8_t kKeepNear = 2;
+__device__ inline bool same_line(double x0, double x1, double y0, double y1, double eps) {
+    return (fabs(x0 - y0) < eps && fabs(x1 - y1) < eps) || (fabs(x0 + y0) < eps && fabs(x1 + y1) < eps);
+}
+
 template <bool CELLS>
 __global__ __launch_bounds__(256) void k_rsys_pairs(TermPool P, TermPool S, int ns, int64_t n, int d,
                                                     const int* __restrict__ idx,
@@ -4144,9 +4152,12 @@ __global__ __launch_bounds__(256) void k_rsys_pairs(TermPool P, TermPool S, int 
         }
         u++;
     };
-    auto coaligned = [](double x0, double x1, double y0, double y1) {
-        return (fabs(x0 - y0) < kCoalignEps && fabs(x1 - y1) < kCoalignEps) ||
-               (fabs(x0 + y0) < kCoalignEps && fabs(x1 + y1) < kCoalignEps);
+    bool near = false;
+    // whether the row x, neighbour of y, has the same line
+    auto coaligned = [&](double x0, double x1, double y0, double y1) {
+        if (!same_line(x0, x1, y0, y1, kCoalignEps)) return false;
+        near |= !same_line(x0, x1, y0, y1, kSameLine);
+        return true;
     };
     double fs = 0, fc = 1, fa0 = 0, fa1 = 0;  // the first line
     double ls = 0, lc = 1, la0 = 0, la1 = 0;  // the line the open cell begins at
@@ -4179,11 +4190,18 @@ __global__ __launch_bounds__(256) void k_rsys_pairs(TermPool P, TermPool S, int 
             n1 = fromA ? A.a1 : B.a1;
             nt = fromA ? A.th : B.th;
         } while (nt < __builtin_inf() && coaligned(n0, n1, la0, la1));
+        if (near) break;
+    }
+    if (open) coaligned(la0, la1, fa0, fa1);
+    if (near) {
+        if constexpr (CELLS) C.mc[k] = -1;
+        else keep[k] = kKeepNear;
+        return;
     }
     if (open) {
         // the last cell ends at the first line's other half, or, where that is coaligned with
         // the last line, has ended there
-        const bool ended = u > 0 && coaligned(la0, la1, fa0, fa1);
+        const bool ended = u > 0 && same_line(la0, la1, fa0, fa1, kCoalignEps);
         const double es = ended ? ls : -fs, ec = ended ? lc : -fc;
         if (!ended) cell(ls, lc, es, ec);
         if constexpr (CELLS) {
@@ -4198,6 +4216,163 @@ __global__ __launch_bounds__(256) void k_rsys_pairs(TermPool P, TermPool S, int 
     } else {
         total *= (2 * R.norm_fact);
         keep[k] = (keep_term || !(fabs(total) < R.eps)) ? 1 : 0;
+    }
+}
+
+// The pairs that k_rsys_pairs left: rows that agree within kCoalignEps up to sign, but not to
+// rounding, are merged as the reference merges them (marg2d_remove_zeros_and_coalign,
+// cpdf_ndim.hpp:405-517): in row order, the primary's rows first, each row that is left takes
+// in every later one that agrees with it, and the cells are those of the rows that are left.  A
+// wavefront per pair, a lane per row and then per cell; two estimators of nearly equal systems
+// have such pairs, others hardly any, and then a wavefront only reads 64 pairs' flags at a time.
+// (Private arrays with computed indices, a thread per pair, are not an option: this compiler
+// keeps them in registers and gave wrong densities.)
+template <bool CELLS>
+__global__ __launch_bounds__(256) void k_rsys_near(TermPool P, TermPool S, int ns, int64_t n, int d,
+                                                   const int* __restrict__ idx, const uint32_t* __restrict__ pkeys,
+                                                   const cplx* __restrict__ pvals, const uint32_t* __restrict__ skeys,
+                                                   const cplx* __restrict__ svals, RsysArgs R, Cpdf2D C,
+                                                   uint8_t* __restrict__ keep) {
+    const int lane = wave_lane();
+    const int64_t waves = (int64_t)gridDim.x * (blockDim.x / kWave);
+    int64_t k0 = ((int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave) * kWave;
+    for (; k0 < n; k0 += waves * kWave) {
+        const bool mine = k0 + lane < n && (CELLS ? C.mc[k0 + lane] < 0 : keep[k0 + lane] == kKeepNear);
+        for (uint64_t todo = __ballot(mine); todo; todo &= todo - 1) {
+            const int64_t k = k0 + __ffsll((unsigned long long)todo) - 1;
+            const int64_t q = CELLS ? idx[k] : k;
+            const int tp = (int)(q / ns), ts = (int)(q % ns);
+            const int mp = P.m[tp], ms = S.m[ts], m = mp + ms;
+            // this lane's row, normalised; those that vanish keep the side of nu
+            const bool pr = lane < mp, row = lane < m;
+            double x0 = 0.0, x1 = 0.0, w = 0.0, ip = 0.0;
+            if (row) {
+                const double* A = pr ? P.A + ((int64_t)tp * P.MM + lane) * d : S.A + ((int64_t)ts * S.MM + lane - mp) * d;
+                const double sg = pr ? -1.0 : 1.0;
+                for (int j = 0; j < d; j++) {
+                    x0 += (A[j] * sg) * R.T[j];
+                    x1 += (A[j] * sg) * R.T[d + j];
+                    ip += (A[j] * sg) * R.nu[j];
+                }
+                w = pr ? P.p[(int64_t)tp * P.MM + lane] : S.p[(int64_t)ts * S.MM + lane - mp];
+            }
+            const bool line = row && !(fabs(x0) < kMuEps && fabs(x1) < kMuEps);
+            if (line) {
+                const double sa = fabs(x0) + fabs(x1);
+                x0 /= sa;
+                x1 /= sa;
+                w *= sa;
+            }
+            // the row that takes this one in, and whether they point opposite ways
+            int into = lane;
+            bool opposite = false;
+            for (int r = 0; r < m; r++) {
+                const double y0 = __shfl(x0, r, kWave), y1 = __shfl(x1, r, kWave);
+                const bool free_row = line && into == lane;
+                const uint64_t free_rows = __ballot(free_row);
+                if (!((free_rows >> r) & 1u) || !free_row || lane <= r) continue;
+                const bool pos = fabs(y0 - x0) < kCoalignEps && fabs(y1 - x1) < kCoalignEps;
+                if (pos || (fabs(y0 + x0) < kCoalignEps && fabs(y1 + x1) < kCoalignEps)) {
+                    into = r;
+                    opposite = !pos;
+                }
+            }
+            const bool left = line && into == lane;
+            const uint64_t lefts = __ballot(left);
+            const int u = __popcll(lefts);
+            for (int j = 0; j < m; j++) {  // the weights of what it took in, in row order
+                const double wj = __shfl(w, j, kWave);
+                const int rj = __shfl(into, j, kWave);
+                const bool lj = __shfl((int)line, j, kWave) != 0;
+                if (left && lj && rj == lane && j > lane) w += wj;
+            }
+            double t = 0.0, sn = 0.0, cs = 1.0;
+            if (left) {
+                const bool flat = fabs(x0) < fabs(x1);
+                t = flat ? atan2(-x0 / x1, 1.0) : atan2(1.0, -x1 / x0);
+                if (t < 0) t += kPi;
+                sn = sin(t);
+                cs = cos(t);
+            }
+            // place of its line going round; side of the row before the line
+            int place = 0;
+            for (int j = 0; j < m; j++) {
+                const double tj = __shfl(t, j, kWave);
+                place += ((lefts >> j) & 1u) && (tj < t || (tj == t && j < lane));
+            }
+            const bool neg = left && !(x0 * sn - x1 * cs > 0);
+            const bool neg_into = __shfl((int)neg, into, kWave) != 0;
+            const bool before = line ? neg_into != opposite : row && ip < 0;
+            const int at = __shfl(place, into, kWave);  // of the line it changes sides at
+            const double signedw = neg ? -w : w;
+            // lane c takes the cell between line c and the next, the last one half a turn on
+            double s1 = 0.0, c1 = 1.0, s2 = 0.0, c2 = 1.0, g1 = 0.0, g2 = 0.0;
+            uint32_t enc = 0;
+            for (int j = 0; j < m; j++) {
+                const bool lj = __shfl((int)line, j, kWave) != 0;
+                const bool crossed = __shfl(at, j, kWave) <= lane;
+                const bool bj = __shfl((int)before, j, kWave) != 0;
+                const double y0 = __shfl(x0, j, kWave), y1 = __shfl(x1, j, kWave), wj = __shfl(signedw, j, kWave);
+                const double tj = __shfl(t, j, kWave), sj = __shfl(sn, j, kWave), cj = __shfl(cs, j, kWave);
+                const int pj = __shfl(place, j, kWave);
+                enc |= (uint32_t)(bj != (lj && crossed)) << j;
+                if ((lefts >> j) & 1u) {
+                    const double v = crossed ? -wj : wj;
+                    g1 -= y0 * v;
+                    g2 -= y1 * v;
+                    if (pj == lane) {
+                        s1 = sj;
+                        c1 = cj;
+                    }
+                    if (pj == lane + 1) {
+                        s2 = sj;
+                        c2 = cj;
+                    }
+                    if (pj == 0 && lane == u - 1) {
+                        s2 = sin(tj + kPi);
+                        c2 = cos(tj + kPi);
+                    }
+                }
+            }
+            cplx g = cmake(0.0, 0.0);
+            if (lane < u) {
+                const int pmask = (1 << mp) - 1, smask = (1 << ms) - 1;
+                const int64_t po = P.gp_off[tp], so = S.gp_off[ts];
+                g = cmul(lookup_num((int)enc & pmask, 1 << (mp - 1), pmask, pkeys + po, pvals + po, P.gp_n[tp]),
+                         lookup_num((int)(enc >> mp), 1 << (ms - 1), smask, skeys + so, svals + so, S.gp_n[ts]));
+            }
+            if constexpr (CELLS) {
+                if (lane < u) {
+                    C.wall[k * (C.MM + 1) + lane] = wall2d(s1, c1, s2, c2, g1, g2, g);
+                    C.cell[k * C.MM + lane] = Cell2D{g1, g2, g};
+                }
+                if (lane == u - 1) {
+                    const double r = g1 * c2 + g2 * s2;
+                    C.wall[k * (C.MM + 1) + u] = Wall2D{c2, s2, r, r * r, 0.0, 0.0};
+                }
+                if (lane == 0) {
+                    double b0 = 0.0, b1 = 0.0;
+                    for (int j = 0; j < d; j++) {
+                        const double br = S.b[(int64_t)ts * d + j] - P.b[(int64_t)tp * d + j];
+                        b0 += R.T[j] * br;
+                        b1 += R.T[d + j] * br;
+                    }
+                    C.mc[k] = u;
+                    C.b2[2 * k] = b0;
+                    C.b2[2 * k + 1] = b1;
+                }
+            } else {
+                // the approximation's bound on the pair's contribution, as in k_rsys_pairs
+                const double den1 = g1 * (g1 * c1 + g2 * s1), den2 = g1 * (g1 * c2 + g2 * s2);
+                const bool stays = __any(lane < u && (fabs(den1) < 1e-14 || fabs(den2) < 1e-14));
+                const double gr = hypot(g.re, g.im);
+                const double bound = fabs((gr * s2) / den2) + fabs((gr * s1) / den1);
+                double total = 0.0;
+                for (int c = 0; c < u; c++) total += __shfl(bound, c, kWave);
+                total *= (2 * R.norm_fact);
+                if (lane == 0) keep[k] = (stays || !(fabs(total) < R.eps)) ? 1 : 0;
+            }
+        }
     }
 }
 

@@ -244,3 +244,42 @@ def test_rsys_matches_reference(name):
         assert _rel(got[:, 2], exp[:, 2]) <= TOL, f"{name} eps {e['eps']}: density"
     P.shutdown()
     S.shutdown()
+
+
+# The secondary's system is the primary's with every entry off by up to `delta` of itself, so each
+# line of one has a neighbour of the other that agrees with it within the coalignment tolerance
+# (1e-8) but not to rounding; at 2e-8 some do and some do not.  Library and restatement then merge
+# the same rows and differ by rounding alone: sums of some thousand cells, 1e-11 of the largest.
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["rsys_lti3", "rsys_lti2"])
+@pytest.mark.parametrize("delta", [0.0, 1e-10, 3e-9, 6e-9, 2e-8])
+def test_rows_that_nearly_coalign_merge_like_the_reference(name, delta):
+    from cauchyfriendly_amd.cauchy_estimator import eval_2d_relative_system_cpdf
+    print(f"case {name} {delta}", flush=True)
+    rec = _load(name)
+    rng = np.random.default_rng(20261205)
+    sec = json.loads(json.dumps(rec["primary"]["system"]))
+    for key in ("Phis", "Gamma", "H"):
+        a = np.array(sec[key], dtype=float)
+        sec[key] = (a * (1 + delta * rng.uniform(-1, 1, a.shape))).tolist()
+    sec["zs"] = (np.array(sec["zs"], dtype=float) + 0.3).tolist()
+    rec["secondary"] = {"system": sec, "steps": rec["primary"]["steps"]}
+    sp, ss = W.System.from_dict(rec["primary"]["system"]), W.System.from_dict(sec)
+    tp_terms, fzp = _oracle(sp, rec["primary"]["steps"])
+    ts_terms, fzs = _oracle(ss, rec["secondary"]["steps"])
+    P, S = _gpu_pair(rec)
+    e = rec["evals"][0]
+    libc = ct.CDLL("libc.so.6")
+    norm = (1 / (2 * np.pi)) ** 2 / fzp / fzs
+    for eps in (0.0, 1e-3):
+        libc.srand(ct.c_uint(7))
+        fz, xh, Ph, _, _, _, pts, nx, ny = eval_2d_relative_system_cpdf(e["Trel"], S, P, eps, *e["grid"])
+        libc.srand(ct.c_uint(7))
+        nu = np.array([2 * ((libc.rand() + 1.0) / (RAND_MAX + 2.0)) - 1 for _ in range(sp.n)])
+        nf, mean, cov, want, wx, wy = _rsys(tp_terms, ts_terms, e["Trel"], nu, eps, norm, e["grid"])
+        assert (nx, ny) == (wx, wy)
+        assert _rel(fz, nf.real) <= TOL and _rel(xh, mean.real) <= TOL and _rel(Ph, cov.real) <= TOL
+        z = 2 * want.reshape(-1, 3)[:, 2] * (1 / (2 * np.pi)) ** 2 / (fzp * fzs)
+        assert _rel(pts.reshape(-1, 3)[:, 2], z) <= 1e-11
+    P.shutdown()
+    S.shutdown()
