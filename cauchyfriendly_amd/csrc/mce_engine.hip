@@ -2588,7 +2588,9 @@ static int64_t rsys_2d(Engine& P, Engine& S, const double* Trel, double eps, dou
     const int64_t npairs = (int64_t)np * ns;
     const int CM = P.MM + S.MM;
     if (CM > kMaxM) throw std::runtime_error("the relative arrangement would exceed 31 hyperplanes");
-    const double bytes = (double)npairs * (CM * 32.0 + 48.0 * (CM + 1) + 14 * 8 + 32);
+    // What the pairs need if all are kept, at 88 bytes a cell: 80 are stored, and the limit has
+    // not moved with the layout.
+    const double bytes = (double)npairs * (CM * 72.0 + 8.0 * (CM + 1) * 2 + 14 * 8 + 32);
     if (bytes > 64.0 * (1ull << 30))
         throw std::runtime_error("the relative system's pairs need more than 64 GiB; use estimators with fewer terms");
     GraveyardScope gs(&P.graveyard);
