@@ -94,24 +94,4 @@ __device__ inline void coalign_gates(const double* r, const double* c, int d, bo
     }
 }
 
-// Orientation mask between two +/- equal arrangements: per row, sign of the
-// first element non-negligible in both, cell_enumeration.hpp:586-599.
-__device__ inline int orientation_mask(const double* Ai, const double* Aj, int m, int d) {
-    int sig = 0;
-    for (int k = 0; k < m; k++) {
-        int l = 0;
-        const int kd = k * d;
-        while (kd + l < m * d && ((fabs(Ai[kd + l]) < kReductionEps) || (fabs(Aj[kd + l]) < kReductionEps))) l++;
-        if (kd + l >= m * d) continue;
-        if ((Ai[kd + l] * Aj[kd + l]) < 0) sig |= (1 << k);
-    }
-    return sig;
-}
-
-// Order-preserving map of an FP64 value to an unsigned 64-bit radix key.
-__device__ inline uint64_t f64_radix_key(double x) {
-    uint64_t u = (uint64_t)__double_as_longlong(x);
-    return (u >> 63) ? ~u : (u | 0x8000000000000000ull);
-}
-
 }  // namespace mce

@@ -428,7 +428,6 @@ struct GraveyardScope {
     ~GraveyardScope() { t_graveyard = saved; }
 };
 
-// Grow-only device buffer; growing discards the contents.
 // Grow-only device buffer; growing discards the contents.  Its block comes from the block
 // cache; the owner's streams are idle whenever it is destroyed (every engine call ends with
 // its streams synchronised), so the block goes straight back.
@@ -706,7 +705,6 @@ struct Engine {
     std::vector<cplx> mean, cov, last_mean, last_cov;
     double gscale = 0;
     std::vector<int> in_count;  // per-shape term counts of the parent pool
-    // largest hyperplane count among the parent pool's terms (0 when it is empty)
     // diagnostics of the last update
     bool have_diag = false;
     std::vector<double> diag_mom;
@@ -724,9 +722,9 @@ struct Engine {
     long long terms_generated = 0;  // terms after MU/MUC (after MU on a window's last update), summed over updates
     // MCE_GEVAL_MODE=0..3 selects the g-table lookup mode (tuning; unsupported choices are ignored)
     int geval_mode_override = getenv("MCE_GEVAL_MODE") ? atoi(getenv("MCE_GEVAL_MODE")) : -1;
-    // MCE_BIG_GROUP_MEMBERS: groups with more members add them one wavefront per member
-    // groups from which on one wavefront takes a group's tangents (k_group_tan)
+    // MCE_TAN_ONE_WAVE: groups from which on one wavefront takes a group's tangents (k_group_tan)
     int tan_one_wave = getenv("MCE_TAN_ONE_WAVE") ? atoi(getenv("MCE_TAN_ONE_WAVE")) : kTanOneWave;
+    // MCE_BIG_GROUP_MEMBERS: groups with more members add them one wavefront per member
     int big_group_members = getenv("MCE_BIG_GROUP_MEMBERS") ? std::max(0, atoi(getenv("MCE_BIG_GROUP_MEMBERS")))
                                                             : kBigGroupMembers;
     // MCE_ENUM_THREADS=64|128|256: lanes per parent in the TP cell enumerator
@@ -1786,7 +1784,7 @@ struct Engine {
 
         if (skip) {
             MCE_RUN(k_hist, dim3(std::min(ceil_div(nslots, 256), 1024)), dim3(256), 0, st, nslots, sr + 1, 0,
-                               out.flags.ptr, out.m.ptr, (const int*)nullptr, (const uint32_t*)nullptr, hist.ptr);
+                               out.flags.ptr, out.m.ptr, (const int*)nullptr, hist.ptr);
             std::vector<int> h(sr + 1);
             co_await rd(hist.ptr, h.data(), sr + 1);
             if (prof.on && !bs)
@@ -1807,7 +1805,7 @@ struct Engine {
             MCE_RUN(k_iota, dim3(ceil_div(nslots, 256)), dim3(256), 0, st, iota.ptr, nslots);
             sort_pairs(keys.ptr, skeys.ptr, iota.ptr, perm.ptr, nslots, 0, kGatherKeyBits);
             MCE_RUN(k_hist, dim3(std::min(ceil_div(nslots, 256), 1024)), dim3(256), 0, st, nslots, sr + 1, 0,
-                               out.flags.ptr, out.m.ptr, (const int*)nullptr, (const uint32_t*)nullptr, hist.ptr);
+                               out.flags.ptr, out.m.ptr, (const int*)nullptr, hist.ptr);
             std::vector<int> cnt(sr + 1);
             co_await rd(hist.ptr, cnt.data(), sr + 1);
             if (prof.on && !bs)
@@ -2063,7 +2061,7 @@ struct Engine {
         }
         HIPCHK(hipGetLastError());
         MCE_RUN(k_hist, dim3(std::min(ceil_div(ng, 256), 1024)), dim3(256), 0, st, ng, sr + 1, 1,
-                           (const uint8_t*)nullptr, grp_m.ptr, surv.ptr, (const uint32_t*)nullptr, hist_mx.ptr);
+                           (const uint8_t*)nullptr, grp_m.ptr, surv.ptr, hist_mx.ptr);
         std::vector<int> h(sr + 2);
         {
             // histogram and the largest g-table (the next update's parent tables) in one read

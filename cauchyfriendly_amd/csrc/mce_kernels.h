@@ -1410,7 +1410,7 @@ __device__ __forceinline__ void k_mu_r(MG<256, 3> mg, TermPool IN, int np, const
 }
 
 // A window's last update: its terms are summed into the moments and not kept, so only the
-// moment inputs, the shape and the chain key of each slot are formed; the rows are never
+// moment inputs and the shape of each slot are formed; the rows are never
 // written, and the output pool holds nothing but flags and shapes.  The same operations in
 // the same order as k_mu and k_mu_r for any shape.
 template <int D>
@@ -1658,9 +1658,9 @@ __device__ __forceinline__ void k_mom_sum(MG<64 * kSumWaves, 2> mg, const double
 }
 
 // Histogram of small integer values privatised in LDS (nbins <= 64).  mode 0: valid
-// slots by shape; mode 1: surviving groups by shape; mode 2: chain keys.
+// slots by shape; mode 1: surviving groups by shape.
 __device__ __forceinline__ void k_hist(MG<1024, 1> mg, int n, int nbins, int mode, const uint8_t* __restrict__ flags, const int* __restrict__ vals,
-                       const int* __restrict__ surv, const uint32_t* __restrict__ ukeys, int* __restrict__ hist) {
+                       const int* __restrict__ surv, int* __restrict__ hist) {
     __shared__ int h[64];
     for (int b = threadIdx.x; b < nbins; b += blockDim.x) h[b] = 0;
     __syncthreads();
@@ -1668,10 +1668,8 @@ __device__ __forceinline__ void k_hist(MG<1024, 1> mg, int n, int nbins, int mod
         int v = -1;
         if (mode == 0) {
             if (flags[i] & kValid) v = vals[i];
-        } else if (mode == 1) {
-            if (surv[i] >= 0) v = vals[i];
-        } else {
-            v = (int)ukeys[i];
+        } else if (surv[i] >= 0) {
+            v = vals[i];
         }
         if (v >= 0 && v < nbins) atomicAdd(&h[v], 1);
     }
@@ -2556,9 +2554,10 @@ __device__ __forceinline__ void k_group_btab(MG<1024, 1> mg, const TermPool OUT,
 //   kLookupRankVals   rank structure and an LDS copy of the parent values
 // Every mode finds the same entry; they differ only in where the index comes from.
 // Largest shape of an estimator, and the largest for which the rank structure is used.  A rank
-// structure has 2^(shape-1) bits and as many prefix words / 32; beyond kRankShape it would leave
-// few wavefronts their LDS for tables of some hundred keys, which a binary search of the staged
-// keys finds in 5 to 9 steps.
+// structure has 2^(shape-1) bits and as many prefix words / 32: beyond kRankShape 16 KiB and more
+// for tables of some hundred keys, which a binary search of the staged keys finds in 5 to 9
+// steps.  The limit is not a measured crossover: the instantiation for 17 and more rows faulted
+// the GPU once, for a reason that was not found, and does not exist.
 constexpr int kMaxShape = 20;
 constexpr int kRankShape = 16;
 enum LookupMode { kLookupSearch = 0, kLookupSearchLds = 1, kLookupRank = 2, kLookupRankVals = 3 };
@@ -2672,8 +2671,10 @@ __device__ __forceinline__ double wave_psum2(const TermPool& T, int64_t s, int m
     return ps * ps;
 }
 
-// orientation_mask of two terms' rows by a whole wavefront, lane k on row k.  `ai` holds
-// Ai[k d] on lane k (kept by the caller for its root, which meets every member of its group).
+// Orientation mask between two +/- equal arrangements: per row, sign of the first element
+// non-negligible in both, cell_enumeration.hpp:586-599, by a whole wavefront, lane k on row k.
+// `ai` holds Ai[k d] on lane k (kept by the caller for its root, which meets every member of its
+// group).
 __device__ __forceinline__ int wave_orientation(const double* Ai, double ai, const double* Aj, int m, int d) {
     const int k = wave_lane();
     const bool row = k < m;
@@ -3468,7 +3469,9 @@ __global__ void k_sum_fixed(const double* __restrict__ v, int n, double* __restr
 
 // 1 / d to the last bit or two: the hardware's 2^-24 estimate x with error e = 1 - d x, then
 // x (1 + e + e^2), three fused operations where a division takes about ten.  Not finite where
-// d is zero, subnormal or not finite; the callers look for that in their sums.
+// d is zero, infinite or not a number, or 1 / d beyond the largest double; the callers look for
+// that in their sums.  Above 2^1022 1 / d is subnormal, and correct to its fewer bits at most: a
+// sum of such terms stays finite and is not formed again by divisions.
 __device__ __forceinline__ double fast_rcp(double d) {
     const double x = __builtin_amdgcn_rcp(d);
     const double e = __builtin_fma(-d, x, 1.0);
@@ -3805,7 +3808,6 @@ __global__ void k_cpdf2d_terms(TermPool P, int n, int i1, int i2, VecArg bar_nu,
 
 // Partial sums over one chunk of terms for kGridLanes * P grid points (the cached cell
 // integrals, marg2d_cached_eval_term_for_cpdf, cpdf_ndim.hpp:1654-1735).
-// `idx`, when given, lists the terms to add (the kept ones of a relative system).
 //
 // FP64 VALU bound.  A wavefront holds P points per lane and goes through a quarter of the
 // chunk's terms, whose walls it reads as scalars (every lane is at the same term).  The sum over a

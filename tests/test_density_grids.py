@@ -29,9 +29,12 @@ def test_a_point_is_alike_on_every_grid(name):
                    for a in density(g["xlow"] + 5 * rx, g["xlow"] + (5 + nx) * rx, rx, g["ylow"] + 5 * ry,
                                     g["ylow"] + (5 + ny) * ry, ry))
         print(f"case {name}: {z.size} of {Z.size} points", flush=True)
+        compared = 0
         for k in range(z.size):
             at = np.argmin(np.abs(X - x[k]) / rx + np.abs(Y - y[k]) / ry)
             # every grid's last column and row are its upper limits, which may lie off the others'
             if abs(X[at] - x[k]) < 1e-9 * rx and abs(Y[at] - y[k]) < 1e-9 * ry:
                 assert abs(Z[at] - z[k]) <= 1e-11 * peak
+                compared += 1
+        assert compared >= nx * ny
     est.shutdown()
